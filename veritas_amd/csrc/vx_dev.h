@@ -56,6 +56,17 @@ __device__ __forceinline__ double hwmin(double a, double b) {
     asm("v_min_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
     return r;
 }
+// the larger, smaller of 0 and a
+__device__ __forceinline__ double hwmax0(double a) {
+    double r;
+    asm("v_max_f64 %0, 0, %1" : "=v"(r) : "v"(a));
+    return r;
+}
+__device__ __forceinline__ double hwmin0(double a) {
+    double r;
+    asm("v_min_f64 %0, 0, %1" : "=v"(r) : "v"(a));
+    return r;
+}
 
 // Rectangle.hpp:86-88: lower p-face of cell j (pmin + dp * (j + p_pos))
 __device__ __forceinline__ double momentum(double pmin, double dp, int j, int p_pos) {
@@ -80,9 +91,23 @@ __device__ __forceinline__ double patch_E(const double *E, int n_f, int rtb, int
     return t;
 }
 
+// sqrt(x) for x >= 1 (or NaN): the compiler's FP64 sequence without its
+// scaling of arguments below 2^-767, so the same correctly rounded value; an
+// infinite x (rsq 0) returns itself as there.  Measured on an MI355X: 86
+// cycles per wave64 square root with the scaling, 70 without.
+__device__ __forceinline__ double sqrt_ge1(double x) {
+    const double y = __builtin_amdgcn_rsq(x);
+    const double s0 = x * y, h0 = 0.5 * y;
+    const double r0 = __builtin_fma(-h0, s0, 0.5);
+    const double s1 = __builtin_fma(s0, r0, s0), h1 = __builtin_fma(h0, r0, h0);
+    const double s2 = __builtin_fma(__builtin_fma(-s1, s1, x), h1, s1);
+    const double s3 = __builtin_fma(__builtin_fma(-s2, s2, x), h1, s2);
+    return x == __builtin_inf() ? x : s3;
+}
+
 // Rectangle.hpp:181-183 with mc2inv = (m_inv*c_inv)*(m_inv*c_inv)
 __device__ __forceinline__ double gamma_(double p, double a2, double mc2inv) {
-    return sqrt(1.0 + ((p * p) + a2) * mc2inv);
+    return sqrt_ge1(1.0 + ((p * p) + a2) * mc2inv);
 }
 
 // Rectangle.cpp:979-1030 (two-candidate WENO, upwind side takes the larger
@@ -110,6 +135,86 @@ __device__ __forceinline__ double weno(double f1, double f2, double f3, double f
     double fwL = w;
     double fwR = 1 - w;
     return fwL * fL + fwR * fR;
+}
+
+// Division without the scaling and fix-up steps of the compiler's FP64
+// sequence (v_div_scale, v_div_fmas, v_div_fixup): the same v_rcp_f64, Newton
+// and remainder steps, so the same correctly rounded quotient wherever no
+// intermediate leaves the normal range.  That holds for divisors in
+// [2^-900, 2^900] and numerators that are 0 or in [2^-900, 2^900] with
+// quotients in that range too (the remainder of a numerator n is a multiple of
+// 2^-106 |n|).  Measured on an MI355X in independent streams: 50 cycles per
+// wave64 division against 69 (v_div_scale_f64 alone takes 13, v_rcp_f64 18, an
+// FMA 5), and one reciprocal serves several numerators.
+__device__ __forceinline__ double rcp_refined(double d) {
+    double r = __builtin_amdgcn_rcp(d);
+    r = __builtin_fma(r, __builtin_fma(-d, r, 1.0), r);
+    return __builtin_fma(r, __builtin_fma(-d, r, 1.0), r);
+}
+// n / d from r = rcp_refined(d)
+__device__ __forceinline__ double div_refined(double n, double d, double r) {
+    const double q = n * r;
+    return __builtin_fma(__builtin_fma(-d, q, n), r, q);
+}
+
+// The parts of vxd::weno that belong to one cell, from the cell's value f and
+// its lower and upper neighbours: its candidate and weight as the left cell of
+// the face above it (fL, oL) and as the right cell of the face below it (fR,
+// oR).  Both share A, B and their three products, which vxd::weno forms once
+// per face and side.  The weights are 1 / (mm + b)^2, twice vxd::weno's: the
+// ratios oL / (oL + oR) have the same bits.  Valid for |f| below WENO_MAX (the
+// squares then stay below 2^770 and the weights above 2^-770, inside
+// rcp_refined's range); the callers take vxd::weno for larger values and NaN.
+constexpr double WENO_MAX = 0x1p190;
+struct WenoCell {
+    double fL, oL, fR, oR;
+};
+__device__ __forceinline__ WenoCell weno_cell(double fm, double f, double fp) {
+    WenoCell c;
+    const double m5 = 5 * f;
+    c.fL = (1.0 / 6) * (-fm + m5 + 2 * fp);
+    c.fR = (1.0 / 6) * (2 * fm + m5 - fp);
+    const double A = fm - 2 * f + fp;
+    const double B = fp - fm;
+    const double aa = 4.0 / 3 * (A * A), ab = 0.5 * A * B, bb = 0.25 * (B * B);
+    const double mm = 1.0e-10;
+    const double sL = mm + (aa + ab + bb), sR = mm + (aa - ab + bb);
+    const double dL = sL * sL, dR = sR * sR;
+    const double rL = rcp_refined(dL), rR = rcp_refined(dR);
+    c.oL = __builtin_fma(__builtin_fma(-dL, rL, 1.0), rL, rL);
+    c.oR = __builtin_fma(__builtin_fma(-dR, rR, 1.0), rR, rR);
+    return c;
+}
+// Face value from the left cell's (fL, oL) and the right cell's (fR, oR): the
+// bits of vxd::weno.
+__device__ __forceinline__ double weno_face(double fL, double oL, double fR, double oR, bool right) {
+    const double d = oL + oR;
+    const double r = rcp_refined(d);
+    const double wL = div_refined(oL, d, r);
+    const double wR = div_refined(oR, d, r);
+    const double wL0 = wL * (0.75 + wL * (wL - 0.5));
+    const double wR0 = wR * (0.75 + wR * (wR - 0.5));
+    const double s = wL0 + wR0;
+    // vxd::weno's choice: the larger weight for right, else the smaller (equal
+    // weights give the same value either way)
+    const double hi = hwmax(wL0, wR0), lo = hwmin(wL0, wR0);
+    const double w = div_refined(right ? hi : lo, s, rcp_refined(s));
+    return w * fL + (1 - w) * fR;
+}
+// Lanes whose value is outside weno_cell's range.
+__device__ __forceinline__ uint64_t weno_wide(double f) {
+    return __builtin_amdgcn_ballot_w64(!(__builtin_fabs(f) < WENO_MAX));
+}
+
+// A value that no lane of the launch writes, at a uniform index: read through
+// the scalar cache (s_load), so that it does not queue behind the wavefront's
+// vector loads (waiting for the youngest vector load waits for all of them).
+__device__ __forceinline__ double ld_uniform(const double *p, int i) {
+    typedef const double __attribute__((address_space(4))) *cptr;
+    return ((cptr)(uintptr_t)p)[i];
+}
+__device__ __forceinline__ bool same_bits(double a, double b) {
+    return __builtin_bit_cast(uint64_t, a) == __builtin_bit_cast(uint64_t, b);
 }
 
 // EMSolver.cpp:558-585: plain two-candidate WENO for the face potentials
@@ -161,6 +266,39 @@ __device__ __forceinline__ double weno_mp(double f1, double f2, double f3, doubl
     const float bR = eps + (4.0f / 3 * (AR * AR) - 0.5f * AR * BR + 0.25f * (BR * BR));
     // oL / (oL + oR) with o = 0.5 / b^2 is bR^2 / (bL^2 + bR^2); both are
     // divided by the larger b first, so the squares stay in [0, 1]
+    const float m = fmaxf(bL, bR);
+    const bool ok = m > 1e-30f;
+    const float rm = __builtin_amdgcn_rcpf(ok ? m : 1.0f);
+    const float x = bL * rm, y = bR * rm, x2 = x * x, y2 = y * y;
+    const float rden = __builtin_amdgcn_rcpf(x2 + y2);
+    const float wL = ok ? y2 * rden : 0.5f, wR = ok ? x2 * rden : 0.5f;
+    const float wL0 = wL * (0.75f + wL * (wL - 0.5f));
+    const float wR0 = wR * (0.75f + wR * (wR - 0.5f));
+    const bool takeL = right ? (wL0 > wR0) : (wL0 < wR0);
+    const float w = (takeL ? wL0 : wR0) * __builtin_amdgcn_rcpf(wL0 + wR0);
+    return fR + (double)w * (fL - fR);
+}
+
+// The parts of weno_mp that belong to one cell, as vxd::WenoCell: candidates
+// in FP64 and smoothness measures in FP32 (the same operations, so the same
+// bits), each formed once per cell instead of once per face and side.
+struct WenoCellMp {
+    double fL, fR;
+    float bL, bR;
+};
+__device__ __forceinline__ WenoCellMp weno_cell_mp(double fm, double f, double fp, float gm, float g, float gp,
+                                                   float eps) {
+    WenoCellMp c;
+    const double m5 = 5 * f;
+    c.fL = (1.0 / 6) * (-fm + m5 + 2 * fp);
+    c.fR = (1.0 / 6) * (2 * fm + m5 - fp);
+    const float A = gm - 2 * g + gp, B = gp - gm;
+    const float aa = 4.0f / 3 * (A * A), ab = 0.5f * A * B, bb = 0.25f * (B * B);
+    c.bL = eps + (aa + ab + bb);
+    c.bR = eps + (aa - ab + bb);
+    return c;
+}
+__device__ __forceinline__ double weno_face_mp(double fL, float bL, double fR, float bR, bool right) {
     const float m = fmaxf(bL, bR);
     const bool ok = m > 1e-30f;
     const float rm = __builtin_amdgcn_rcpf(ok ? m : 1.0f);

@@ -74,31 +74,42 @@ struct StageArgs {
     int nbx;      // tiles along p
     double sinv;  // MP: 2^-k, the scale of the FP32 copies of f
     float eps32;  // MP: the WENO epsilon (1e-10) in the scaled units
+    double inv_rtb;  // 1.0 / relativeToBottom
 };
 
-__device__ __forceinline__ double ldp(const double *pl, int pitch, int nx, int np, int i, int j) {
-    return (i >= -2 && i < nx + 2 && j >= -2 && j < np + 2) ? pl[pidx(pitch, i, j)] : 0.0;
+// Element of row i (uniform) at the lane's byte lb of a row: the row's address
+// stays in scalar registers and the lane adds a 32-bit offset.
+__device__ __forceinline__ double *elem(double *pl, int pitch, int i, uint32_t lb) {
+    return (double *)((char *)(pl + (long)(i + 2) * pitch) + lb);
 }
 
-// Row i of a plane at the clamped column jc, with i clamped into the plane:
-// no branch around the load, so that the loads in flight are counted one by
-// one and a row waits only for its own; the caller masks the value (0 outside
-// the plane) where it uses it, as ldp would have.
-__device__ __forceinline__ double ldr(const double *pl, int pitch, int nx, int i, int jc) {
+// Row i of a plane at the lane's (clamped) column, with i clamped into the
+// plane: no branch around the load, so that the loads in flight are counted
+// one by one and a row waits only for its own; the caller masks the value (0
+// outside the plane) where it uses it.
+__device__ __forceinline__ double ldr(const double *pl, int pitch, int nx, int i, uint32_t lb) {
     const int ic = i < -2 ? -2 : (i > nx + 1 ? nx + 1 : i);
-    return pl[pidx(pitch, ic, jc)];
+    return *elem(const_cast<double *>(pl), pitch, ic, lb);
 }
 
-// q^2 A^2 at x-face i (Rectangle.cpp:1280, 1296-1297; EMSolver.cpp:133-135)
-__device__ __forceinline__ double face_as(const StageArgs &A, const double *a2, int i) {
+// A^2 at x-face i (Rectangle.cpp:1280, 1296-1297; EMSolver.cpp:133-135)
+__device__ __forceinline__ double face_a2(const StageArgs &A, const double *a2, int i) {
     int fi = A.p.rtb * (i + A.p.x_pos);
     int c = fi < 0 ? 0 : (fi > A.n_f ? A.n_f : fi);
-    return A.p.q * A.p.q * a2[c];
+    return ld_uniform(a2, c);
 }
 
-// q * Rectangle::GetEfield(i) (Rectangle.cpp:1055-1067, 1298)
+// q * Rectangle::GetEfield(i) (Rectangle.cpp:1055-1067, 1298; vxd::patch_E)
 __device__ __forceinline__ double col_qE(const StageArgs &A, const double *E, int i) {
-    return A.p.q * patch_E(E, A.n_f, A.p.rtb, A.p.x_pos, i);
+    const int j = A.p.rtb * (i + A.p.x_pos);
+    double t = 0.0;
+    for (int k = 0; k < A.p.rtb; k++) {
+        int m = j + k;
+        m = m < 0 ? m + A.n_f : (m >= A.n_f ? m - A.n_f : m);
+        t += ld_uniform(E, m);
+    }
+    t *= A.inv_rtb;
+    return A.p.q * t;
 }
 
 // XCD-aware tile order (vxd::xcd_order): p-neighbouring tiles march over the
@@ -110,8 +121,22 @@ __device__ __forceinline__ int xcd_tile() { return xcd_order((int)blockIdx.x, (i
 // that every reference loop-range test below holds for every lane and every
 // march row (interior_strip states the margins), so IN only drops tests that
 // are true, and the IN and general forms give the same bits.
-template <int STEP, bool MP, bool IN>
-__device__ __forceinline__ void stage_strip(const StageArgs &A, const int jw, const int i0) {
+// FULL: divisions over the whole FP64 range (vxd::weno).  The other form
+// (vxd::weno_cell, weno_face) holds for |f| below vxd::WENO_MAX; it returns
+// the lanes that met a larger value (or NaN), and the caller then runs the
+// strip again as FULL: a strip reads nothing that it writes, so the second
+// run replaces every value of the first.
+//
+// What bounds it (4096 x 4096, MI355X): FP64 VALU issue, about 345 wave64
+// instructions per 58-cell row (461 before the parts that both sides of a face
+// share were formed once per cell, the divisions shortened, the x-speeds kept
+// where A^2 does not change and each limited flux formed once), two thirds of
+// the issue slots at three waves per SIMD; at stages 3 and 4 the stored fluxes
+// (88 and 104 B/cell) come close to the memory's rate as well.  The six stages
+// of a step: 2.62 ms before, 2.04 ms now (stage 0..5: 262, 290, 330, 384, 472,
+// 267 us).
+template <int STEP, bool MP, bool IN, bool FULL>
+__device__ __forceinline__ uint64_t stage_strip(const StageArgs &A, const int jw, const int i0) {
     const vx_patch &P = A.p;
     const int nx = P.n_x, np = P.n_p, pitch = P.pitch;
     const int lane = threadIdx.x & 63;
@@ -132,47 +157,62 @@ __device__ __forceinline__ void stage_strip(const StageArgs &A, const int jw, co
     const bool jr_ep = IN || (j >= -1 && j < np + 2);   // ep
     const bool jr_fp = IN || (j >= 0 && j < np + 1);    // fp, FpH, FpL p-faces
     const bool jr_R = IN || (j >= -1 && j < np + 1);    // R
+    const bool jint = IN || (j >= 0 && j < np);
     // update loop ranges (walls on all sides: xm = 1, xp = n_x, pm = 1, pp = n_p)
     const int xm = P.left ? 1 : 0, xp = P.right ? nx : nx + 1;
     const int pm = P.down ? 1 : 0, pp = P.up ? np : np + 1;
+    const bool jr_u = IN || (j >= pm && j < pp), jr_u1 = IN || (j + 1 >= pm && j + 1 < pp);
 
     const double mc2 = P.mc2inv;
     const double dpcc = P.dp_inv * P.cc;
     const double ccdx = P.cc * P.dx_inv;
     const double w3 = 1 / 48.0;
     const double pj = momentum(P.pmin, P.dp, j, P.p_pos);
-    const double pj2 = pj * pj;
 
     const double *fin = A.fin, *f0p = P.f[0];
     const int r0 = i0 - HALO;
 
     // pipeline state (names: _mK = row/face r-K)
-    double fs_m3 = 0, fs_m2 = 0, fs_m1 = 0, fs_0 = 0;
-    double f0_m3 = 0, f0_m2 = 0, f0_m1 = 0, f0_0 = 0;
+    double fs_m3 = 0, fs_m2 = 0, fs_m1 = 0, fs_0 = 0;  // (fs_m3: FULL only)
+    double f0_m1 = 0, f0_0 = 0;
     double ep_m2 = 0, ep_m1 = 0, ep_0 = 0, fp_m2 = 0, fp_m1 = 0, fp_0 = 0;
-    double FxL_m1 = 0, FxL_0 = 0, FpL_m1 = 0, FpL_0 = 0;
-    double f2_m3 = 0, f2_m2 = 0, f2_m1 = 0;
-    double FxD_m3 = 0, FxD_m2 = 0, FxD_m1 = 0;
-    double FpD_m3 = 0, FpD_m2 = 0, FpD_m1 = 0;
-    double Rp_m4 = 0, Rp_m3 = 0, Rp_m2 = 0, Rm_m4 = 0, Rm_m3 = 0, Rm_m2 = 0;
-    float gs_m3 = 0, gs_m2 = 0, gs_m1 = 0, gs_0 = 0;  // MP: FP32 copies of f_s rows
+    double xL_m1 = 0, xL_0 = 0, pL_m1 = 0, pL_0 = 0;  // stage-0 low-order fluxes times aSum
+    double f2_m2 = 0, f2_m1 = 0;
+    double hi_m3 = 0, hi_m2 = 0, hi_m1 = 0, lo_m3 = 0, lo_m2 = 0, lo_m1 = 0;  // larger, smaller of f^n and f^td
+    double FxD_m2 = 0, FxD_m1 = 0, FpD_m2 = 0, FpD_m1 = 0;
+    double Rp_m3 = 0, Rp_m2 = 0, Rm_m3 = 0, Rm_m2 = 0;
+    double t_m3 = 0;  // corrected value of cell r-3 but for its upper x-face
+    float gs_m2 = 0, gs_m1 = 0, gs_0 = 0;  // MP: FP32 copies of f_s rows
+    double fL_m2 = 0, oL_m2 = 0;  // WENO candidate and weight of cell r-2 at its upper x-face
+    float bL_m2 = 0;              // MP: its smoothness measure in place of the weight
+    uint64_t wide = 0;
     const double sinv = A.sinv;
     const float eps32 = A.eps32;
 
-    // Gamma(p_j, q^2 A^2 at x-face i), current fields and stage-0 fields
-    double as_m1 = face_as(A, A.a2, r0 - 1), as_0 = face_as(A, A.a2, r0);
-    double G_m1 = gamma_(pj, as_m1, mc2);
-    double G_0 = (as_0 == as_m1) ? G_m1 : gamma_(pj, as_0, mc2);
-    double as0_0 = face_as(A, A.a20, r0);
-    double G0_0 = (STEP == 0 || as0_0 == as_0) ? G_0 : gamma_(pj, as0_0, mc2);
+    // Gamma(p_j, q^2 A^2 at x-face i), current fields and stage-0 fields.  It
+    // changes along x only where A^2 does (inside a pulse), and so do the
+    // x-speeds ex formed from it: each is formed again only where the face's
+    // A^2 differs from the face before (a uniform branch).
+    const double qq = P.q * P.q;
+    double a2_0 = face_a2(A, A.a2, r0), a2_m1 = face_a2(A, A.a2, r0 - 1);
+    double G_m1 = gamma_(pj, qq * a2_m1, mc2);
+    double G_0 = same_bits(a2_0, a2_m1) ? G_m1 : gamma_(pj, qq * a2_0, mc2);
+    double a20_0 = face_a2(A, A.a20, r0);
+    double G0_0 = (STEP == 0 || same_bits(a20_0, a2_0)) ? G_0 : gamma_(pj, qq * a20_0, mc2);
+    // ex at x-face r-1 and its difference over lanes j+1, j-1; ex of stage 0
+    // at x-face r (lanes outside the p-range hold 0)
+    double ex = 0.0, dex = 0.0, ex0 = 0.0;
+    bool new_m1 = true, new_0 = true, new0_0 = true;  // face r-1, r / stage 0's face r differs from the one before
+    double a2_p1 = face_a2(A, A.a2, r0 + 1), a20_p1 = face_a2(A, A.a20, r0 + 1);
 
     // software prefetch: rows r and r+1 are in flight before iteration r, the
     // stored fluxes of x-face / column r-1 one iteration ahead
     const bool in_j = IN || (j >= -2 && j < np + 2);
     const int jc = IN ? j : (j < -2 ? -2 : (j > np + 1 ? np + 1 : j));
+    const uint32_t lb = 8u * (uint32_t)(jc + 2);  // the lane's byte in a row
     auto row_ok = [&](int i) { return IN || (i >= -2 && i < nx + 2 && in_j); };
-    double pfs_a = ldr(fin, pitch, nx, r0, jc), pf0_a = ldr(f0p, pitch, nx, r0, jc);
-    double pfs_b = ldr(fin, pitch, nx, r0 + 1, jc), pf0_b = ldr(f0p, pitch, nx, r0 + 1, jc);
+    double pfs_a = ldr(fin, pitch, nx, r0, lb), pf0_a = ldr(f0p, pitch, nx, r0, lb);
+    double pfs_b = ldr(fin, pitch, nx, r0 + 1, lb), pf0_b = ldr(f0p, pitch, nx, r0 + 1, lb);
     // stored flux planes read by this stage; stage 5 reads only plane 4, which
     // holds its partial sum
     constexpr int NH = STEP == 5 ? 1 : (STEP > 0 ? STEP : 1);
@@ -184,8 +224,8 @@ __device__ __forceinline__ void stage_strip(const StageArgs &A, const int jw, co
 #pragma unroll
         for (int k = 0; k < NH; k++) {
             const int plane = STEP == 5 ? 4 : k;
-            hx[k] = (k < STEP) ? ldr(P.FxH[plane], pitch, nx, face, jc) : 0.0;
-            hp[k] = (k < STEP) ? ldr(P.FpH[plane], pitch, nx, face, jc) : 0.0;
+            hx[k] = (k < STEP) ? ldr(P.FxH[plane], pitch, nx, face, lb) : 0.0;
+            hp[k] = (k < STEP) ? ldr(P.FpH[plane], pitch, nx, face, lb) : 0.0;
         }
     };
     load_h(r0 - 1);
@@ -204,8 +244,8 @@ __device__ __forceinline__ void stage_strip(const StageArgs &A, const int jw, co
         if (MP) gs_0 = (float)(fs_0 * sinv);
         pfs_a = pfs_b;
         pf0_a = pf0_b;
-        pfs_b = ldr(fin, pitch, nx, r + 2, jc);
-        pf0_b = ldr(f0p, pitch, nx, r + 2, jc);
+        pfs_b = ldr(fin, pitch, nx, r + 2, lb);
+        pf0_b = ldr(f0p, pitch, nx, r + 2, lb);
         if (STEP == 5) {
             // b_0 F_0 + ... + b_4 F_4 as stage 4 formed it; outside the face
             // ranges the masked sum of the five terms is +0
@@ -230,36 +270,72 @@ __device__ __forceinline__ void stage_strip(const StageArgs &A, const int jw, co
             }
         }
         load_h(r);
-        double as_p1 = face_as(A, A.a2, r + 1);
-        double G_p1 = (as_p1 == as_0) ? G_0 : gamma_(pj, as_p1, mc2);
-        double as0_p1 = face_as(A, A.a20, r + 1);
-        double G0_p1 = (STEP == 0 || as0_p1 == as_p1) ? G_p1 : gamma_(pj, as0_p1, mc2);
+        // the next row's A^2 is read one row ahead
+        const double a2_p2 = face_a2(A, A.a2, r + 2), a20_p2 = STEP == 0 ? a2_p2 : face_a2(A, A.a20, r + 2);
+        const bool new_p1 = !same_bits(a2_p1, a2_0);
+        const bool new0_p1 = STEP == 0 ? new_p1 : !same_bits(a20_p1, a20_0);
+        double G_p1 = G_0, dG = 0.0;  // dG: the force's Gamma term at column r
+        if (new_p1) {
+            G_p1 = gamma_(pj, qq * a2_p1, mc2);
+            dG = ccdx * (G_p1 - G_0);
+        }
+        double G0_p1, dG0 = 0.0;
+        if (STEP == 0) {
+            G0_p1 = G_p1;
+            dG0 = dG;
+        } else {
+            G0_p1 = G0_0;
+            if (new0_p1) {
+                G0_p1 = same_bits(a20_p1, a2_p1) ? G_p1 : gamma_(pj, qq * a20_p1, mc2);
+                dG0 = ccdx * (G0_p1 - G0_0);
+            }
+        }
 
         // ---- x-face r-1: ex, fx (Rectangle.cpp:1278-1293), FxH_s (1313-1334)
         const int ix = r - 1;
         const bool vFx = IN || (ix >= 0 && ix < nx + 1 && jr_ex);
-        double Gd = shdn1(G_m1);  // Gamma at p-face j+1
-        double ex = (IN || (ix >= -1 && ix < nx + 2 && jr_ex)) ? dpcc * (Gd - G_m1) : 0.0;
-        double fx = 0.0;
-        if (vFx) {
-            if (MP) fx = weno_mp(fs_m3, fs_m2, fs_m1, fs_0, gs_m3, gs_m2, gs_m1, gs_0, eps32, ex > 0.0);
-            else fx = weno(fs_m3, fs_m2, fs_m1, fs_0, ex > 0.0);
+        if (new_m1) {  // (used on rows of the face range only)
+            const double Gd = shdn1(G_m1);  // Gamma at p-face j+1
+            ex = jr_ex ? dpcc * (Gd - G_m1) : 0.0;
+            dex = shdn1(ex) - shup1(ex);
         }
-        double ex_u = shdn1(ex), ex_d = shup1(ex);
+        double fx = 0.0;
+        if (MP) {
+            const WenoCellMp c = weno_cell_mp(fs_m2, fs_m1, fs_0, gs_m2, gs_m1, gs_0, eps32);  // cell r-1
+            if (vFx) fx = weno_face_mp(fL_m2, bL_m2, c.fR, c.bR, ex > 0.0);
+            fL_m2 = c.fL;
+            bL_m2 = c.bL;
+        } else if (FULL) {
+            if (vFx) fx = weno(fs_m3, fs_m2, fs_m1, fs_0, ex > 0.0);
+        } else {
+            wide |= weno_wide(fs_0);
+            const WenoCell c = weno_cell(fs_m2, fs_m1, fs_0);  // cell r-1
+            if (vFx) fx = weno_face(fL_m2, oL_m2, c.fR, c.oR, ex > 0.0);
+            fL_m2 = c.fL;
+            oL_m2 = c.oL;
+        }
         double fx_u = shdn1(fx), fx_d = shup1(fx);
-        double FxH = vFx ? P.dx_inv * (fx * ex + w3 * (fx_u - fx_d) * (ex_u - ex_d)) : 0.0;
+        double FxH = vFx ? P.dx_inv * (fx * ex + w3 * (fx_u - fx_d) * dex) : 0.0;
 
         // ---- column r: ep, fp (Rectangle.cpp:1294-1312)
         const bool cr = IN || (r >= -1 && r < nx + 1);
         double qE = cr ? col_qE(A, A.E, r) : 0.0;
-        ep_0 = (cr && jr_ep) ? qE - ccdx * (G_p1 - G_0) : 0.0;
-        double s1 = shup1(fs_0), s2 = shup1(s1), s3 = shdn1(fs_0);
+        ep_0 = (cr && jr_ep) ? qE - dG : 0.0;
+        double s1 = shup1(fs_0), s3 = shdn1(fs_0);
         fp_0 = 0.0;
+        // the left cell's candidate and weight come from the lane below
         if (MP) {
-            float t1 = shup1f(gs_0), t2 = shup1f(t1), t3 = shdn1f(gs_0);
-            if (cr && jr_fp) fp_0 = weno_mp(s2, s1, fs_0, s3, t2, t1, gs_0, t3, eps32, ep_0 > 0.0);
-        } else if (cr && jr_fp) {
-            fp_0 = weno(s2, s1, fs_0, s3, ep_0 > 0.0);
+            const WenoCellMp c = weno_cell_mp(s1, fs_0, s3, shup1f(gs_0), gs_0, shdn1f(gs_0), eps32);
+            const double fl = shup1(c.fL);
+            const float bl = shup1f(c.bL);
+            if (cr && jr_fp) fp_0 = weno_face_mp(fl, bl, c.fR, c.bR, ep_0 > 0.0);
+        } else if (FULL) {
+            const double s2 = shup1(s1);
+            if (cr && jr_fp) fp_0 = weno(s2, s1, fs_0, s3, ep_0 > 0.0);
+        } else {
+            const WenoCell c = weno_cell(s1, fs_0, s3);
+            const double fl = shup1(c.fL), ol = shup1(c.oL);
+            if (cr && jr_fp) fp_0 = weno_face(fl, ol, c.fR, c.oR, ep_0 > 0.0);
         }
         // ---- column r-1: FpH_s (Rectangle.cpp:1353-1375)
         const bool vFp = IN || (ix >= -1 && ix < nx + 1 && jr_fp);
@@ -271,120 +347,142 @@ __device__ __forceinline__ void stage_strip(const StageArgs &A, const int jw, co
             // stage 4 stores stage 5's partial sum instead of its fluxes
             const double hx_out = STEP == 4 ? Qx + A.b5[4] * FxH : FxH;
             const double hp_out = STEP == 4 ? Qp + A.b5[4] * FpH : FpH;
-            if (vFx && own_x && own_row_x) __builtin_nontemporal_store(hx_out, &P.FxH[STEP][pidx(pitch, ix, j)]);
-            if (vFp && own_c && own_row_p) __builtin_nontemporal_store(hp_out, &P.FpH[STEP][pidx(pitch, ix, j)]);
+            if (vFx && own_x && own_row_x) __builtin_nontemporal_store(hx_out, elem(P.FxH[STEP], pitch, ix, lb));
+            if (vFp && own_c && own_row_p) __builtin_nontemporal_store(hp_out, elem(P.FpH[STEP], pitch, ix, lb));
         }
 
         // ---- low-order fluxes of stage 0 at x-face r and column r
         // (Rectangle.cpp:1335-1352, 1376-1394 evaluated with the stage-0 fields)
-        double G0d = shdn1(G0_0);
-        double ex0 = dpcc * (G0d - G0_0);
-        FxL_0 = (IN || (r >= 0 && r < nx + 1 && jr_ex)) ? P.dx_inv * ((ex0 > 0.0 ? f0_m1 : f0_0) * ex0) : 0.0;
+        if (new0_0) ex0 = dpcc * (shdn1(G0_0) - G0_0);
+        xL_0 = (IN || (r >= 0 && r < nx + 1 && jr_ex)) ? A.aSum * (P.dx_inv * ((ex0 > 0.0 ? f0_m1 : f0_0) * ex0)) : A.aSum * 0.0;
         double qE0 = cr ? col_qE(A, A.E0, r) : 0.0;
-        double ep0 = qE0 - ccdx * (G0_p1 - G0_0);
+        double ep0 = qE0 - dG0;
         double f0_jm1 = shup1(f0_0);
-        FpL_0 = (cr && jr_fp) ? P.dp_inv * ((ep0 > 0.0 ? f0_jm1 : f0_0) * ep0) : 0.0;
+        pL_0 = (cr && jr_fp) ? A.aSum * (P.dp_inv * ((ep0 > 0.0 ? f0_jm1 : f0_0) * ep0)) : A.aSum * 0.0;
 
         // ---- cell r-1: low-order predictor (Rectangle.cpp:1518-1534, gather form)
         {
             const int i = r - 1;
-            double FpL_up = shdn1(FpL_m1);  // FpL0 at (i, j+1)
+            double pL_up = shdn1(pL_m1);  // at (i, j+1)
             double t = 0.0;
-            if (IN || (i >= 0 && i < nx && j >= 0 && j < np)) {
+            if (IN || (i >= 0 && i < nx && jint)) {
                 t = f0_m1;
-                const bool in0 = IN || (i >= xm && i < xp && j >= pm && j < pp);
+                const bool in0 = IN || (i >= xm && i < xp && jr_u);
                 if (in0) {
-                    t += A.aSum * FxL_m1;
-                    t += A.aSum * FpL_m1;
+                    t += xL_m1;
+                    t += pL_m1;
                 }
-                if (IN || (i >= xm && i < xp && j + 1 >= pm && j + 1 < pp)) t -= A.aSum * FpL_up;
-                if (IN || (i + 1 >= xm && i + 1 < xp && j >= pm && j < pp)) t -= A.aSum * FxL_0;
+                if (IN || (i >= xm && i < xp && jr_u1)) t -= pL_up;
+                if (IN || (i + 1 >= xm && i + 1 < xp && jr_u)) t -= xL_0;
             }
             f2_m1 = t;  // ghost cells: zero fill of the walls (BoundaryCondition.cpp:6-8)
+            hi_m1 = hwmax(f0_m1, t);
+            lo_m1 = hwmin(f0_m1, t);
         }
 
         // ---- x-face r-1 and column r-1: RK flux combination (Rectangle.cpp:1396-1517)
         {
-            double xLS = A.aSum * FxL_m1, pLS = A.aSum * FpL_m1;
             double sx = STEP == 0 ? A.a[0] * FxH : Sx + A.a[STEP] * FxH;
             double sp = STEP == 0 ? A.a[0] * FpH : Sp + A.a[STEP] * FpH;
-            FxD_m1 = sx - xLS;
-            FpD_m1 = sp - pLS;
+            FxD_m1 = sx - xL_m1;
+            FpD_m1 = sp - pL_m1;
         }
 
         // ---- cell r-2: Zalesak R+- (Rectangle.cpp:1538-1579)
         {
             const int i = r - 2;
             double FpDu = shdn1(FpD_m2);  // FpDS at (i, j+1)
-            double f0u = shdn1(f0_m2), f0d = shup1(f0_m2);
-            double f2u = shdn1(f2_m2), f2d = shup1(f2_m2);
+            double hu = shdn1(hi_m2), hd = shup1(hi_m2);
+            double lu = shdn1(lo_m2), ld = shup1(lo_m2);
             double rp = 0.0, rm = 0.0;
             if (IN || (i >= -1 && i < nx + 1 && jr_R)) {
-                // fmax/fmin (one v_max_f64/v_min_f64 each) give the reference's
+                // hwmax/hwmin (one v_max_f64/v_min_f64 each) give the reference's
                 // a > b ? a : b bits here: f is never -0 (every update adds to a
                 // +0 or positive start), R and Q are never -0, nothing is NaN,
                 // and a signed zero among the P terms reaches P only when P is
                 // zero, where R is 0 either way
-                double Pp = fmax(0.0, FxD_m2) - fmin(0.0, FxD_m1) + fmax(0.0, FpD_m2) - fmin(0.0, FpDu);
-                double Pm = fmax(0.0, FxD_m1) - fmin(0.0, FxD_m2) + fmax(0.0, FpDu) - fmin(0.0, FpD_m2);
-                double wMax = hwmax(hwmax(f0_m2, f2_m2), hwmax(hwmax(f0_m1, f2_m1),
-                              hwmax(hwmax(f0_m3, f2_m3), hwmax(hwmax(f0u, f2u), hwmax(f0d, f2d)))));
-                double wMin = hwmin(hwmin(f0_m2, f2_m2), hwmin(hwmin(f0_m1, f2_m1),
-                              hwmin(hwmin(f0_m3, f2_m3), hwmin(hwmin(f0u, f2u), hwmin(f0d, f2d)))));
+                double Pp = hwmax0(FxD_m2) - hwmin0(FxD_m1) + hwmax0(FpD_m2) - hwmin0(FpDu);
+                double Pm = hwmax0(FxD_m1) - hwmin0(FxD_m2) + hwmax0(FpDu) - hwmin0(FpD_m2);
+                double wMax = hwmax(hi_m2, hwmax(hi_m1, hwmax(hi_m3, hwmax(hu, hd))));
+                double wMin = hwmin(lo_m2, hwmin(lo_m1, hwmin(lo_m3, hwmin(lu, ld))));
                 double Qm = -wMin + f2_m2;
                 double Qp = wMax - f2_m2;
                 if (MP) {
                     rp = Pp > 0.0 ? zalesak_mp(Qp, Pp, sinv) : 0.0;
                     rm = Pm > 0.0 ? zalesak_mp(Qm, Pm, sinv) : 0.0;
                 } else {
-                    rp = Pp > 0.0 ? fmin(1.0, Qp / Pp) : 0.0;
-                    rm = Pm > 0.0 ? fmin(1.0, Qm / Pm) : 0.0;
+                    // min(1, Q / P) is 1 where Q >= P: only a wavefront with a
+                    // lane below that (beside an extremum of f) divides
+                    rp = Pp > 0.0 ? 1.0 : 0.0;
+                    rm = Pm > 0.0 ? 1.0 : 0.0;
+                    if (__builtin_amdgcn_ballot_w64(!(Qp - Pp >= 0.0) || !(Qm - Pm >= 0.0)) != 0) {
+                        if (Pp > 0.0) rp = fmin(1.0, Qp / Pp);
+                        if (Pm > 0.0) rm = fmin(1.0, Qm / Pm);
+                    }
                 }
             }
             Rp_m2 = rp;
             Rm_m2 = rm;
         }
 
-        // ---- cell r-3: limiter C on its faces (Rectangle.cpp:1581-1594) and the
-        // corrected value (Rectangle.cpp:1596-1612, gather form)
+        // ---- limiter C of cell r-2's lower faces (Rectangle.cpp:1581-1594) and
+        // the corrected value (Rectangle.cpp:1596-1612, gather form): a cell
+        // takes its lower x-face and its p-faces at this row and its upper x-face
+        // at the next, each limited flux formed once, in the reference's order
         {
-            const int i = r - 3;
-            double Rpd = shup1(Rp_m3), Rmd = shup1(Rm_m3);  // R at (i, j-1)
-            const bool jint = IN || (j >= 0 && j < np);
-            double cxl = (IN || (i >= 1 && i < nx && jint))
-                             ? (FxD_m3 > 0.0 ? hwmin(Rp_m3, Rm_m4) : hwmin(Rp_m4, Rm_m3)) : 1.0;
-            double cxr = (IN || (i + 1 >= 1 && i + 1 < nx && jint))
-                             ? (FxD_m2 > 0.0 ? hwmin(Rp_m2, Rm_m3) : hwmin(Rp_m3, Rm_m2)) : 1.0;
-            double cpl = (IN || (i >= 1 && i < nx && jint))
-                             ? (FpD_m3 > 0.0 ? hwmin(Rp_m3, Rmd) : hwmin(Rpd, Rm_m3)) : 1.0;
-            double cpu = shdn1(cpl);      // C at (i, j+1), computed by the next lane
-            double FpDu = shdn1(FpD_m3);  // FpDS at (i, j+1)
-            if (out_lane && i >= i0 && i < i1) {
-                double t = f2_m3;
-                if (IN || (i >= xm && i < xp && j >= pm && j < pp)) {
-                    t += cxl * FxD_m3;
-                    t += cpl * FpD_m3;
-                }
-                if (IN || (i >= xm && i < xp && j + 1 >= pm && j + 1 < pp)) t -= cpu * FpDu;
-                if (IN || (i + 1 >= xm && i + 1 < xp && j >= pm && j < pp)) t -= cxr * FxD_m2;
-                A.fout[pidx(pitch, i, j)] = t;
+            const int i = r - 2;
+            double Rpd = shup1(Rp_m2), Rmd = shup1(Rm_m2);  // R at (i, j-1)
+            const bool lim = IN || (i >= 1 && i < nx && jint);
+            double cx = lim ? (FxD_m2 > 0.0 ? hwmin(Rp_m2, Rm_m3) : hwmin(Rp_m3, Rm_m2)) : 1.0;
+            double cp = lim ? (FpD_m2 > 0.0 ? hwmin(Rp_m2, Rmd) : hwmin(Rpd, Rm_m2)) : 1.0;
+            const double lx = cx * FxD_m2, lp = cp * FpD_m2;
+            const double lpu = shdn1(lp);  // the limited flux at (i, j+1), formed by the next lane
+            if (out_lane && i - 1 >= i0 && i - 1 < i1) {
+                double t = t_m3;
+                if (IN || (i >= xm && i < xp && jr_u)) t -= lx;
+                *elem(A.fout, pitch, i - 1, lb) = t;
             }
+            double t = f2_m2;
+            if (IN || (i >= xm && i < xp && jr_u)) {
+                t += lx;
+                t += lp;
+            }
+            if (IN || (i >= xm && i < xp && jr_u1)) t -= lpu;
+            t_m3 = t;
         }
 
         // ---- shift the pipeline by one row
-        fs_m3 = fs_m2; fs_m2 = fs_m1; fs_m1 = fs_0;
-        gs_m3 = gs_m2; gs_m2 = gs_m1; gs_m1 = gs_0;
-        f0_m3 = f0_m2; f0_m2 = f0_m1; f0_m1 = f0_0;
-        as_0 = as_p1; G_m1 = G_0; G_0 = G_p1; G0_0 = G0_p1;
+        if (FULL) fs_m3 = fs_m2;
+        fs_m2 = fs_m1; fs_m1 = fs_0;
+        gs_m2 = gs_m1; gs_m1 = gs_0;
+        f0_m1 = f0_0;
+        a2_0 = a2_p1; a2_p1 = a2_p2; a20_0 = a20_p1; a20_p1 = a20_p2;
+        new_m1 = new_0; new_0 = new_p1; new0_0 = new0_p1;
+        G_m1 = G_0; G_0 = G_p1; G0_0 = G0_p1;
         ep_m2 = ep_m1; ep_m1 = ep_0; fp_m2 = fp_m1; fp_m1 = fp_0;
-        FxL_m1 = FxL_0; FpL_m1 = FpL_0;
-        f2_m3 = f2_m2; f2_m2 = f2_m1;
-        FxD_m3 = FxD_m2; FxD_m2 = FxD_m1;
-        FpD_m3 = FpD_m2; FpD_m2 = FpD_m1;
-        Rp_m4 = Rp_m3; Rp_m3 = Rp_m2; Rm_m4 = Rm_m3; Rm_m3 = Rm_m2;
+        xL_m1 = xL_0; pL_m1 = pL_0;
+        f2_m2 = f2_m1;
+        hi_m3 = hi_m2; hi_m2 = hi_m1; lo_m3 = lo_m2; lo_m2 = lo_m1;
+        FxD_m2 = FxD_m1; FpD_m2 = FpD_m1;
+        Rp_m3 = Rp_m2; Rm_m3 = Rm_m2;
     };
 
-    for (int r = r0; r <= i1 + HALO - 1; r++) row(r);
+    // Two rows at a time turn the pipeline's shifts (37 64-bit moves of 362 VALU
+    // instructions a row) into register names.  Stage 4 holds eight stored
+    // fluxes in flight and would spill (4096 x 4096: 472 us one row at a time,
+    // 495 two), as would the mixed-precision stage 3.
+    constexpr bool TWO = IN && STEP != 4 && !(MP && STEP == 3);
+    if (TWO) {
+        int r = r0;
+        for (; r < i1 + HALO - 1; r += 2) {
+            row(r);
+            row(r + 1);
+        }
+        if (r == i1 + HALO - 1) row(r);
+    } else {
+        for (int r = r0; r <= i1 + HALO - 1; r++) row(r);
+    }
+    return wide;
 }
 
 // Whether a strip takes the IN form.  Lanes hold j in [jw - 3, jw + 60] and
@@ -405,8 +503,9 @@ __device__ __forceinline__ void stage_tile(const StageArgs &A, const int tile) {
     const int strip = by * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     if (strip >= A.nstrip) return;  // uniform per wavefront
     const int jw = bx * OUTW, i0 = strip * A.TI;
-    if (interior_strip(A, jw, i0)) stage_strip<STEP, MP, true>(A, jw, i0);
-    else stage_strip<STEP, MP, false>(A, jw, i0);
+    const uint64_t wide = interior_strip(A, jw, i0) ? stage_strip<STEP, MP, true, false>(A, jw, i0)
+                                                    : stage_strip<STEP, MP, false, false>(A, jw, i0);
+    if (!MP && wide != 0) stage_strip<STEP, MP, false, true>(A, jw, i0);
 }
 
 // Compiled for at least three resident waves per SIMD (at most 168 VGPRs):
@@ -438,7 +537,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
         if (wg_start[mid] <= tile) lo = mid;
         else hi = mid - 1;
     }
-    stage_tile<STEP, MP>(items[lo], tile - wg_start[lo]);
+    // a copy through the scalar cache, so that the row loop's reads of it do
+    // not go back to memory behind the plane stores
+    StageArgs A;
+    typedef const uint32_t __attribute__((address_space(4))) *cptr;
+    cptr src = (cptr)(uintptr_t)(items + lo);
+    uint32_t w[sizeof(StageArgs) / 4];
+#pragma unroll
+    for (size_t k = 0; k < sizeof(StageArgs) / 4; k++) w[k] = src[k];
+    __builtin_memcpy(&A, w, sizeof A);
+    stage_tile<STEP, MP>(A, tile - wg_start[lo]);
 }
 
 template <bool MP>
@@ -687,6 +795,7 @@ static int stage_args(vx_ctx *ctx, const vx_patch *p, int step, double dt, const
     A.nbx = (p->n_p + OUTW - 1) / OUTW;
     A.sinv = 1.0;
     A.eps32 = 0.0f;
+    A.inv_rtb = 1.0 / (double)p->rtb;
     if (mp) {
         if (!(f_scale > 0.0) || !std::isfinite(f_scale))
             return fail(ctx, VX_EINVAL, "stage_fused_mp: f scale must be positive and finite");
