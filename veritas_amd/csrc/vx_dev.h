@@ -5,6 +5,7 @@
 #pragma once
 
 #include <hip/hip_runtime.h>
+#include <stdint.h>
 
 #include "vx_consts.h"
 
@@ -213,6 +214,18 @@ __device__ __forceinline__ double ld_uniform(const double *p, int i) {
     typedef const double __attribute__((address_space(4))) *cptr;
     return ((cptr)(uintptr_t)p)[i];
 }
+// The same for a whole struct of 32-bit words at a uniform address.
+template <class T>
+__device__ __forceinline__ T ld_uniform_struct(const T *p) {
+    typedef const uint32_t __attribute__((address_space(4))) *cptr;
+    cptr src = (cptr)(uintptr_t)p;
+    uint32_t w[sizeof(T) / 4];
+#pragma unroll
+    for (size_t k = 0; k < sizeof(T) / 4; k++) w[k] = src[k];
+    T t;
+    __builtin_memcpy(&t, w, sizeof(T));
+    return t;
+}
 __device__ __forceinline__ bool same_bits(double a, double b) {
     return __builtin_bit_cast(uint64_t, a) == __builtin_bit_cast(uint64_t, b);
 }
@@ -233,6 +246,21 @@ __device__ __forceinline__ double face_weno(double f1, double f2, double f3, dou
     double wL = oL / (oL + oR);
     double wR = oR / (oL + oR);
     return wL * fL + wR * fR;
+}
+
+// Element of row i (uniform) at the lane's byte lb of a row: the row's address
+// stays in scalar registers and the lane adds a 32-bit offset.
+__device__ __forceinline__ double *elem(double *pl, int pitch, int i, uint32_t lb) {
+    return (double *)((char *)(pl + (long)(i + 2) * pitch) + lb);
+}
+
+// Row i of a plane at the lane's (clamped) column, with i clamped into the
+// plane: no branch around the load, so that the loads in flight are counted
+// one by one and a row waits only for its own; the caller masks the value (0
+// outside the plane) where it uses it.
+__device__ __forceinline__ double ldr(const double *pl, int pitch, int nx, int i, uint32_t lb) {
+    const int ic = i < -2 ? -2 : (i > nx + 1 ? nx + 1 : i);
+    return *elem(const_cast<double *>(pl), pitch, ic, lb);
 }
 
 // Whole-wavefront lane shifts by one lane (DPP wave_shl:1 / wave_shr:1, plain

@@ -77,21 +77,6 @@ struct StageArgs {
     double inv_rtb;  // 1.0 / relativeToBottom
 };
 
-// Element of row i (uniform) at the lane's byte lb of a row: the row's address
-// stays in scalar registers and the lane adds a 32-bit offset.
-__device__ __forceinline__ double *elem(double *pl, int pitch, int i, uint32_t lb) {
-    return (double *)((char *)(pl + (long)(i + 2) * pitch) + lb);
-}
-
-// Row i of a plane at the lane's (clamped) column, with i clamped into the
-// plane: no branch around the load, so that the loads in flight are counted
-// one by one and a row waits only for its own; the caller masks the value (0
-// outside the plane) where it uses it.
-__device__ __forceinline__ double ldr(const double *pl, int pitch, int nx, int i, uint32_t lb) {
-    const int ic = i < -2 ? -2 : (i > nx + 1 ? nx + 1 : i);
-    return *elem(const_cast<double *>(pl), pitch, ic, lb);
-}
-
 // A^2 at x-face i (Rectangle.cpp:1280, 1296-1297; EMSolver.cpp:133-135)
 __device__ __forceinline__ double face_a2(const StageArgs &A, const double *a2, int i) {
     int fi = A.p.rtb * (i + A.p.x_pos);
@@ -539,13 +524,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
     }
     // a copy through the scalar cache, so that the row loop's reads of it do
     // not go back to memory behind the plane stores
-    StageArgs A;
-    typedef const uint32_t __attribute__((address_space(4))) *cptr;
-    cptr src = (cptr)(uintptr_t)(items + lo);
-    uint32_t w[sizeof(StageArgs) / 4];
-#pragma unroll
-    for (size_t k = 0; k < sizeof(StageArgs) / 4; k++) w[k] = src[k];
-    __builtin_memcpy(&A, w, sizeof A);
+    const StageArgs A = ld_uniform_struct(items + lo);
     stage_tile<STEP, MP>(A, tile - wg_start[lo]);
 }
 
