@@ -149,12 +149,15 @@ typedef struct vx_stage_item {
 int vx_fct_stage_fused_batch(vx_ctx *ctx, const vx_stage_item *items, int n, int step);
 /* Rows per strip that the fused stage uses at RK stage `step` for patches of
  * n_x x n_p cells, in FP64 (mixed = 0) or mixed precision (mixed = 1); timed
- * on the first call for that shape, stage and precision, 0 before it.  No
- * counterpart in the reference: it reports the tile shape the library chose. */
+ * on the first vx_fct_stage_fused (or _mp) call for that shape, stage and
+ * precision, 0 before it (a batched launch chooses its own strips by its total
+ * size).  No counterpart in the reference: it reports the tile shape the
+ * library chose. */
 int vx_stage_tile_rows(vx_ctx *ctx, int32_t n_x, int32_t n_p, int step, int mixed);
 /* Resident waves per SIMD of the kernel form chosen with those strips: 4 (the
- * form compiled for at most 128 VGPRs) or 3 (the other), 0 before the first
- * call; both forms give the same bits.  No counterpart in the reference. */
+ * forms of at most 128 VGPRs, the one with a wavefront per row among them) or 3
+ * (the other), 0 before the first call; all forms give the same bits.  No
+ * counterpart in the reference. */
 int vx_stage_tile_waves(vx_ctx *ctx, int32_t n_x, int32_t n_p, int step, int mixed);
 int vx_fct_stage_fused_available(void);
 

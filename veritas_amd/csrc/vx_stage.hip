@@ -69,7 +69,7 @@ struct StageArgs {
     double a[6], aSum;
     double b5[6];  // stage 5's coefficients times dt (stage 4 forms its partial sum)
     int TI;       // output rows per strip
-    int w4;       // 1: the kernel form held to four waves per SIMD (k_stage_w4)
+    int form;     // 0: k_stage; 1: held to four waves per SIMD (k_stage_w4); 2: k_stage_rows
     int nstrip;   // strips in x
     int nbx;      // tiles along p
     double sinv;  // MP: 2^-k, the scale of the FP32 copies of f
@@ -509,30 +509,302 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
     stage_tile<STEP, MP>(A, xcd_tile());
 }
 
+// The same stage with one wavefront per row, for patches too small to fill the
+// device with long strips: a workgroup owns TI output rows of a p-column and
+// runs TI + 4 wavefronts, wavefront w at row r = i0 - 2 + w (x-face r, column r
+// and cell r).  What a row takes from the rows beside it goes through LDS, with
+// a workgroup barrier per hand-over: (fp, ep), then (FxDS and the extrema of
+// f^n and f^td), then R.  Each value is formed by the strip's operations, so
+// the bits are the strip's.
+// A strip of TI rows walks TI + 6 rows one after another, each a dependent
+// chain of two reconstructions; here they run at once.  601 x 333 cells with a
+// pulse (MI355X): 21 to 25 us a stage as strips, 10 to 12 here; 64 x 256 cells:
+// 23 and 6 us.  The price is (TI + 4) / TI rows of work per output row,
+// so strips win where they fill the device.
+constexpr int RT_ARRAYS = 7;  // LDS rows of 64 doubles per wavefront
+
+__device__ __forceinline__ double &lds_row(double *lds, int nw, int q, int w) {
+    return lds[(q * nw + w) * 64 + (threadIdx.x & 63)];
+}
+
+template <int STEP, bool MP>
+__device__ __forceinline__ void stage_rows(const StageArgs &A, const int tile, double *lds) {
+    const vx_patch &P = A.p;
+    const int nx = P.n_x, np = P.n_p, pitch = P.pitch;
+    const int lane = threadIdx.x & 63;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nw = A.TI + 4;
+    const int bx = tile % A.nbx, by = tile / A.nbx;
+    const int jw = bx * OUTW, i0 = by * A.TI, r = i0 - 2 + w;
+    const int i1 = min(i0 + A.TI, nx);  // output rows [i0, i1)
+    const bool last_strip = i0 + A.TI >= nx;
+    const int j = jw - HALO + lane;
+    const bool mid_lane = lane >= HALO && lane < 64 - HALO;
+    const bool out_lane = mid_lane && j < np;
+    const bool own_row_p = out_lane || (j == np && lane >= HALO && lane < 65 - HALO);
+    const bool own_row_x = own_row_p || (jw == 0 && j == -1);
+    // reference loop ranges (Rectangle.cpp:1279-1394, 1518-1612)
+    const bool jint = j >= 0 && j < np;
+    const bool jr_ex = j >= -1 && j < np + 1, jr_ep = j >= -1 && j < np + 2, jr_fp = j >= 0 && j < np + 1;
+    const int xm = P.left ? 1 : 0, xp = P.right ? nx : nx + 1;
+    const int pm = P.down ? 1 : 0, pp = P.up ? np : np + 1;
+    const bool jr_u = j >= pm && j < pp, jr_u1 = j + 1 >= pm && j + 1 < pp;
+    const bool in_r = r >= xm && r < xp, in_r1 = r + 1 >= xm && r + 1 < xp;
+    const bool vFx = r >= 0 && r < nx + 1 && jr_ex;
+    const bool cr = r >= -1 && r < nx + 1;
+    const bool vFp = cr && jr_fp;
+
+    // every load of the row at once
+    const bool in_j = j >= -2 && j < np + 2;
+    const int jc = j < -2 ? -2 : (j > np + 1 ? np + 1 : j);
+    const uint32_t lb = 8u * (uint32_t)(jc + 2);
+    auto row_ok = [&](int i) { return i >= -2 && i < nx + 2 && in_j; };
+    double fs[4], f0[3];  // f_s at rows r-2 .. r+1, f^n at rows r-1 .. r+1
+#pragma unroll
+    for (int k = 0; k < 4; k++) fs[k] = ldr(A.fin, pitch, nx, r - 2 + k, lb);
+#pragma unroll
+    for (int k = 0; k < 3; k++) f0[k] = ldr(P.f[0], pitch, nx, r - 1 + k, lb);
+    constexpr int NH = STEP == 5 ? 1 : (STEP > 0 ? STEP : 1);
+    double hx[NH], hp[NH];
+#pragma unroll
+    for (int k = 0; k < NH; k++) {
+        const int plane = STEP == 5 ? 4 : k;
+        hx[k] = k < STEP ? ldr(P.FxH[plane], pitch, nx, r, lb) : 0.0;
+        hp[k] = k < STEP ? ldr(P.FpH[plane], pitch, nx, r, lb) : 0.0;
+    }
+    const double qq = P.q * P.q, mc2 = P.mc2inv;
+    const double dpcc = P.dp_inv * P.cc, ccdx = P.cc * P.dx_inv, w3 = 1 / 48.0;
+    const double pj = momentum(P.pmin, P.dp, j, P.p_pos);
+
+    // Gamma at x-faces r, r+1 (and r+1 of stage 0), the speeds
+    const double a2_0 = face_a2(A, A.a2, r), a2_1 = face_a2(A, A.a2, r + 1);
+    const double G_0 = gamma_(pj, qq * a2_0, mc2);
+    double G_1 = G_0, dG = 0.0;
+    if (!same_bits(a2_1, a2_0)) {
+        G_1 = gamma_(pj, qq * a2_1, mc2);
+        dG = ccdx * (G_1 - G_0);
+    }
+    const double Gd = shdn1(G_0);  // (lane shifts run with every lane active)
+    const double ex = jr_ex ? dpcc * (Gd - G_0) : 0.0;
+    const double dex = shdn1(ex) - shup1(ex);
+    double G0_0 = G_0, G0_1 = G_1, dG0 = dG;
+    if (STEP > 0) {
+        const double b_0 = face_a2(A, A.a20, r), b_1 = face_a2(A, A.a20, r + 1);
+        if (!same_bits(b_0, a2_0)) G0_0 = gamma_(pj, qq * b_0, mc2);
+        if (!same_bits(b_1, a2_1)) G0_1 = gamma_(pj, qq * b_1, mc2);
+        dG0 = ccdx * (G0_1 - G0_0);
+    }
+    const double ex0 = dpcc * (shdn1(G0_0) - G0_0), ex0_1 = dpcc * (shdn1(G0_1) - G0_1);
+
+    uint64_t wide[4];
+    float gs[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        fs[k] = row_ok(r - 2 + k) ? fs[k] : 0.0;
+        if (MP) gs[k] = (float)(fs[k] * A.sinv);
+        else wide[k] = weno_wide(fs[k]);
+    }
+#pragma unroll
+    for (int k = 0; k < 3; k++) f0[k] = row_ok(r - 1 + k) ? f0[k] : 0.0;
+
+    // ---- x-face r
+    double fx = 0.0;
+    if (MP) {
+        const WenoCellMp cl = weno_cell_mp(fs[0], fs[1], fs[2], gs[0], gs[1], gs[2], A.eps32);
+        const WenoCellMp ch = weno_cell_mp(fs[1], fs[2], fs[3], gs[1], gs[2], gs[3], A.eps32);
+        if (vFx) fx = weno_face_mp(cl.fL, cl.bL, ch.fR, ch.bR, ex > 0.0);
+    } else if (__builtin_expect((wide[0] | wide[1] | wide[2] | wide[3]) != 0, 0)) {
+        if (vFx) fx = weno(fs[0], fs[1], fs[2], fs[3], ex > 0.0);
+    } else {
+        const WenoCell cl = weno_cell(fs[0], fs[1], fs[2]), ch = weno_cell(fs[1], fs[2], fs[3]);
+        if (vFx) fx = weno_face(cl.fL, cl.oL, ch.fR, ch.oR, ex > 0.0);
+    }
+    const double fx_u = shdn1(fx), fx_d = shup1(fx);
+    const double FxH = vFx ? P.dx_inv * (fx * ex + w3 * (fx_u - fx_d) * dex) : 0.0;
+
+    // ---- column r
+    const double qE = cr ? col_qE(A, A.E, r) : 0.0;
+    const double ep = (cr && jr_ep) ? qE - dG : 0.0;
+    const double s1 = shup1(fs[2]), s3 = shdn1(fs[2]);
+    double fp = 0.0;
+    if (MP) {
+        const WenoCellMp c = weno_cell_mp(s1, fs[2], s3, shup1f(gs[2]), gs[2], shdn1f(gs[2]), A.eps32);
+        const double fl = shup1(c.fL);
+        const float bl = shup1f(c.bL);
+        if (vFp) fp = weno_face_mp(fl, bl, c.fR, c.bR, ep > 0.0);
+    } else if (__builtin_expect(wide[2] != 0, 0)) {
+        const double s2 = shup1(s1);
+        if (vFp) fp = weno(s2, s1, fs[2], s3, ep > 0.0);
+    } else {
+        const WenoCell c = weno_cell(s1, fs[2], s3);
+        const double fl = shup1(c.fL), ol = shup1(c.oL);
+        if (vFp) fp = weno_face(fl, ol, c.fR, c.oR, ep > 0.0);
+    }
+    lds_row(lds, nw, 0, w) = fp;
+    lds_row(lds, nw, 1, w) = ep;
+
+    // ---- stage-0 low-order fluxes of x-faces r, r+1 and column r, and the
+    // low-order predictor of cell r
+    const double qE0 = cr ? col_qE(A, A.E0, r) : 0.0;
+    const double ep0 = qE0 - dG0;
+    const double f0_jm1 = shup1(f0[1]);
+    auto xl = [&](int face, double e, double lo, double hi) {
+        return (face >= 0 && face < nx + 1 && jr_ex) ? A.aSum * (P.dx_inv * ((e > 0.0 ? lo : hi) * e)) : A.aSum * 0.0;
+    };
+    const double xL = xl(r, ex0, f0[0], f0[1]), xL_1 = xl(r + 1, ex0_1, f0[1], f0[2]);
+    const double pL = vFp ? A.aSum * (P.dp_inv * ((ep0 > 0.0 ? f0_jm1 : f0[1]) * ep0)) : A.aSum * 0.0;
+    const double pL_u = shdn1(pL);
+    double f2 = 0.0;  // ghost cells: zero fill of the walls
+    if (r >= 0 && r < nx && jint) {
+        f2 = f0[1];
+        if (in_r && jr_u) {
+            f2 += xL;
+            f2 += pL;
+        }
+        if (in_r && jr_u1) f2 -= pL_u;
+        if (in_r1 && jr_u) f2 -= xL_1;
+    }
+    const double hi = hwmax(f0[1], f2), lo = hwmin(f0[1], f2);
+
+    // ---- RK sums of the earlier stages' fluxes (left to right)
+    double Sx = 0.0, Sp = 0.0, Qx = 0.0, Qp = 0.0;
+    if (STEP == 5) {
+        Sx = vFx ? hx[0] : 0.0;
+        Sp = vFp ? hp[0] : 0.0;
+    } else if (STEP > 0) {
+        Sx = A.a[0] * (vFx ? hx[0] : 0.0);
+        Sp = A.a[0] * (vFp ? hp[0] : 0.0);
+#pragma unroll
+        for (int k = 1; k < NH; k++) {
+            Sx = Sx + A.a[k] * (vFx ? hx[k] : 0.0);
+            Sp = Sp + A.a[k] * (vFp ? hp[k] : 0.0);
+        }
+        if (STEP == 4) {
+            Qx = A.b5[0] * (vFx ? hx[0] : 0.0);
+            Qp = A.b5[0] * (vFp ? hp[0] : 0.0);
+#pragma unroll
+            for (int k = 1; k < NH; k++) {
+                Qx = Qx + A.b5[k] * (vFx ? hx[k] : 0.0);
+                Qp = Qp + A.b5[k] * (vFp ? hp[k] : 0.0);
+            }
+        }
+    }
+    const double FxD = (STEP == 0 ? A.a[0] * FxH : Sx + A.a[STEP] * FxH) - xL;
+    lds_row(lds, nw, 2, w) = FxD;
+    lds_row(lds, nw, 3, w) = hi;
+    lds_row(lds, nw, 4, w) = lo;
+    __syncthreads();
+
+    // ---- column r: FpH_s from the columns beside it (a wavefront at the end of
+    // the workgroup reads its own row instead: its value is not used)
+    const int wd = w > 0 ? w - 1 : w, wu = w + 1 < nw ? w + 1 : w;
+    const double fp_d = lds_row(lds, nw, 0, wd), fp_u = lds_row(lds, nw, 0, wu);
+    const double ep_d = lds_row(lds, nw, 1, wd), ep_u = lds_row(lds, nw, 1, wu);
+    const double FpH = vFp ? P.dp_inv * (fp * ep + w3 * (fp_u - fp_d) * (ep_u - ep_d)) : 0.0;
+    if (STEP < 5) {
+        const bool own_x = r >= i0 && (r < i0 + A.TI || last_strip);
+        const bool own_c = (r >= i0 || (i0 == 0 && r >= -1)) && (r < i0 + A.TI || last_strip);
+        const double hx_out = STEP == 4 ? Qx + A.b5[4] * FxH : FxH;
+        const double hp_out = STEP == 4 ? Qp + A.b5[4] * FpH : FpH;
+        if (vFx && own_x && own_row_x) __builtin_nontemporal_store(hx_out, elem(P.FxH[STEP], pitch, r, lb));
+        if (vFp && own_c && own_row_p) __builtin_nontemporal_store(hp_out, elem(P.FpH[STEP], pitch, r, lb));
+    }
+    const double FpD = (STEP == 0 ? A.a[0] * FpH : Sp + A.a[STEP] * FpH) - pL;
+
+    // ---- cell r: Zalesak R+-
+    const double FxDu = lds_row(lds, nw, 2, wu), FpDu = shdn1(FpD);
+    const double hiu = lds_row(lds, nw, 3, wu), hid = lds_row(lds, nw, 3, wd);
+    const double lou = lds_row(lds, nw, 4, wu), lod = lds_row(lds, nw, 4, wd);
+    const double hju = shdn1(hi), hjd = shup1(hi), lju = shdn1(lo), ljd = shup1(lo);
+    double Rp = 0.0, Rm = 0.0;
+    if (r >= -1 && r < nx + 1 && jr_ex) {
+        const double Pp = hwmax0(FxD) - hwmin0(FxDu) + hwmax0(FpD) - hwmin0(FpDu);
+        const double Pm = hwmax0(FxDu) - hwmin0(FxD) + hwmax0(FpDu) - hwmin0(FpD);
+        const double wMax = hwmax(hi, hwmax(hiu, hwmax(hid, hwmax(hju, hjd))));
+        const double wMin = hwmin(lo, hwmin(lou, hwmin(lod, hwmin(lju, ljd))));
+        const double Qm = -wMin + f2;
+        const double Qu = wMax - f2;
+        if (MP) {
+            Rp = Pp > 0.0 ? zalesak_mp(Qu, Pp, A.sinv) : 0.0;
+            Rm = Pm > 0.0 ? zalesak_mp(Qm, Pm, A.sinv) : 0.0;
+        } else {
+            Rp = Pp > 0.0 ? 1.0 : 0.0;
+            Rm = Pm > 0.0 ? 1.0 : 0.0;
+            if (__builtin_amdgcn_ballot_w64(!(Qu - Pp >= 0.0) || !(Qm - Pm >= 0.0)) != 0) {
+                if (Pp > 0.0) Rp = fmin(1.0, Qu / Pp);
+                if (Pm > 0.0) Rm = fmin(1.0, Qm / Pm);
+            }
+        }
+    }
+    lds_row(lds, nw, 5, w) = Rp;
+    lds_row(lds, nw, 6, w) = Rm;
+    __syncthreads();
+
+    // ---- limiter C on the faces of cell r and the corrected value
+    if (r < i0 || r >= i1) return;  // uniform; no barrier follows
+    const double Rp_d = lds_row(lds, nw, 5, wd), Rm_d = lds_row(lds, nw, 6, wd);
+    const double Rp_u = lds_row(lds, nw, 5, wu), Rm_u = lds_row(lds, nw, 6, wu);
+    const double Rpl = shup1(Rp), Rml = shup1(Rm);  // R at (r, j-1)
+    const bool lim = r >= 1 && r < nx && jint, lim_u = r + 1 >= 1 && r + 1 < nx && jint;
+    const double cx = lim ? (FxD > 0.0 ? hwmin(Rp, Rm_d) : hwmin(Rp_d, Rm)) : 1.0;
+    const double cxu = lim_u ? (FxDu > 0.0 ? hwmin(Rp_u, Rm) : hwmin(Rp, Rm_u)) : 1.0;
+    const double cp = lim ? (FpD > 0.0 ? hwmin(Rp, Rml) : hwmin(Rpl, Rm)) : 1.0;
+    const double lx = cx * FxD, lxu = cxu * FxDu, lp = cp * FpD;
+    const double lpu = shdn1(lp);
+    if (out_lane) {
+        double t = f2;
+        if (in_r && jr_u) {
+            t += lx;
+            t += lp;
+        }
+        if (in_r && jr_u1) t -= lpu;
+        if (in_r1 && jr_u) t -= lxu;
+        *elem(A.fout, pitch, r, lb) = t;
+    }
+}
+
+template <int STEP, bool MP>
+__global__ __launch_bounds__(1024) void k_stage_rows(StageArgs A) {
+    extern __shared__ double lds[];
+    stage_rows<STEP, MP>(A, xcd_tile(), lds);
+}
+
 // Several patches (of independent runs) at the same RK stage in one launch:
 // workgroups [wg_start[k], wg_start[k+1]) of the XCD-ordered tile sequence
-// belong to item k.  Held to three waves per SIMD like k_stage (stages 3 and
-// 4 would take 185-206 VGPRs, two waves).
-template <int STEP, bool MP>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k_stage_batch(const StageArgs *items, const int *wg_start, int n) {
-    const int tile = xcd_tile();
+// belong to item k; the item's arguments come through the scalar cache.  Strips
+// (k_stage_batch) or one wavefront per row (k_stage_rows_batch), one form for
+// the launch (batch_form).
+__device__ __forceinline__ int batch_item(const int *wg_start, int n, int tile) {
     int lo = 0, hi = n - 1;  // the last k with wg_start[k] <= tile (uniform)
     while (lo < hi) {
         const int mid = (lo + hi + 1) >> 1;
         if (wg_start[mid] <= tile) lo = mid;
         else hi = mid - 1;
     }
-    // a copy through the scalar cache, so that the row loop's reads of it do
-    // not go back to memory behind the plane stores
-    const StageArgs A = ld_uniform_struct(items + lo);
-    stage_tile<STEP, MP>(A, tile - wg_start[lo]);
+    return lo;
+}
+template <int STEP, bool MP>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k_stage_batch(const StageArgs *items, const int *wg_start, int n) {
+    const int tile = xcd_tile(), k = batch_item(wg_start, n, tile);
+    const StageArgs A = ld_uniform_struct(items + k);
+    stage_tile<STEP, MP>(A, tile - wg_start[k]);
+}
+template <int STEP, bool MP>
+__global__ __launch_bounds__(1024) void k_stage_rows_batch(const StageArgs *items, const int *wg_start, int n) {
+    extern __shared__ double lds[];
+    const int tile = xcd_tile(), k = batch_item(wg_start, n, tile);
+    const StageArgs A = ld_uniform_struct(items + k);
+    stage_rows<STEP, MP>(A, tile - wg_start[k], lds);
 }
 
 template <bool MP>
-void launch_stage_t(vx_ctx *ctx, const StageArgs &A, dim3 grid) {
+void launch_stage_t(vx_ctx *ctx, const StageArgs &A) {
+    const int strips_wg = A.form == 2 ? 1 : 4, waves = A.form == 2 ? A.TI + 4 : 4;
+    const dim3 grid((unsigned)(A.nbx * ((A.nstrip + strips_wg - 1) / strips_wg))), block(64 * waves);
+    const size_t lds = sizeof(double) * 64 * RT_ARRAYS * waves;
 #define VX_STAGE(S)                                                        \
-    if (A.w4) k_stage_w4<S, MP><<<grid, 256, 0, ctx->stream>>>(A);         \
-    else k_stage<S, MP><<<grid, 256, 0, ctx->stream>>>(A);
+    if (A.form == 2) k_stage_rows<S, MP><<<grid, block, lds, ctx->stream>>>(A);  \
+    else if (A.form == 1) k_stage_w4<S, MP><<<grid, block, 0, ctx->stream>>>(A); \
+    else k_stage<S, MP><<<grid, block, 0, ctx->stream>>>(A);
     switch (A.step) {
         case 0: VX_STAGE(0) break;
         case 1: VX_STAGE(1) break;
@@ -546,9 +818,8 @@ void launch_stage_t(vx_ctx *ctx, const StageArgs &A, dim3 grid) {
 
 void launch_stage(vx_ctx *ctx, StageArgs &A, bool mp) {
     A.nstrip = (A.p.n_x + A.TI - 1) / A.TI;
-    dim3 grid((unsigned)(A.nbx * ((A.nstrip + 3) / 4)));
-    if (mp) launch_stage_t<true>(ctx, A, grid);
-    else launch_stage_t<false>(ctx, A, grid);
+    if (mp) launch_stage_t<true>(ctx, A);
+    else launch_stage_t<false>(ctx, A);
 }
 
 // Rows per strip (the tile height) of a patch shape and RK stage (the later
@@ -563,10 +834,12 @@ void launch_stage(vx_ctx *ctx, StageArgs &A, bool mp) {
 // is being recorded the choice falls back to the shortest strip that still
 // gives 2048 wavefronts.
 //
-// Each strip height is timed in both kernel forms (k_stage: three waves per
-// SIMD for the stages that need more than 128 VGPRs; k_stage_w4: four), the
-// four-wave form winning only when more than 3 % faster; a choice is kept as
-// rows + W4_FORM for the four-wave form.
+// A choice is kept as rows, rows + W4_FORM for the four-wave form (k_stage_w4)
+// and rows + 2 W4_FORM for the row form (k_stage_rows), which is timed
+// where a SIMD gets at most ROWS_PER_SIMD rows of the patch: it redoes 4 rows
+// in 12, strips that fill the device about 6 in 50.  Measured, all stages of
+// 1024 x 1024 (18 rows a SIMD): 31 to 45 us as rows, 54 to 64 as strips before
+// this form; 2048 x 1024 mixed (36 rows): 49 to 59 us as rows, 45 to 60 as strips.
 // The choices are kept per device for the whole process (every context on the
 // device shares them: a serving loop's runs of one shape time it once).
 struct TileKey {
@@ -575,7 +848,7 @@ struct TileKey {
         return std::tie(device, nx, np, mp, step) < std::tie(o.device, o.nx, o.np, o.mp, o.step);
     }
 };
-constexpr int W4_FORM = 4096;
+constexpr int W4_FORM = 4096, ROWS_MAX = 12, ROWS_PER_SIMD = 64;
 std::mutex g_tile_mu;
 std::map<TileKey, int> g_tiles;
 
@@ -635,7 +908,8 @@ int tile_rows(vx_ctx *ctx, const StageArgs &A0, bool mp) {
             if (*q == ',') q++;
         }
         const int ti = n == 6 ? v[A0.step] : (n >= 1 ? v[0] : 0);
-        if ((ti >= 1 && ti <= 1024) || (ti > W4_FORM && ti <= W4_FORM + 1024)) {
+        if ((ti >= 1 && ti <= 1024) || (ti > W4_FORM && ti <= W4_FORM + 1024) ||
+            (ti > 2 * W4_FORM && ti <= 2 * W4_FORM + ROWS_MAX)) {
             ctx->ti_cache.push_back({nx, np, ti, (int)mp, A0.step});  // this context only
             return ti;
         }
@@ -678,7 +952,7 @@ int tile_rows(vx_ctx *ctx, const StageArgs &A0, bool mp) {
         auto timed = [&](int code) {
             StageArgs A = A0;
             A.TI = code % W4_FORM;
-            A.w4 = code / W4_FORM;
+            A.form = code / W4_FORM;
             float t = 1e30f;
             if (hipEventRecord(e0, ctx->stream) != hipSuccess) failed = true;
             if (!failed) launch_stage(ctx, A, mp);
@@ -697,17 +971,26 @@ int tile_rows(vx_ctx *ctx, const StageArgs &A0, bool mp) {
         {
             StageArgs A = A0;
             A.TI = guess;
-            A.w4 = 0;
+            A.form = 0;
             launch_stage(ctx, A, mp);  // warm
         }
+        // The four-wave form is timed at stage 0, which nearly fits its 128
+        // VGPRs (4096 x 4096: 272 us against 261); the later stages spill there
+        // (354 against 291 us at stage 1, 2.4 times as long at stage 3).  Strips
+        // under 8 rows lose to the row form wherever the launch is small enough
+        // to want them (601 x 333: 21 to 25 us against 10 to 13).
+        std::vector<int> codes;
         for (int ti : cands) {
-            if (ti > 2 && ti >= 2 * nx) continue;  // a single strip either way
-            for (int w4 = 0; w4 < 2 && !failed; w4++) {
-                const int code = ti + (w4 ? W4_FORM : 0);
-                const float t = timed(code);
-                if (!failed) res.push_back({code, t});
-            }
+            if (ti < 8 || (ti > 8 && ti >= 2 * nx)) continue;  // a single strip either way
+            codes.push_back(ti);
+            if (A0.step == 0) codes.push_back(ti + W4_FORM);
+        }
+        if ((long)A0.nbx * nx <= (long)ROWS_PER_SIMD * 4 * ctx->n_cu)
+            for (int ti : {12, 8, 4}) codes.push_back(ti + 2 * W4_FORM);
+        for (int code : codes) {
+            const float t = timed(code);
             if (failed) break;
+            res.push_back({code, t});
         }
         if (!failed && !res.empty()) {
             std::vector<int> order(res.size());
@@ -744,7 +1027,7 @@ int vx_fct_stage_fused_available(void) { return 1; }
 
 // Checks and kernel arguments of one patch's fused stage.
 static int stage_args(vx_ctx *ctx, const vx_patch *p, int step, double dt, const vx_fields *fl,
-                      const double *fin, double *fout, bool mp, double f_scale, StageArgs &A) {
+                      const double *fin, double *fout, bool mp, double f_scale, bool choose, StageArgs &A) {
     int rc = validate_patch(ctx, p);
     if (rc) return rc;
     if (step < 0 || step > 5 || !fl || !fl->E0 || !fl->a20)
@@ -781,10 +1064,12 @@ static int stage_args(vx_ctx *ctx, const vx_patch *p, int step, double dt, const
         A.sinv = std::ldexp(1.0, -std::ilogb(f_scale));
         A.eps32 = (float)(1.0e-10 * A.sinv * A.sinv);
     }
-    A.w4 = 0;
+    A.form = 0;
+    A.TI = 0;
+    if (!choose) return VX_OK;  // (batch_launch chooses for all of its items)
     const int choice = tile_rows(ctx, A, mp);
     A.TI = choice % W4_FORM;
-    A.w4 = choice / W4_FORM;
+    A.form = choice / W4_FORM;
     A.nstrip = (p->n_x + A.TI - 1) / A.TI;
     return VX_OK;
 }
@@ -792,7 +1077,7 @@ static int stage_args(vx_ctx *ctx, const vx_patch *p, int step, double dt, const
 static int stage_fused(vx_ctx *ctx, const vx_patch *p, int step, double dt, const vx_fields *fl,
                        const double *fin, double *fout, bool mp, double f_scale) {
     StageArgs A;
-    int rc = stage_args(ctx, p, step, dt, fl, fin, fout, mp, f_scale, A);
+    int rc = stage_args(ctx, p, step, dt, fl, fin, fout, mp, f_scale, true, A);
     if (rc) return rc;
     LaunchTimer lt(ctx, "k_stage");
     launch_stage(ctx, A, mp);
@@ -820,8 +1105,46 @@ static void batch_ring_free(void *r) {
     delete b;
 }
 
-static int batch_launch(vx_ctx *ctx, const std::vector<StageArgs> &A, int step, bool mp) {
+// Strip height and kernel form of a batched launch, one for all items and by
+// the launch's total size, so that no shape is timed on the serving path (an
+// item alone would want short strips, which redo their warm-up rows in a
+// launch that fills the device anyway).  Up to BATCH_ROWS rows a SIMD: the row
+// form (measured, stages 0..5: twelve FP64 patches of 49 rows a SIMD 84 to 120
+// us as strips, 96 to 122 as rows; four mixed ones of 24 rows 38 to 55 as
+// strips, 34 to 61 as rows; a 1024 x 1024 patch of 18 rows 39 to 60 as strips,
+// 31 to 45 as rows); above: the strip height of the least rounds x (rows + 6), a round being
+// the resident wavefronts (three a SIMD) walking a strip each.
+constexpr int BATCH_ROWS = 20;
+static void batch_form(vx_ctx *ctx, std::vector<StageArgs> &A) {
+    const double simds = 4.0 * ctx->n_cu;
+    auto waves = [&](int ti) {
+        double w = 0;
+        for (const StageArgs &a : A) w += (double)a.nbx * ((a.p.n_x + ti - 1) / ti);
+        return w;
+    };
+    int form = 2, ti = ROWS_MAX;
+    if (waves(1) > BATCH_ROWS * simds) {
+        form = 0;
+        double best = 1e300;
+        for (int t = 96; t >= 8; t -= 4) {
+            const double cost = std::max(1.0, waves(t) / (3 * simds)) * (t + 2 * HALO);
+            if (cost < 0.99 * best) {
+                best = cost;
+                ti = t;
+            }
+        }
+    }
+    for (StageArgs &a : A) {
+        a.form = form;
+        a.TI = ti;
+        a.nstrip = (a.p.n_x + ti - 1) / ti;
+    }
+}
+
+static int batch_launch(vx_ctx *ctx, std::vector<StageArgs> &A, int step, bool mp) {
     if (A.empty()) return VX_OK;
+    batch_form(ctx, A);
+    const bool rows = A[0].form == 2;
     if (ctx->capturing) return fail(ctx, VX_EINVAL, "stage batch while a step graph is recorded");
     if (!ctx->batch_ring) {
         BatchRing *b = new BatchRing;
@@ -847,7 +1170,7 @@ static int batch_launch(vx_ctx *ctx, const std::vector<StageArgs> &A, int step, 
     int total = 0;
     for (int q = 0; q < n; q++) {
         start[q] = total;
-        total += A[q].nbx * ((A[q].nstrip + 3) / 4);
+        total += A[q].nbx * (rows ? A[q].nstrip : (A[q].nstrip + 3) / 4);
     }
     start[n] = total;
     int rc = check_hip(ctx, hipMemcpyAsync(d, h, BATCH_SLOT_BYTES, hipMemcpyHostToDevice, ctx->stream), "batch upload");
@@ -857,10 +1180,14 @@ static int batch_launch(vx_ctx *ctx, const std::vector<StageArgs> &A, int step, 
     if (rc) return rc;
     const StageArgs *dA = (const StageArgs *)d;
     const int *dS = (const int *)(d + sizeof(StageArgs) * BATCH_MAX);
-    dim3 grid((unsigned)total);
+    const int wf = rows ? ROWS_MAX + 4 : 4;
+    const size_t lds = rows ? sizeof(double) * 64 * RT_ARRAYS * wf : 0;
+    dim3 grid((unsigned)total), block(64 * wf);
 #define VX_BATCH(S)                                                                                   \
-    if (mp) k_stage_batch<S, true><<<grid, 256, 0, ctx->stream>>>(dA, dS, n);                        \
-    else k_stage_batch<S, false><<<grid, 256, 0, ctx->stream>>>(dA, dS, n);
+    if (mp && rows) k_stage_rows_batch<S, true><<<grid, block, lds, ctx->stream>>>(dA, dS, n);       \
+    else if (rows) k_stage_rows_batch<S, false><<<grid, block, lds, ctx->stream>>>(dA, dS, n);       \
+    else if (mp) k_stage_batch<S, true><<<grid, block, 0, ctx->stream>>>(dA, dS, n);                 \
+    else k_stage_batch<S, false><<<grid, block, 0, ctx->stream>>>(dA, dS, n);
     switch (step) {
         case 0: VX_BATCH(0) break;
         case 1: VX_BATCH(1) break;
@@ -893,7 +1220,7 @@ int vx_fct_stage_fused_batch(vx_ctx *ctx, const vx_stage_item *items, int n, int
         const vx_stage_item &it = items[q];
         StageArgs A;
         const bool mp = it.f_scale > 0.0;
-        int rc = stage_args(ctx, &it.p, step, it.dt, &it.fl, it.fin, it.fout, mp, it.f_scale, A);
+        int rc = stage_args(ctx, &it.p, step, it.dt, &it.fl, it.fin, it.fout, mp, it.f_scale, false, A);
         if (rc) return rc;
         (mp ? mixed : fp64).push_back(A);
     }
