@@ -42,60 +42,99 @@ struct PoissonArgs {
 };
 
 
-__device__ __forceinline__ double wave_incl_scan(double v) {
-    const int lane = threadIdx.x & 63;
-    for (int off = 1; off < 64; off <<= 1) {
-        double t = __shfl_up(v, off, 64);
-        if (lane >= off) v += t;
-    }
+// DPP move of a double; lanes outside row_mask or without a source lane get 0
+template <int CTRL, int ROW_MASK = 0xf>
+__device__ __forceinline__ double dpp_or_0(double v) {
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, ROW_MASK, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, ROW_MASK, 0xf, true);
+    return __hiloint2double(hi, lo);
+}
+
+// Inclusive scan over the wavefront's lanes: within rows of 16 by row shifts
+// of 1, 2, 4, 8, then row 0's total into row 1 and row 2's into row 3
+// (row_bcast:15), then rows 0-1's total into rows 2 and 3 (row_bcast:31).
+__device__ __forceinline__ double wave_scan_dpp(double v) {
+    v += dpp_or_0<0x111>(v);
+    v += dpp_or_0<0x112>(v);
+    v += dpp_or_0<0x114>(v);
+    v += dpp_or_0<0x118>(v);
+    v += dpp_or_0<0x142, 0xa>(v);
+    v += dpp_or_0<0x143, 0xc>(v);
     return v;
 }
 
-__device__ __forceinline__ double wave_sum(double v) {
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-    return v;
+__device__ __forceinline__ double lane63(double v) {
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), 63),
+                            __builtin_amdgcn_readlane(__double2loint(v), 63));
+}
+
+// sh + sl -= a xq, the product and sums error-free
+__device__ __forceinline__ void dd_sub(double &sh, double &sl, double a, double xq) {
+    const double p = a * xq;
+    const double e = fma(a, xq, -p);
+    const double tt = sh - p;
+    const double bv = tt - sh;
+    const double err = (sh - (tt - bv)) + (-p - bv);
+    sl = sl + (err - e);
+    sh = tt;
 }
 
 // ------------------------------------------------ multi-workgroup solve, n_f > 4096
-// Workgroup b owns the CHUNK consecutive entries [b*CHUNK, b*CHUNK + CHUNK).
-// One approximate solve of A c = v (the same steps as the single-workgroup
-// variant below) is three launches:
-//   k_pm_scan_s  S_i = sum_{k<i} v'_k with v'_0 = -sum_{k>=1} v_k, and per-chunk sums of S;
-//   k_pm_scan_y  d0 = mean(S), D_i = d0 - S_i (D_0 = 0), y_i = sum_{k<=i} D_k;
-//   k_pm_conv    c = M^-1 y - (M^-1 y)_0 with c_0 from row 0, x (+)= c, then either the
-//                next residual r = b - A x (double-double) with its per-chunk sums, or
-//                phi, Ex0 and E.
-// A sum across workgroups is formed from per-chunk partials that every workgroup
-// reads and adds in the same order, so all of them hold the same bits.  k_pm_conv
-// recomputes x on a 2-entry halo around its chunk (for the residual and E
-// stencils) and at the six entries around 0 (row 0 and Ex0) with the owner's
-// operations, so every copy of an entry has the owner's bits.  x and r alternate
-// between two buffers: a launch reads one and writes the other.
-constexpr int MT = 256, MW = MT / 64, MPER = 4, CHUNK = MT * MPER;
+// Workgroup b owns the chunk of CHUNK consecutive entries [b CHUNK, (b + 1)
+// CHUNK), wavefront w of it the sub-chunk w of 64 entries.  One approximate
+// solve of A c = v and the residual of the next round are one launch:
+//   S_i = sum_{k<i} v'_k with v'_0 = -tail, tail = sum_{k>=1} v_k,
+//   d0 = mean(S), D_i = d0 - S_i (D_0 = 0), y_i = sum_{k<=i} D_k,
+//   c = M^-1 y - (M^-1 y)_0 with c_0 from row 0, x (+)= c, then either the
+//   next residual r = b - A x (double-double) or phi, Ex0 and E.
+// Both prefix sums at a chunk's first entry follow from two numbers per earlier
+// chunk, the sum M of its v and the sum P of its local exclusive prefixes of v:
+//   S = -tail + sum_q M_q,   sum_{i<start} S_i = sum_q (M_q (start - end_q) + P_q) - tail (start - 1)
+// (and within a chunk the same over its sub-chunks), so the launch that forms v
+// writes M and P (k_pm_rhs for the first solve) and the next one needs no launch
+// in between.  The terms M (start - end) are up to n_f times what they sum to
+// (v is a difference of differences), so M, P and these sums are held in
+// double-double: in double, entries of phi that cancel lose their last bits.  Every
+// wavefront forms a sub-chunk's y from those sums by the same operations,
+// whichever workgroup it is in, so the y of a neighbour's sub-chunk, formed again
+// for the reach of M^-1, has the owner's bits; so have the x on a 2-entry halo
+// (for the residual and E stencils) and at the six entries around 0 (row 0 and
+// Ex0).  x and r alternate between two buffers: a launch reads one and writes
+// the other.
+// Bound by launch latency and each launch's chain (sums, two scans,
+// convolution, residual, sums).  32768 entries on an MI355X: 77 us as 13
+// launches (the two scans and the convolution apart), 42 us as 5.
+constexpr int SUB = 64, MW = 8, CHUNK = SUB * MW;
+constexpr int MT = 64 * (MW + 5);  // k_pm_solve: a wavefront per sub-chunk that it forms
 constexpr int HALO = 2;
 constexpr int CW = NG - 1 + HALO;  // y window margin: convolution reach + halo
 constexpr int NSPEC = 6;           // entries N-3, N-2, N-1, 0, 1, 2
+constexpr int YS = NSPEC + 2 * (NG - 1);  // y window of those entries
 
 __host__ __device__ constexpr int pm_chunks(int n) { return (n + CHUNK - 1) / CHUNK; }
 
-// Work layout (doubles): b | xa | xb | ra | rb | S | y | Pa[nb] | Pb[nb] | Ex0 on entry
+// M and P of a chunk or sub-chunk, double-double
+struct PmSum {
+    double mh, ml, ph, pl;
+};
+
+// Work layout (doubles): b | xa | xb | ra | rb | Ex0 on entry | per parity: the chunks'
+// sums, the sub-chunks'
 struct PmWork {
-    double *b, *xa, *xb, *ra, *rb, *S, *y, *Pa, *Pb, *ex0;
+    double *b, *xa, *xb, *ra, *rb, *ex0;
+    PmSum *sums[2];
 };
 __host__ __device__ inline PmWork pm_work(double *w, int n) {
-    const size_t N = n;
-    const int nb = pm_chunks(n);
+    const size_t N = n, ns = (size_t)pm_chunks(n) * (1 + MW);
     PmWork W;
     W.b = w;
     W.xa = w + N;
     W.xb = w + 2 * N;
     W.ra = w + 3 * N;
     W.rb = w + 4 * N;
-    W.S = w + 5 * N;
-    W.y = w + 6 * N;
-    W.Pa = w + 7 * N;
-    W.Pb = W.Pa + nb;
-    W.ex0 = W.Pb + nb;
+    W.ex0 = w + 5 * N;
+    W.sums[0] = (PmSum *)(W.ex0 + 1);
+    W.sums[1] = W.sums[0] + ns;
     return W;
 }
 
@@ -107,43 +146,14 @@ struct PoissonMB {
     int nb;
     PmWork W;
     const double *in;    // right-hand side of this solve (b, then residuals)
+    const PmSum *sums;   // its M, P
+    PmSum *sums_out;     // those of the next residual
     const double *x_in;  // x before this solve's correction
     double *x_out;       // x after it
     double *r_out;       // next residual
 };
 
 __device__ __forceinline__ int wrap(int u, int N) { return u < 0 ? u + N : (u >= N ? u - N : u); }
-
-// sum of v[lo..hi) in a fixed order; every lane of every wave gets the same bits
-__device__ __forceinline__ double wave_range_sum(const double *v, int lo, int hi) {
-    double s = 0.0;
-    for (int k = lo + (threadIdx.x & 63); k < hi; k += 64) s += v[k];
-    return wave_sum(s);
-}
-
-__device__ __forceinline__ double mb_sum(double v, double *lds) {
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    v = wave_sum(v);
-    if (lane == 0) lds[w] = v;
-    __syncthreads();
-    double r = ((lds[0] + lds[1]) + lds[2]) + lds[3];
-    __syncthreads();
-    return r;
-}
-
-// exclusive prefix of the per-thread totals over the workgroup
-__device__ __forceinline__ double mb_offset(double tot, double *lds) {
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    double inc = wave_incl_scan(tot);
-    double exc = __shfl_up(inc, 1, 64);
-    if (lane == 0) exc = 0.0;
-    if (lane == 63) lds[w] = inc;
-    __syncthreads();
-    double off = 0.0;
-    for (int k = 0; k < w; k++) off += lds[k];
-    __syncthreads();
-    return off + exc;
-}
 
 // (M^-1 y) at window position c: the periodic 33-tap convolution
 __device__ __forceinline__ double conv_at(const double *w, int c, const double *g) {
@@ -152,101 +162,136 @@ __device__ __forceinline__ double conv_at(const double *w, int c, const double *
     return s;
 }
 
-// b = dx^2 eps0_inv (charge + neutral) (EMSolver.cpp:157-167), its chunk sums
-// over entries >= 1, and the entry value of Ex0
-__global__ __launch_bounds__(MT) void k_pm_rhs(PoissonMB P) {
-    __shared__ double lds[MW];
+struct DD {
+    double h, l;
+};
+__device__ __forceinline__ DD dd_add(DD a, DD b) {
+    const double s = a.h + b.h, z = s - a.h;
+    return {s, ((a.h - (s - z)) + (b.h - z)) + (a.l + b.l)};
+}
+__device__ __forceinline__ DD dd_neg(DD a) { return {-a.h, -a.l}; }
+__device__ __forceinline__ DD dd_mul(DD a, double b) {
+    const double p = a.h * b;
+    return {p, __builtin_fma(a.h, b, -p) + a.l * b};
+}
+template <int CTRL, int ROW_MASK>
+__device__ __forceinline__ DD dd_step(DD v) {
+    return dd_add(v, {dpp_or_0<CTRL, ROW_MASK>(v.h), dpp_or_0<CTRL, ROW_MASK>(v.l)});
+}
+// sum over the wavefront's lanes (wave_scan_dpp's steps), the same in every lane
+__device__ __forceinline__ DD wave_dd_sum(DD v) {
+    v = dd_step<0x111, 0xf>(v);
+    v = dd_step<0x112, 0xf>(v);
+    v = dd_step<0x114, 0xf>(v);
+    v = dd_step<0x118, 0xf>(v);
+    v = dd_step<0x142, 0xa>(v);
+    v = dd_step<0x143, 0xc>(v);
+    return {lane63(v.h), lane63(v.l)};
+}
+
+// M and P of a wavefront's 64 entries v (entry 0 and entries past N passed as
+// 0) and of the workgroup's chunk of n_own entries, into out.  P is the sum of v_l
+// (n - 1 - l), n the wavefront's entries below N.
+__device__ __forceinline__ void pm_store_sums(double v, int n_own, PmSum *out, int nb, PmSum *ms) {
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, blk = blockIdx.x;
+    const int n = min(SUB, n_own - w * SUB);
+    const DD m = wave_dd_sum({v, 0.0}), p = wave_dd_sum(dd_mul({v, 0.0}, (double)max(n - 1 - lane, 0)));
+    if (lane == 0 && w < MW) {
+        const PmSum q{m.h, m.l, p.h, p.l};
+        ms[w] = q;
+        out[nb + blk * MW + w] = q;
+    }
+    __syncthreads();
+    if (w == 0) {  // lane k: sub-chunk k, moved to the chunk's end
+        DD M{0.0, 0.0}, P{0.0, 0.0};
+        if (lane < MW) {
+            const int end = min((lane + 1) * SUB, n_own);
+            M = {ms[lane].mh, ms[lane].ml};
+            P = dd_add({ms[lane].ph, ms[lane].pl}, dd_mul(M, (double)(n_own - end)));
+        }
+        M = wave_dd_sum(M);
+        P = wave_dd_sum(P);
+        if (lane == 0) out[blk] = {M.h, M.l, P.h, P.l};
+    }
+}
+
+// b = dx^2 eps0_inv (charge + neutral) (EMSolver.cpp:157-167), its sums over
+// entries >= 1, and the entry value of Ex0
+__global__ __launch_bounds__(CHUNK) void k_pm_rhs(PoissonMB P) {
+    __shared__ PmSum ms[MW];
     const vx_field_state &F = P.fs;
-    const int N = F.n_f, base = blockIdx.x * CHUNK + threadIdx.x * MPER;
-    const double te = vx_eps0_inv;
-    double s = 0.0;
-#pragma unroll
-    for (int k = 0; k < MPER; k++) {
-        const int i = base + k;
-        if (i < N) {
-            double v = te * (F.charge[i] + F.neutral[i]);
-            v *= F.dx2;
-            P.W.b[i] = v;
-            if (i >= 1) s += v;
-        }
+    const int N = F.n_f, i = blockIdx.x * CHUNK + threadIdx.x;
+    double v = 0.0;
+    if (i < N) {
+        v = vx_eps0_inv * (F.charge[i] + F.neutral[i]);
+        v *= F.dx2;
+        P.W.b[i] = v;
     }
-    const double tot = mb_sum(s, lds);
-    if (threadIdx.x == 0) {
-        P.W.Pa[blockIdx.x] = tot;
-        if (blockIdx.x == 0) *P.W.ex0 = *F.Ex0;
-    }
-}
-
-__global__ __launch_bounds__(MT) void k_pm_scan_s(PoissonMB P) {
-    __shared__ double lds[MW];
-    const int N = P.fs.n_f, blk = blockIdx.x, base = blk * CHUNK + threadIdx.x * MPER;
-    const double tail = wave_range_sum(P.W.Pa, 0, P.nb);
-    // S at the chunk's first entry: v'_0 = -tail plus the entries >= 1 before the chunk
-    const double start = blk == 0 ? 0.0 : -tail + wave_range_sum(P.W.Pa, 0, blk);
-    double e[MPER], tot = 0.0;
-#pragma unroll
-    for (int k = 0; k < MPER; k++) {
-        const int i = base + k;
-        e[k] = (i == 0) ? -tail : (i < N ? P.in[i] : 0.0);
-        tot += e[k];
-    }
-    double run = start + mb_offset(tot, lds);
-    double ssum = 0.0;
-#pragma unroll
-    for (int k = 0; k < MPER; k++) {
-        const int i = base + k;
-        if (i < N) {
-            P.W.S[i] = run;
-            ssum += run;
-        }
-        run += e[k];
-    }
-    const double t2 = mb_sum(ssum, lds);
-    if (threadIdx.x == 0) P.W.Pb[blk] = t2;
-}
-
-__global__ __launch_bounds__(MT) void k_pm_scan_y(PoissonMB P) {
-    __shared__ double lds[MW];
-    const int N = P.fs.n_f, blk = blockIdx.x, base = blk * CHUNK + threadIdx.x * MPER;
-    const double d0 = wave_range_sum(P.W.Pb, 0, P.nb) * P.invN;
-    // sum of D over the earlier chunks: (entries - [chunk 0]) * d0 - (chunk sum of S)
-    double sd = 0.0;
-    for (int k = threadIdx.x & 63; k < blk; k += 64) {
-        const int n = min(CHUNK, N - k * CHUNK) - (k == 0 ? 1 : 0);
-        sd += (double)n * d0 - P.W.Pb[k];
-    }
-    const double offD = wave_sum(sd);
-    double D[MPER], tot = 0.0;
-#pragma unroll
-    for (int k = 0; k < MPER; k++) {
-        const int i = base + k;
-        D[k] = (i == 0 || i >= N) ? 0.0 : d0 - P.W.S[i];
-        tot += D[k];
-    }
-    double run = offD + mb_offset(tot, lds);
-#pragma unroll
-    for (int k = 0; k < MPER; k++) {
-        const int i = base + k;
-        run += D[k];
-        if (i < N) P.W.y[i] = run;
-    }
+    pm_store_sums(i >= 1 ? v : 0.0, min(CHUNK, N - (int)blockIdx.x * CHUNK), P.sums_out, P.nb, ms);
+    if (i == 0) *P.W.ex0 = *F.Ex0;
 }
 
 // MODE 0: first solve (x = c); 1: refinement (x += c); both then form the next
 // residual.  MODE 2: last refinement, writes phi (x_out), Ex0 and E.
 template <int MODE>
-__global__ __launch_bounds__(MT) void k_pm_conv(PoissonMB P) {
+__global__ __launch_bounds__(MT) void k_pm_solve(PoissonMB P) {
     __shared__ double yw[CHUNK + 2 * CW];
-    __shared__ double ys[NSPEC + 2 * (NG - 1)];
+    __shared__ double ys[YS];
     __shared__ double xw[CHUNK + 2 * HALO];
     __shared__ double cs[NSPEC];
-    __shared__ double lds[MW];
+    __shared__ PmSum ms[MW];
     const vx_field_state &F = P.fs;
-    const int N = F.n_f, blk = blockIdx.x, lo = blk * CHUNK;
+    const int N = F.n_f, blk = blockIdx.x, lo = blk * CHUNK, nb = P.nb;
     const int n_own = min(CHUNK, N - lo);
-    const double *y = P.W.y;
-    for (int j = threadIdx.x; j < n_own + 2 * CW; j += MT) yw[j] = y[wrap(lo - CW + j, N)];
-    for (int j = threadIdx.x; j < NSPEC + 2 * (NG - 1); j += MT) ys[j] = y[wrap(-3 - (NG - 1) + j, N)];
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    // this thread's entry of x (chunk and halo) and b, loaded ahead of their use
+    const int j = threadIdx.x, gi = wrap(lo - HALO + j, N);
+    const bool own = j >= HALO && j < n_own + HALO, have = j < n_own + 2 * HALO;
+    const double xo = MODE > 0 && have ? P.x_in[gi] : 0.0;
+    const double bv = MODE < 2 && j < n_own ? P.W.b[lo + j] : 0.0;
+    const PmSum *C = P.sums, *U = C + nb;  // chunks, sub-chunks
+    // (sum v, sum v (pos - 1 - i)) of item q that ends at `end`, seen from pos
+    auto item = [](const PmSum &q, int pos, int end, DD &t, DD &g) {
+        const DD m{q.mh, q.ml};
+        t = dd_add(t, m);
+        g = dd_add(g, dd_add(dd_mul(m, (double)(pos - end)), {q.ph, q.pl}));
+    };
+    // over every chunk: tail and d0
+    DD t{0.0, 0.0}, g{0.0, 0.0};
+    for (int q = lane; q < nb; q += 64) item(C[q], N, min((q + 1) * CHUNK, N), t, g);
+    const DD tail = wave_dd_sum(t);
+    g = dd_add(wave_dd_sum(g), dd_mul(tail, -(double)(N - 1)));
+    const double d0 = (g.h + g.l) * P.invN, tl = tail.h + tail.l;
+    // y of sub-chunk s, into the windows it reaches
+    auto sub_y = [&](int s) {
+        const int b = s / MW, i0 = s * SUB, i = i0 + lane;
+        const double in = i < N ? P.in[i] : 0.0;
+        // S and the sum of D before the sub-chunk
+        DD a{0.0, 0.0}, h{0.0, 0.0};
+        for (int q = lane; q < b; q += 64) item(C[q], i0, (q + 1) * CHUNK, a, h);
+        if (lane < s - b * MW) item(U[b * MW + lane], i0, (b * MW + lane + 1) * SUB, a, h);
+        a = dd_add(wave_dd_sum(a), dd_neg(tail));
+        h = dd_add(wave_dd_sum(h), dd_mul(tail, -(double)(i0 - 1)));
+        h = dd_add(dd_mul({d0, 0.0}, (double)(i0 - 1)), dd_neg(h));
+        // (entry 0: S = 0, D = 0)
+        const double S = s == 0 ? 0.0 : a.h + a.l, Y = s == 0 ? 0.0 : h.h + h.l;
+        const double v = i == 0 ? -tl : in;
+        const double Si = S + dpp_or_0<0x138>(wave_scan_dpp(v));
+        const double Di = (i == 0 || i >= N) ? 0.0 : d0 - Si;
+        const double y = Y + wave_scan_dpp(Di);
+        if (i >= N) return;
+        for (int img = -N; img <= N; img += N) {
+            const int p = i + img - lo + CW;
+            if (p >= 0 && p < n_own + 2 * CW) yw[p] = y;
+        }
+        const int e = i < N - i ? i + 3 + NG - 1 : i - N + 3 + NG - 1;
+        if (e >= 0 && e < YS) ys[e] = y;
+    };
+    // the chunk's sub-chunks, the neighbours' and those around entry 0 (the last
+    // one may be shorter than the window, hence the one before it too)
+    const int ns = (N + SUB - 1) / SUB, s0 = blk * MW;
+    const int sub = w < MW ? s0 + w : w == MW ? s0 - 1 : w == MW + 1 ? s0 + MW : w == MW + 2 ? 0 : ns - (w - MW - 2);
+    if (sub >= 0 && sub < ns) sub_y(sub);
     __syncthreads();
     if (threadIdx.x < NSPEC) cs[threadIdx.x] = conv_at(ys, threadIdx.x + NG - 1, P.g);
     __syncthreads();
@@ -255,29 +300,20 @@ __global__ __launch_bounds__(MT) void k_pm_conv(PoissonMB P) {
     const double c0 = P.in[0] - (((P.w1 * (cs[4] - cp0) + P.w2 * (cs[5] - cp0)) + P.w2 * (cs[1] - cp0)) +
                                  P.w1 * (cs[2] - cp0));
     // x on the chunk and its halo
-    for (int j = threadIdx.x; j < n_own + 2 * HALO; j += MT) {
-        const int gi = wrap(lo - HALO + j, N);
-        const double c = (gi == 0) ? c0 : conv_at(yw, j + NG - 1, P.g) - cp0;
-        const double xn = MODE == 0 ? c : P.x_in[gi] + c;
+    if (have) {
+        const double c = gi == 0 ? c0 : conv_at(yw, j + NG - 1, P.g) - cp0;
+        const double xn = MODE == 0 ? c : xo + c;
         xw[j] = xn;
-        if (j >= HALO && j < n_own + HALO) P.x_out[gi] = xn;
+        if (own) P.x_out[gi] = xn;
     }
     __syncthreads();
     if (MODE < 2) {
         // r = b - A x in double-double, rounded once (term order as the oracle's)
-        double s = 0.0;
-        for (int j = threadIdx.x; j < n_own; j += MT) {
-            const int i = lo + j, c = j + HALO;
-            double sh = P.W.b[i], sl = 0.0;
-            auto sub = [&](double a, double xv) {
-                double p = a * xv;
-                double e = fma(a, xv, -p);
-                double tt = sh - p;
-                double bv = tt - sh;
-                double err = (sh - (tt - bv)) + (-p - bv);
-                sl = sl + (err - e);
-                sh = tt;
-            };
+        double r = 0.0;
+        const int i = lo + j, c = j + HALO;
+        if (j < n_own) {
+            double sh = bv, sl = 0.0;
+            auto sub = [&](double a, double xv) { dd_sub(sh, sl, a, xv); };
             if (i == 0) {
                 sub(1.0, xw[c]); sub(P.w1, xw[c + 1]); sub(P.w2, xw[c + 2]); sub(P.w2, xw[c - 2]);
                 sub(P.w1, xw[c - 1]);
@@ -288,30 +324,25 @@ __global__ __launch_bounds__(MT) void k_pm_conv(PoissonMB P) {
                     sub(cf[d + 2], xw[c + d]);
                 }
             }
-            const double r = sh + sl;
+            r = sh + sl;
             P.r_out[i] = r;
-            if (i >= 1) s += r;
         }
-        const double tot = mb_sum(s, lds);
-        if (threadIdx.x == 0) P.W.Pa[blk] = tot;
+        pm_store_sums(i >= 1 ? r : 0.0, n_own, P.sums_out, nb, ms);
     } else {
         // EMSolver.cpp:191: Ex0 += -(E(-1) + E(0)) * 0.5 with the entry Ex0, from phi
         // at N-3..N-1, 0..2 (recomputed here with the owners' operations)
         double ps[NSPEC];
 #pragma unroll
         for (int k = 0; k < NSPEC; k++) {
-            const int gi = wrap(k - 3, N);
-            ps[k] = P.x_in[gi] + (k == 3 ? c0 : cs[k] - cp0);
+            ps[k] = P.x_in[wrap(k - 3, N)] + (k == 3 ? c0 : cs[k] - cp0);
         }
         const double ex0 = *P.W.ex0, fc = F.field_coef;
         const double e_m1 = -fc * (8 * (ps[3] - ps[1]) - ps[4] + ps[0]) + ex0;
         const double e_0 = -fc * (8 * (ps[4] - ps[2]) - ps[5] + ps[1]) + ex0;
         const double ex0n = ex0 + -(e_m1 + e_0) * 0.5;
         if (blk == 0 && threadIdx.x == 0) *F.Ex0 = ex0n;
-        for (int j = threadIdx.x; j < n_own; j += MT) {
-            const int c = j + HALO;
-            F.E[lo + j] = -fc * (8 * (xw[c + 1] - xw[c - 1]) - xw[c + 2] + xw[c - 2]) + ex0n;
-        }
+        const int c = j + HALO;
+        if (j < n_own) F.E[lo + j] = -fc * (8 * (xw[c + 1] - xw[c - 1]) - xw[c + 2] + xw[c - 2]) + ex0n;
     }
 }
 
@@ -355,32 +386,6 @@ struct SmallLds {
         return v[p + (p >> 3)];
     }
 };
-
-// DPP move of a double; lanes outside row_mask or without a source lane get 0
-template <int CTRL, int ROW_MASK = 0xf>
-__device__ __forceinline__ double dpp_or_0(double v) {
-    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, ROW_MASK, 0xf, true);
-    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, ROW_MASK, 0xf, true);
-    return __hiloint2double(hi, lo);
-}
-
-// Inclusive scan over the wavefront's lanes: within rows of 16 by row shifts
-// of 1, 2, 4, 8, then row 0's total into row 1 and row 2's into row 3
-// (row_bcast:15), then rows 0-1's total into rows 2 and 3 (row_bcast:31).
-__device__ __forceinline__ double wave_scan_dpp(double v) {
-    v += dpp_or_0<0x111>(v);
-    v += dpp_or_0<0x112>(v);
-    v += dpp_or_0<0x114>(v);
-    v += dpp_or_0<0x118>(v);
-    v += dpp_or_0<0x142, 0xa>(v);
-    v += dpp_or_0<0x143, 0xc>(v);
-    return v;
-}
-
-__device__ __forceinline__ double lane63(double v) {
-    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), 63),
-                            __builtin_amdgcn_readlane(__double2loint(v), 63));
-}
 
 // Workgroup sum of v; every thread gets the same bits.
 __device__ __forceinline__ double block_sum1(double v, double (&part)[2][PW1], int &buf) {
@@ -544,15 +549,6 @@ __device__ void residual_one(const PoissonArgs &P, const double *b, const double
     double w[CH + 4];
 #pragma unroll
     for (int m = 0; m < CH + 4; m++) w[m] = L.at(base - 2 + m);
-    auto sub = [](double &sh, double &sl, double a, double xq) {
-        const double p = a * xq;
-        const double e = fma(a, xq, -p);
-        const double tt = sh - p;
-        const double bv = tt - sh;
-        const double err = (sh - (tt - bv)) + (-p - bv);
-        sl = sl + (err - e);
-        sh = tt;
-    };
     const double cf[5] = {P.w2, P.w1, P.w3, P.w1, P.w2};
 #pragma unroll
     for (int k = 0; k < CH; k++) {
@@ -563,17 +559,17 @@ __device__ void residual_one(const PoissonArgs &P, const double *b, const double
 #pragma unroll
         for (int d = -2; d <= 2; d++) {
             const int j = i + d;
-            sub(sh, sl, (j == 0 || j == N) ? 0.0 : cf[d + 2], w[k + d + 2]);
+            dd_sub(sh, sl, (j == 0 || j == N) ? 0.0 : cf[d + 2], w[k + d + 2]);
         }
         r[k] = i < N ? sh + sl : 0.0;
     }
     if (base == 0) {  // row 0
         double sh = b[0], sl = 0.0;
-        sub(sh, sl, 1.0, L.at(0));
-        sub(sh, sl, P.w1, L.at(1));
-        sub(sh, sl, P.w2, L.at(2));
-        sub(sh, sl, P.w2, L.at(N - 2));
-        sub(sh, sl, P.w1, L.at(N - 1));
+        dd_sub(sh, sl, 1.0, L.at(0));
+        dd_sub(sh, sl, P.w1, L.at(1));
+        dd_sub(sh, sl, P.w2, L.at(2));
+        dd_sub(sh, sl, P.w2, L.at(N - 2));
+        dd_sub(sh, sl, P.w1, L.at(N - 1));
         r[0] = sh + sl;
     }
 }
@@ -674,84 +670,103 @@ struct MaxArgs {
 
 __device__ __forceinline__ int fidx(int ne, int i, int slot) { return slot * ne + i; }
 
-// EMSolver.cpp:479-553
-__global__ void k_maxwell_rhs(MaxArgs A) {
+// A field stage is two launches (three, with the faces apart, took 12.6 us at
+// 4096 elements on an MI355X, these 8.9): the right-hand sides, which read
+// slot 1 at the neighbouring elements and write slot step + 2, then the update
+// of slot 1 and A^2 at the faces from it.  A face's four potentials are formed
+// again from the update's inputs rather than read from slot 1, which the launch
+// writes: those inputs (slots 0 and 2..step + 2) are not written by it.  At the
+// last stage, whose update reads slot 1, the first launch forms the new value
+// into slot 0 (which nothing reads any more) and the second copies it.
+
+// EMSolver.cpp:479-553; blockIdx.y = 0: By, Ez, Az; 1: Bz, Ey, Ay (each set
+// reads only itself)
+__device__ __forceinline__ void maxwell_last(double *y, int ne, int i, const double *b, double k5) {
+    double t = y[fidx(ne, i, 1)] + b[0] * y[fidx(ne, i, 2)];
+#pragma unroll
+    for (int k = 1; k < 5; k++) t = t + b[k] * y[fidx(ne, i, k + 2)];
+    t = t + b[5] * k5;
+    y[fidx(ne, i, 0)] = t;
+}
+
+__global__ __launch_bounds__(256) void k_maxwell_rhs(MaxArgs A) {
     const vx_field_state &F = A.fs;
     const int ne = F.n_e, npre = F.n_prepad, N = F.n_f;
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= ne) return;
-    const int s = fidx(ne, i, A.step + 2);
-    double *By = F.By, *Bz = F.Bz, *Ey = F.Ey, *Ez = F.Ez, *Ay = F.Ay, *Az = F.Az;
-    const double dx_inv = A.dx_inv;
-    double rBy = 0, rBz = 0, rEy = 0, rEz = 0, rAy = 0, rAz = 0;
-    int i1 = fidx(ne, i, 1);
+    const bool z = blockIdx.y == 0;  // By, Ez, Az; else Bz, Ey, Ay
+    double *B = z ? F.By : F.Bz, *E = z ? F.Ez : F.Ey, *V = z ? F.Az : F.Ay;
+    const int s = fidx(ne, i, A.step + 2), i1 = fidx(ne, i, 1);
+    const double dx_inv = A.dx_inv, db = z ? dx_inv : -dx_inv, de = z ? dx_inv : -dx_inv;
+    double rB = 0, rE = 0, rV = 0;
     if (i == 0) {
-        int ip1 = fidx(ne, i + 1, 1);
-        rBy = dx_inv * (Ez[ip1] - Ez[i1]);
-        rBz = -dx_inv * (Ey[ip1] - Ey[i1]);
-        const double by0 = A.drive ? A.drive[0] : A.by0, bz0 = A.drive ? A.drive[1] : A.bz0;
-        rEy = -dx_inv * (Bz[i1] - bz0) * vx_eps0_inv * vx_mu_inv;
-        rEz = dx_inv * (By[i1] - by0) * vx_eps0_inv * vx_mu_inv;
-        rAy = -Ey[i1];
-        rAz = -Ez[i1];
+        const double b0 = z ? (A.drive ? A.drive[0] : A.by0) : (A.drive ? A.drive[1] : A.bz0);
+        rB = db * (E[i1 + 1] - E[i1]);
+        rE = de * (B[i1] - b0) * vx_eps0_inv * vx_mu_inv;
+        rV = -E[i1];
     } else if (i < npre || (i >= npre + N && i < ne - 2)) {
-        int ip1 = fidx(ne, i + 1, 1), in1 = fidx(ne, i - 1, 1);
-        rBy = dx_inv * (Ez[ip1] - Ez[i1]);
-        rBz = -dx_inv * (Ey[ip1] - Ey[i1]);
-        rEy = -dx_inv * (Bz[i1] - Bz[in1]) * vx_eps0_inv * vx_mu_inv;
-        rEz = dx_inv * (By[i1] - By[in1]) * vx_eps0_inv * vx_mu_inv;
-        rAy = -Ey[i1];
-        rAz = -Ez[i1];
+        rB = db * (E[i1 + 1] - E[i1]);
+        rE = de * (B[i1] - B[i1 - 1]) * vx_eps0_inv * vx_mu_inv;
+        rV = -E[i1];
     } else if (i >= npre && i < npre + N) {
         const double c1 = -1.0 / 24;
         const double c2 = 9.0 / 8.0;
-        int ip1 = fidx(ne, i + 1, 1), in1 = fidx(ne, i - 1, 1);
-        int ip2 = fidx(ne, i + 2, 1), in2 = fidx(ne, i - 2, 1);
-        double Jc = F.J[i - npre];
-        rBy = dx_inv * (c1 * (Ez[ip2] - Ez[in1]) + c2 * (Ez[ip1] - Ez[i1]));
-        rBz = -dx_inv * (c1 * (Ey[ip2] - Ey[in1]) + c2 * (Ey[ip1] - Ey[i1]));
-        rEy = -dx_inv * (c1 * (Bz[ip1] - Bz[in2]) + c2 * (Bz[i1] - Bz[in1])) * vx_eps0_inv * vx_mu_inv -
-              vx_eps0_inv * Jc * Ay[i1];
-        rEz = dx_inv * (c1 * (By[ip1] - By[in2]) + c2 * (By[i1] - By[in1])) * vx_eps0_inv * vx_mu_inv -
-              vx_eps0_inv * Jc * Az[i1];
-        rAy = -Ey[i1];
-        rAz = -Ez[i1];
+        const double Jc = F.J[i - npre];
+        rB = db * (c1 * (E[i1 + 2] - E[i1 - 1]) + c2 * (E[i1 + 1] - E[i1]));
+        rE = de * (c1 * (B[i1 + 1] - B[i1 - 2]) + c2 * (B[i1] - B[i1 - 1])) * vx_eps0_inv * vx_mu_inv -
+             vx_eps0_inv * Jc * V[i1];
+        rV = -E[i1];
     }
-    By[s] = rBy; Bz[s] = rBz; Ey[s] = rEy; Ez[s] = rEz; Ay[s] = rAy; Az[s] = rAz;
+    B[s] = rB;
+    E[s] = rE;
+    V[s] = rV;
+    if (A.step == 5) {
+        maxwell_last(B, ne, i, A.b, rB);
+        maxwell_last(E, ne, i, A.b, rE);
+        maxwell_last(V, ne, i, A.b, rV);
+    }
 }
 
-// EMSolver.cpp:204-338; one thread per element and field (blockIdx.y): the
-// six fields' updates are independent
-__global__ void k_maxwell_update(MaxArgs A) {
+// Slot 1 of element i after the stage's update (EMSolver.cpp:204-338)
+__device__ __forceinline__ double maxwell_new(const double *y, const MaxArgs &A, int ne, int i) {
+    if (A.step > 4) return y[fidx(ne, i, 0)];
+    double t = y[fidx(ne, i, 0)] + A.a[0] * y[fidx(ne, i, 2)];
+    for (int k = 1; k <= A.step; k++) t = t + A.a[k] * y[fidx(ne, i, k + 2)];
+    return t;
+}
+
+// The update, one thread per element and field (blockIdx.y 0..3: By, Bz, Ey,
+// Ez), and at blockIdx.y = 4 Ay, Az and A^2 at the faces (EMSolver.cpp:555-619;
+// a_squared[n_f] is never written by the reference)
+constexpr int MXT = 256;
+__global__ __launch_bounds__(MXT) void k_maxwell_update(MaxArgs A) {
     const vx_field_state &F = A.fs;
-    const int ne = F.n_e;
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= ne) return;
+    const int ne = F.n_e, e0 = blockIdx.x * MXT, i = e0 + (int)threadIdx.x;
     const int v = blockIdx.y;
-    double *y = v == 0 ? F.By : v == 1 ? F.Bz : v == 2 ? F.Ey : v == 3 ? F.Ez : v == 4 ? F.Ay : F.Az;
-    if (A.step <= 4) {
-        double t = y[fidx(ne, i, 0)] + A.a[0] * y[fidx(ne, i, 2)];
-        for (int k = 1; k <= A.step; k++) t = t + A.a[k] * y[fidx(ne, i, k + 2)];
-        y[fidx(ne, i, 1)] = t;
-    } else {
-        double t = y[fidx(ne, i, 1)] + A.b[0] * y[fidx(ne, i, 2)];
-        for (int k = 1; k < 6; k++) t = t + A.b[k] * y[fidx(ne, i, k + 2)];
-        y[fidx(ne, i, 0)] = t;
-        y[fidx(ne, i, 1)] = t;
+    if (v < 4) {
+        if (i >= ne) return;
+        double *y = v == 0 ? F.By : v == 1 ? F.Bz : v == 2 ? F.Ey : F.Ez;
+        y[fidx(ne, i, 1)] = maxwell_new(y, A, ne, i);
+        return;
     }
-}
-
-// EMSolver.cpp:555-619; a_squared[n_f] is never written by the reference
-__global__ void k_faces(vx_field_state F) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= F.n_f) return;
-    const int ne = F.n_e, np_ = F.n_prepad;
-    const double *Ay = F.Ay, *Az = F.Az;
-    double ay = face_weno(Ay[fidx(ne, np_ + i - 2, 1)], Ay[fidx(ne, np_ + i - 1, 1)],
-                          Ay[fidx(ne, np_ + i, 1)], Ay[fidx(ne, np_ + i + 1, 1)]);
-    double az = face_weno(Az[fidx(ne, np_ + i - 2, 1)], Az[fidx(ne, np_ + i - 1, 1)],
-                          Az[fidx(ne, np_ + i, 1)], Az[fidx(ne, np_ + i + 1, 1)]);
-    F.a2[i] = (ay * ay) + (az * az);
+    __shared__ double ay[MXT + 3], az[MXT + 3];  // elements e0 - 2 .. e0 + MXT
+    for (int k = threadIdx.x; k < MXT + 3; k += MXT) {
+        const int e = e0 - 2 + k;
+        if (e < 0 || e >= ne) continue;
+        const double y = maxwell_new(F.Ay, A, ne, e), z = maxwell_new(F.Az, A, ne, e);
+        ay[k] = y;
+        az[k] = z;
+        if (k >= 2 && k < MXT + 2) {
+            F.Ay[fidx(ne, e, 1)] = y;
+            F.Az[fidx(ne, e, 1)] = z;
+        }
+    }
+    __syncthreads();
+    const int face = i - F.n_prepad, k = (int)threadIdx.x;
+    if (face < 0 || face >= F.n_f) return;
+    const double y = face_weno(ay[k], ay[k + 1], ay[k + 2], ay[k + 3]);
+    const double z = face_weno(az[k], az[k + 1], az[k + 2], az[k + 3]);
+    F.a2[face] = (y * y) + (z * z);
 }
 
 __global__ void k_neutralize(vx_field_state F) {
@@ -767,8 +782,12 @@ __global__ void k_neutralize(vx_field_state F) {
 // until the process ends.  Host code never uses this name as an address: the
 // device address comes from hipGetSymbolAddress, once per device, with that
 // device current (scratch_address, at context creation).
-constexpr size_t NOALLOC_WORK =
-    7 * (size_t)VX_POISSON_NOALLOC_MAX_NF + 2 * (size_t)pm_chunks(VX_POISSON_NOALLOC_MAX_NF) + 1;
+__host__ __device__ constexpr size_t pm_work_elems(int n) { return 7 * (size_t)n + 2 * (((size_t)n + 1023) / 1024) + 1; }
+constexpr size_t NOALLOC_WORK = pm_work_elems(VX_POISSON_NOALLOC_MAX_NF);
+// pm_work's 5 n + 1 doubles and 72 per chunk of sums fit for
+// every n that the multi-workgroup solve serves
+static_assert(5 * 4097 + 1 + pm_chunks(4097) * 2 * 4 * (1 + MW) <= pm_work_elems(4097), "work array");
+static_assert(2 * CHUNK > 2 * 4 * (1 + MW), "sums per chunk against 2 doubles per entry");
 static __device__ __align__(256) double scratch[NOALLOC_WORK];
 constexpr int MAX_DEVICES = 64;
 static std::mutex scratch_mu;
@@ -805,7 +824,7 @@ int vx_noalloc_scratch_init(vx_ctx *ctx) {
 
 extern "C" {
 
-size_t vx_field_work_elems(int32_t n_f) { return (size_t)7 * n_f + 2 * (size_t)pm_chunks(n_f) + 1; }
+size_t vx_field_work_elems(int32_t n_f) { return pm_work_elems(n_f); }
 
 static int poisson(vx_ctx *ctx, const vx_field_state *fs, double *work) {
     int rc = validate_fs(ctx, fs);
@@ -846,7 +865,8 @@ static int poisson(vx_ctx *ctx, const vx_field_state *fs, double *work) {
     M.W = pm_work(work, fs->n_f);
     const PmWork &W = M.W;
     const unsigned nb = (unsigned)M.nb;
-    k_pm_rhs<<<nb, MT, 0, ctx->stream>>>(M);
+    M.sums_out = W.sums[0];
+    k_pm_rhs<<<nb, CHUNK, 0, ctx->stream>>>(M);
     // four approximate solves: of b (x = c), then of three residuals (x += c)
     const double *in[4] = {W.b, W.ra, W.rb, W.ra};
     double *r_out[4] = {W.ra, W.rb, W.ra, nullptr};
@@ -857,11 +877,11 @@ static int poisson(vx_ctx *ctx, const vx_field_state *fs, double *work) {
         M.r_out = r_out[s];
         M.x_in = x_in[s];
         M.x_out = x_out[s];
-        k_pm_scan_s<<<nb, MT, 0, ctx->stream>>>(M);
-        k_pm_scan_y<<<nb, MT, 0, ctx->stream>>>(M);
-        if (s == 0) k_pm_conv<0><<<nb, MT, 0, ctx->stream>>>(M);
-        else if (s < 3) k_pm_conv<1><<<nb, MT, 0, ctx->stream>>>(M);
-        else k_pm_conv<2><<<nb, MT, 0, ctx->stream>>>(M);
+        M.sums = W.sums[s & 1];
+        M.sums_out = W.sums[~s & 1];
+        if (s == 0) k_pm_solve<0><<<nb, MT, 0, ctx->stream>>>(M);
+        else if (s < 3) k_pm_solve<1><<<nb, MT, 0, ctx->stream>>>(M);
+        else k_pm_solve<2><<<nb, MT, 0, ctx->stream>>>(M);
     }
     return check_launch(ctx, "k_poisson");
 }
@@ -902,13 +922,11 @@ static int maxwell_stage(vx_ctx *ctx, const vx_field_state *fs, int step, double
         a[5] = 0;
         for (int k = 0; k < 6; k++) A.b[k] = vx::rk_a[5][k] * dt - a[k];
     }
-    unsigned g = (unsigned)((fs->n_e + 255) / 256);
-    k_maxwell_rhs<<<g, 256, 0, ctx->stream>>>(A);
+    unsigned g = (unsigned)((fs->n_e + MXT - 1) / MXT);
+    k_maxwell_rhs<<<dim3(g, 2), MXT, 0, ctx->stream>>>(A);
     if ((rc = check_launch(ctx, "k_maxwell_rhs"))) return rc;
-    k_maxwell_update<<<dim3(g, 6), 256, 0, ctx->stream>>>(A);
-    if ((rc = check_launch(ctx, "k_maxwell_update"))) return rc;
-    k_faces<<<(unsigned)((fs->n_f + 255) / 256), 256, 0, ctx->stream>>>(*fs);
-    return check_launch(ctx, "k_faces");
+    k_maxwell_update<<<dim3(g, 5), MXT, 0, ctx->stream>>>(A);
+    return check_launch(ctx, "k_maxwell_update");
 }
 
 extern "C" {
@@ -935,7 +953,9 @@ int vx_neutralize(vx_ctx *ctx, const vx_field_state *fs) {
 
 // EMSolver.cpp:631-664 on the device: pc = max_i (the per-cell term), each term
 // with the host code's operations; max is exact, so the order does not matter.
-constexpr int CFL_MAXSP = 8;
+// One workgroup per CFL_CHUNK cells writes its maximum, and the host takes the
+// maximum of at most CFL_WG of them.
+constexpr int CFL_MAXSP = 8, CFL_CHUNK = 1024, CFL_WG = 64;
 struct CflArgs {
     vx_field_state fs;
     int n_species;
@@ -943,11 +963,11 @@ struct CflArgs {
     double dpsMax;
 };
 
-__global__ __launch_bounds__(1024) void k_cfl(CflArgs A, double *out) {
+__global__ __launch_bounds__(256) void k_cfl(CflArgs A, double *out) {
     const vx_field_state &F = A.fs;
-    __shared__ double part[16];
+    __shared__ double part[4];
     double pc = 0.0;
-    for (int i = threadIdx.x; i < F.n_f; i += 1024) {
+    for (int i = blockIdx.x * 256 + threadIdx.x; i < F.n_f; i += 256 * gridDim.x) {
         const double Azv = F.Az[i], Ayv = F.Ay[i];
         const double As = Ayv * Ayv + Azv * Azv;
         double temp = 0.0;
@@ -966,25 +986,15 @@ __global__ __launch_bounds__(1024) void k_cfl(CflArgs A, double *out) {
     __syncthreads();
     if (threadIdx.x == 0) {
         double r = 0.0;
-        for (int k = 0; k < 16; k++) r = (r < part[k]) ? part[k] : r;
-        *out = r;
+        for (int k = 0; k < 4; k++) r = (r < part[k]) ? part[k] : r;
+        out[blockIdx.x] = r;
     }
 }
 
-extern "C" {
-
-int vx_cfl_bound_async(vx_ctx *ctx, const vx_field_state *fs, int n_species, const double *q, const double *m,
-                       const double *dp_finest) {
-    int rc = validate_fs(ctx, fs);
-    if (rc) return rc;
-    if (n_species < 1 || n_species > CFL_MAXSP) return fail(ctx, VX_EINVAL, "cfl: %d species", n_species);
-    if (ctx->capturing) return fail(ctx, VX_EINVAL, "cfl bound while a step graph is recorded");
-    if (!ctx->cfl_dev) {
-        if ((rc = check_hip(ctx, hipMalloc((void **)&ctx->cfl_dev, sizeof(double)), "cfl buffer"))) return rc;
-        if ((rc = check_hip(ctx, hipHostMalloc((void **)&ctx->cfl_host, sizeof(double)), "cfl pinned"))) return rc;
-        if ((rc = check_hip(ctx, hipEventCreateWithFlags(&ctx->cfl_ev, hipEventDisableTiming), "cfl event")))
-            return rc;
-    }
+// Launches k_cfl into `out` (device-visible, CFL_WG doubles); returns the number
+// of maxima it writes.
+static int cfl_launch(vx_ctx *ctx, const vx_field_state *fs, int n_species, const double *q, const double *m,
+                      const double *dp_finest, double *out) {
     CflArgs A;
     A.fs = *fs;
     A.n_species = n_species;
@@ -995,11 +1005,34 @@ int vx_cfl_bound_async(vx_ctx *ctx, const vx_field_state *fs, int n_species, con
         A.dps[i] = 1 / dp_finest[i];
         A.dpsMax = std::max(A.dpsMax, std::fabs(q[i]) * A.dps[i]);
     }
-    k_cfl<<<1, 1024, 0, ctx->stream>>>(A, ctx->cfl_dev);
-    if ((rc = check_launch(ctx, "k_cfl"))) return rc;
-    rc = check_hip(ctx, hipMemcpyAsync(ctx->cfl_host, ctx->cfl_dev, sizeof(double), hipMemcpyDeviceToHost,
-                                       ctx->stream), "cfl copy");
+    const int n = std::min((fs->n_f + CFL_CHUNK - 1) / CFL_CHUNK, CFL_WG);
+    k_cfl<<<n, 256, 0, ctx->stream>>>(A, out);
+    return n;
+}
+
+static double cfl_bound(double c_dx, const double *host, int n) {
+    double pc = 0.0;
+    for (int k = 0; k < n; k++) pc = std::max(pc, host[k]);
+    return 1.0 / std::max((c_dx + pc), 1e-40);
+}
+
+extern "C" {
+
+int vx_cfl_bound_async(vx_ctx *ctx, const vx_field_state *fs, int n_species, const double *q, const double *m,
+                       const double *dp_finest) {
+    int rc = validate_fs(ctx, fs);
     if (rc) return rc;
+    if (n_species < 1 || n_species > CFL_MAXSP) return fail(ctx, VX_EINVAL, "cfl: %d species", n_species);
+    if (ctx->capturing) return fail(ctx, VX_EINVAL, "cfl bound while a step graph is recorded");
+    if (!ctx->cfl_ev &&
+        (rc = check_hip(ctx, hipEventCreateWithFlags(&ctx->cfl_ev, hipEventDisableTiming), "cfl event")))
+        return rc;
+    // the maxima go straight to pinned memory
+    if (!ctx->cfl_host &&
+        (rc = check_hip(ctx, hipHostMalloc((void **)&ctx->cfl_host, sizeof(double) * CFL_WG), "cfl pinned")))
+        return rc;
+    ctx->cfl_n = cfl_launch(ctx, fs, n_species, q, m, dp_finest, ctx->cfl_host);
+    if ((rc = check_launch(ctx, "k_cfl"))) return rc;
     if ((rc = check_hip(ctx, hipEventRecord(ctx->cfl_ev, ctx->stream), "cfl event record"))) return rc;
     ctx->cfl_c_dx = vx_cs / fs->dx_f;
     ctx->cfl_pending = true;
@@ -1022,16 +1055,30 @@ int vx_cfl_result(vx_ctx *ctx, double *out) {
     int rc = check_hip(ctx, hipEventSynchronize(ctx->cfl_ev), "cfl wait");
     if (rc) return rc;
     ctx->cfl_pending = false;
-    *out = 1.0 / std::max((ctx->cfl_c_dx + *ctx->cfl_host), 1e-40);
+    *out = cfl_bound(ctx->cfl_c_dx, ctx->cfl_host, ctx->cfl_n);
     return VX_OK;
 }
 
-// EMSolver.cpp:631-664, evaluated on the host from downloaded arrays (the
-// reference indexes the slot-0 fields without the n_prepad offset).
+// EMSolver.cpp:631-664 (the reference indexes the slot-0 fields without the
+// n_prepad offset): the maxima on the device for the species the kernel holds,
+// through the field state's work array (a pinned buffer of its own would cost
+// each new context 0.3 ms), else, and without a work array, on the host from
+// downloaded arrays (five copies: 60 us at 4096 cells, 190 at 32768; one copy of
+// the maxima and the launch: 20 us).
 int vx_cfl_bound(vx_ctx *ctx, const vx_field_state *fs, int n_species, const double *q,
                  const double *m, const double *dp_finest, double *out) {
     int rc = validate_fs(ctx, fs);
     if (rc) return rc;
+    if (ctx->capturing) return fail(ctx, VX_EINVAL, "cfl bound while a step graph is being recorded");
+    if (fs->work && n_species >= 0 && n_species <= CFL_MAXSP) {
+        // (n <= n_f / CFL_CHUNK + 1 of the work array's more than 7 n_f doubles)
+        double part[CFL_WG];
+        const int n = cfl_launch(ctx, fs, n_species, q, m, dp_finest, fs->work);
+        if ((rc = check_launch(ctx, "k_cfl"))) return rc;
+        if ((rc = vx_memcpy_d2h(ctx, part, fs->work, sizeof(double) * n))) return rc;
+        *out = cfl_bound(vx_cs / fs->dx_f, part, n);
+        return VX_OK;
+    }
     int N = fs->n_f;
     std::vector<double> Ay(N), Az(N), By(N), Bz(N), E(N);
     if ((rc = vx_memcpy_d2h(ctx, Ay.data(), fs->Ay, sizeof(double) * N))) return rc;

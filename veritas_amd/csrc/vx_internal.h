@@ -33,8 +33,8 @@ struct vx_ctx {
     size_t live_bytes = 0;
     // cross-context ordering (vx_ctx_wait) and the asynchronous CFL bound
     hipEvent_t xev = nullptr, cfl_ev = nullptr;
-    double *cfl_host = nullptr;  // pinned
-    double *cfl_dev = nullptr;
+    double *cfl_host = nullptr;  // pinned: cfl_n maxima of the pending bound
+    int cfl_n = 0;
     double cfl_c_dx = 0.0;       // c / dx_f of the pending bound
     bool cfl_pending = false;
     // staging of batched stage launches (vx_stage.hip), freed by its own function

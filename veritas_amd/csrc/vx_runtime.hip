@@ -45,7 +45,6 @@ void vx_ctx_destroy(vx_ctx *ctx) {
     if (ctx->xev) (void)hipEventDestroy(ctx->xev);
     if (ctx->cfl_ev) (void)hipEventDestroy(ctx->cfl_ev);
     if (ctx->cfl_host) (void)hipHostFree(ctx->cfl_host);
-    if (ctx->cfl_dev) (void)hipFree(ctx->cfl_dev);
     for (auto &e : ctx->ring_ev)
         if (e) (void)hipEventDestroy(e);
     if (ctx->ring) (void)hipHostFree(ctx->ring);
