@@ -247,8 +247,7 @@ int vx_maxwell_stage_dev(vx_ctx *ctx, const vx_field_state *fs, int step, double
  * J = 0, neutral = -charge. */
 int vx_neutralize(vx_ctx *ctx, const vx_field_state *fs);
 /* EMFieldSolver::EstimateCFLBound (EMSolver.cpp:631-664) for n_species species
- * (host arrays q, m, dp_finest); result written to *out on the host.  Uses
- * fs->work where it is given. */
+ * (host arrays q, m, dp_finest); result written to *out on the host. */
 int vx_cfl_bound(vx_ctx *ctx, const vx_field_state *fs, int n_species, const double *q,
                  const double *m, const double *dp_finest, double *out);
 /* The same bound computed on the device and copied to pinned host memory

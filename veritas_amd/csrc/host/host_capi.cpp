@@ -26,10 +26,19 @@ vxh::Rectangle &base(Run *r) { return *r->sm->meshes[0]->levels.back()->rectangl
 // f slot named "f0", "f1" or "f2", else -1
 int slot_of(const std::string &w) { return w.size() == 2 && w[0] == 'f' && w[1] >= '0' && w[1] <= '2' ? w[1] - '0' : -1; }
 
-std::vector<double> dl(Run *r, const double *d, size_t n) {
-    std::vector<double> v(n);
-    r->sm->dev->check(vx_memcpy_d2h(r->sm->dev->ctx, v.data(), d, sizeof(double) * n), "download");
-    return v;
+// n device doubles into the caller's array of `room` doubles, if they fit;
+// returns n (a call without an array only asks for it and moves nothing)
+int dl(Run *r, const double *d, size_t n, double *out, int room) {
+    if (out && room >= (int)n)
+        r->sm->dev->check(vx_memcpy_d2h(r->sm->dev->ctx, out, d, sizeof(double) * n), "download");
+    return (int)n;
+}
+
+// a plane of patch p with g ghost layers, likewise
+int dl_plane(const vxh::Rectangle &p, const double *plane, int g, double *out, int room) {
+    const int n = (p.n_x + 2 * g) * (p.n_p + 2 * g);
+    if (out && room >= n) p.Download(plane, g, out);
+    return n;
 }
 
 template <class F>
@@ -241,10 +250,9 @@ int vxh_patch_get(void *h, int sp, int lvl, int idx, const char *what, int ghost
         if (lvl < 0 || lvl >= (int)levels.size() || idx < 0 || idx >= (int)levels[lvl]->rectangles.size())
             return -2;
         vxh::Rectangle &p = *levels[lvl]->rectangles[idx];
-        if (slot_of(what) >= 0) return copy_out(p.DownloadSlot(slot_of(what), ghosts), out, n);
         const double *pl = p.Plane(what);
         if (!pl) return -2;
-        return copy_out(p.Download(pl, ghosts), out, n);
+        return dl_plane(p, pl, ghosts, out, n);
     } catch (std::exception &e) {
         r->err = e.what();
         return -1;
@@ -361,37 +369,37 @@ int vxh_get(void *h, const char *what, int ghosts, double *out, int n) {
     try {
         std::string w(what);
         vxh::Rectangle &p = base(r);
-        if (slot_of(w) >= 0) return copy_out(p.DownloadSlot(slot_of(w), ghosts), out, n);
-        if (const double *pl = p.Plane(w)) return copy_out(p.Download(pl, ghosts), out, n);
+        if (const double *pl = p.Plane(w)) return dl_plane(p, pl, ghosts, out, n);
         const vx_field_state &fs = r->sm->EMSolver->state();
         int N = fs.n_f;
         size_t ne8 = (size_t)8 * fs.n_e;
-        if (w == "phi") return copy_out(dl(r, fs.phi, N), out, n);
-        if (w == "charge") return copy_out(dl(r, fs.charge, N), out, n);
+        if (w == "phi") return dl(r, fs.phi, N, out, n);
+        if (w == "charge") return dl(r, fs.charge, N, out, n);
         if (w.rfind("charge_sp", 0) == 0) {  // species i of the last assembly
             const int sp = std::stoi(w.substr(9));
             const double *cs = r->sm->EMSolver->charges_species;
             if (!cs || sp < 0 || sp >= (int)r->sm->meshes.size()) return -2;
-            return copy_out(dl(r, cs + (size_t)sp * N, N), out, n);
+            return dl(r, cs + (size_t)sp * N, N, out, n);
         }
-        if (w == "J") return copy_out(dl(r, fs.J, N), out, n);
-        if (w == "neutral") return copy_out(dl(r, fs.neutral, N), out, n);
-        if (w == "a2") return copy_out(dl(r, fs.a2, N + 1), out, n);
-        if (w == "E") return copy_out(dl(r, fs.E, N), out, n);
-        if (w == "By") return copy_out(dl(r, fs.By, ne8), out, n);
-        if (w == "Bz") return copy_out(dl(r, fs.Bz, ne8), out, n);
-        if (w == "Ey") return copy_out(dl(r, fs.Ey, ne8), out, n);
-        if (w == "Ez") return copy_out(dl(r, fs.Ez, ne8), out, n);
-        if (w == "Ay") return copy_out(dl(r, fs.Ay, ne8), out, n);
-        if (w == "Az") return copy_out(dl(r, fs.Az, ne8), out, n);
+        if (w == "J") return dl(r, fs.J, N, out, n);
+        if (w == "neutral") return dl(r, fs.neutral, N, out, n);
+        if (w == "a2") return dl(r, fs.a2, N + 1, out, n);
+        if (w == "E") return dl(r, fs.E, N, out, n);
+        if (w == "By") return dl(r, fs.By, ne8, out, n);
+        if (w == "Bz") return dl(r, fs.Bz, ne8, out, n);
+        if (w == "Ey") return dl(r, fs.Ey, ne8, out, n);
+        if (w == "Ez") return dl(r, fs.Ez, ne8, out, n);
+        if (w == "Ay") return dl(r, fs.Ay, ne8, out, n);
+        if (w == "Az") return dl(r, fs.Az, ne8, out, n);
         if (w == "dNdP") {
             r->sm->EMSolver->AssembleEnergy();
             return copy_out(r->sm->EMSolver->energies.at(0), out, n);
         }
         if (w == "scalars") {
             const vx_patch &d = p.desc();
-            std::vector<double> ex0 = dl(r, fs.Ex0, 1);
-            std::vector<double> s = {ex0[0], r->settings->time, d.dx, d.dp, d.pmin, d.m, d.q,
+            double ex0 = 0.0;
+            dl(r, fs.Ex0, 1, &ex0, 1);
+            std::vector<double> s = {ex0, r->settings->time, d.dx, d.dp, d.pmin, d.m, d.q,
                                      (double)fs.n_prepad};
             return copy_out(s, out, n);
         }

@@ -471,14 +471,16 @@ std::vector<double> Rectangle::DownloadSlot(int slot, int g) const {
 }
 
 std::vector<double> Rectangle::Download(const double *plane, int g) const {
-    std::vector<double> full(vx_plane_elems(n_x, n_p));
-    dev->check(vx_memcpy_d2h(dev->ctx, full.data(), plane, sizeof(double) * full.size()), "download");
-    int nx = n_x + 2 * g, np = n_p + 2 * g;
-    std::vector<double> out((size_t)nx * np);
-    for (int i = 0; i < nx; i++)
-        for (int j = 0; j < np; j++)
-            out[(size_t)i * np + j] = full[(size_t)(i - g + 2) * P.pitch + (j - g + 2)];
+    std::vector<double> out((size_t)(n_x + 2 * g) * (n_p + 2 * g));
+    Download(plane, g, out.data());
     return out;
+}
+
+// any plane as slot 0 of a patch of this shape
+void Rectangle::Download(const double *plane, int g, double *out) const {
+    vx_patch p = P;
+    p.f[0] = const_cast<double *>(plane);
+    dev->check(vx_patch_download(dev->ctx, &p, 0, g, out), "download");
 }
 
 const double *Rectangle::Plane(const std::string &w) const {

@@ -182,6 +182,7 @@ public:
     bool AllWalls() const { return up && down && left && right; }
     const vx_patch &desc() const { return P; }
     std::vector<double> Download(const double *plane, int ghosts) const;
+    void Download(const double *plane, int ghosts, double *out) const;  // into (n_x + 2g) x (n_p + 2g) doubles
     std::vector<double> DownloadSlot(int slot, int ghosts) const;  // vx_patch_download
     const double *Plane(const std::string &name) const;
     void UploadSlot(int slot, const std::vector<double> &full);  // whole plane incl. ghosts

@@ -1060,23 +1060,20 @@ int vx_cfl_result(vx_ctx *ctx, double *out) {
 }
 
 // EMSolver.cpp:631-664 (the reference indexes the slot-0 fields without the
-// n_prepad offset): the maxima on the device for the species the kernel holds,
-// through the field state's work array (a pinned buffer of its own would cost
-// each new context 0.3 ms), else, and without a work array, on the host from
-// downloaded arrays (five copies: 60 us at 4096 cells, 190 at 32768; one copy of
-// the maxima and the launch: 20 us).
+// n_prepad offset): the maxima on the device, straight into the context's pinned
+// buffer, for the species the kernel holds, else on the host from downloaded
+// arrays (five copies from pageable memory took 110 us at 64 cells, the launch
+// and a wait take 25).
 int vx_cfl_bound(vx_ctx *ctx, const vx_field_state *fs, int n_species, const double *q,
                  const double *m, const double *dp_finest, double *out) {
     int rc = validate_fs(ctx, fs);
     if (rc) return rc;
     if (ctx->capturing) return fail(ctx, VX_EINVAL, "cfl bound while a step graph is being recorded");
-    if (fs->work && n_species >= 0 && n_species <= CFL_MAXSP) {
-        // (n <= n_f / CFL_CHUNK + 1 of the work array's more than 7 n_f doubles)
-        double part[CFL_WG];
-        const int n = cfl_launch(ctx, fs, n_species, q, m, dp_finest, fs->work);
-        if ((rc = check_launch(ctx, "k_cfl"))) return rc;
-        if ((rc = vx_memcpy_d2h(ctx, part, fs->work, sizeof(double) * n))) return rc;
-        *out = cfl_bound(vx_cs / fs->dx_f, part, n);
+    if (n_species >= 0 && n_species <= CFL_MAXSP) {
+        if ((rc = vx_stage_init(ctx))) return rc;
+        const int n = cfl_launch(ctx, fs, n_species, q, m, dp_finest, ctx->stage);
+        if ((rc = check_launch(ctx, "k_cfl")) || (rc = vx_sync(ctx))) return rc;
+        *out = cfl_bound(vx_cs / fs->dx_f, ctx->stage, n);
         return VX_OK;
     }
     int N = fs->n_f;

@@ -51,10 +51,16 @@ struct vx_ctx {
     hipEvent_t ring_ev[RING] = {};
     bool ring_pending[RING] = {};
     int ring_next = 0;
+    // two pinned buffers of the copies to and from pageable host memory
+    static constexpr size_t STAGE_BYTES = (size_t)2 << 20;
+    double *stage = nullptr;
+    hipEvent_t stage_ev[2] = {};
 };
 
 // vx_field.hip: looks up this device's fixed work array (ctx->device current)
 int vx_noalloc_scratch_init(vx_ctx *ctx);
+// vx_runtime.hip: makes sure that ctx->stage is there
+int vx_stage_init(vx_ctx *ctx);
 
 struct vx_graph {
     hipGraphExec_t exec = nullptr;
