@@ -34,6 +34,20 @@ VX_HD uint64_t vx_double_to_bits(double d) {
     return b;
 }
 
+// R = 2 (s^2/3 + s^4/5 + ... + s^20/21) of vx_log, z = s^2
+VX_HD double vx_log_r(double z) {
+    return z * (0.6666666666666666 +
+           z * (0.4 +
+           z * (0.2857142857142857 +
+           z * (0.2222222222222222 +
+           z * (0.18181818181818182 +
+           z * (0.15384615384615385 +
+           z * (0.13333333333333333 +
+           z * (0.11764705882352941 +
+           z * (0.10526315789473684 +
+           z * 0.09523809523809523)))))))));
+}
+
 VX_HD double vx_log(double x) {
     const double ln2_hi = 0.6931471803691238;      // 0x3fe62e42fee00000
     const double ln2_lo = 1.9082149292705877e-10;  // ln 2 - ln2_hi
@@ -62,16 +76,7 @@ VX_HD double vx_log(double x) {
     double f = m - 1.0;
     double s = f / (2.0 + f);
     double z = s * s;
-    double R = z * (0.6666666666666666 +
-               z * (0.4 +
-               z * (0.2857142857142857 +
-               z * (0.2222222222222222 +
-               z * (0.18181818181818182 +
-               z * (0.15384615384615385 +
-               z * (0.13333333333333333 +
-               z * (0.11764705882352941 +
-               z * (0.10526315789473684 +
-               z * 0.09523809523809523)))))))));
+    double R = vx_log_r(z);
     double hfsq = 0.5 * f * f;
     double dk = (double)k;
     return dk * ln2_hi + (f - (hfsq - (s * (hfsq + R) + dk * ln2_lo)));
