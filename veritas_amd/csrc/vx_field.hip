@@ -2,9 +2,9 @@
 //
 // Poisson (EMSolver.cpp:28-88,156-192).  The reference factors the dense N x N
 // matrix with LAPACK and solves it at every RK stage, O(N^2) per solve.  Here
-// the same matrix is solved to near correct rounding in O(N) (one 512-thread
-// workgroup with the vector in registers up to N = 4096, a sequence of
-// multi-workgroup launches above):
+// the same matrix is solved to near correct rounding in O(N) (one workgroup
+// with the vector in registers up to N = 4096, a sequence of multi-workgroup
+// launches above):
 //   rows 1..N-1 of the matrix are the periodic 4th-order stencil
 //   (w2, w1, w3, w1, w2) with column 0 removed, i.e. the periodic operator with
 //   phi_0 pinned to 0; row 0 then gives phi_0.  The periodic operator factors
@@ -12,7 +12,7 @@
 //   an approximate solve is two prefix sums (L2^-1 on zero-mean data) and M^-1,
 //   whose entries decay as (7 - 4 sqrt 3)^|k| (a 33-tap convolution, or two
 //   first-order recurrences).
-//   Three rounds of iterative refinement with a double-double residual of the
+//   Two or three rounds of iterative refinement with a double-double residual of the
 //   reference's own coefficients take the result to the correctly rounded
 //   solution (the CPU oracle reaches the same point with a band LU).
 //
@@ -359,14 +359,29 @@ __global__ __launch_bounds__(MT) void k_pm_solve(PoissonMB P) {
 // has to be accurate: the refinement rounds take x to the correctly rounded
 // solution whatever the rounding inside it.
 //
-// Barriers: a workgroup sum or scan exchanges the PW1 wavefront partials
-// through LDS once (one barrier); every thread then forms the same sums of the
-// partials itself.  Consecutive exchanges alternate between two partial
-// buffers, so a buffer is rewritten only after a later barrier has ordered
-// every read of it.
-constexpr int PT1 = 512;             // threads of the single-workgroup solve
-constexpr int PW1 = PT1 / 64;        // its wavefronts
-constexpr int SMALL_MAX = 8 * PT1;   // largest n_f it serves (CH = 8)
+// Barriers: a workgroup scan exchanges the wavefront partials through LDS once
+// (one barrier); every thread then forms the same sums of the partials itself.
+// Consecutive exchanges alternate between two partial buffers, so a buffer is
+// rewritten only after a later barrier has ordered every read of it.
+//
+// Rounds of refinement: one leaves a fraction q of the error, because of the
+// prefix sums' rounding and because the factors are not quite those of the
+// matrix, whose coefficients are rounded (w3 + 2 w1 + 2 w2 = 1.4e-16, not 0,
+// against a smallest eigenvalue near (pi / n)^2).  Up to n_f = 4096 q is near
+// 1e-9, so two rounds leave what a third one leaves, the rounded solution:
+// against exact solutions of 127 smooth, rough, sparse and wide-ranging right-hand
+// sides (8 to 4096 entries) the same entries, 1 in 30000, were an ulp off after
+// either.  At 32768 entries two rounds leave 1 or 2 ulps where phi is near 0, so
+// the multi-workgroup solve keeps three.
+//
+// Bound by the chain of scans, recurrences, residuals and barriers; from n_f =
+// 2048 also by FP64 issue on the one CU.  Measured on an MI355X, us at n_f = 64,
+// 512, 1024, 2048 and 4096: 10.1, 11.3, 12.9, 17.9 and 24.8 with eight wavefronts
+// at every size, three rounds and the sums apart from the scans; 4.9, 7.1, 8.8,
+// 12.0 and 17.4 as it is.
+constexpr int PW1 = 8;               // most wavefronts of the single-workgroup solve
+constexpr int SMALL_MAX = 4096;      // largest n_f it serves
+constexpr int SOLVES = 3;            // the first and two rounds of refinement
 constexpr int VH = NG - 1;           // periodic halo of the LDS copy
 
 constexpr int VLEN = SMALL_MAX + 2 * VH + 8;  // positions of the LDS copy
@@ -387,31 +402,28 @@ struct SmallLds {
     }
 };
 
-// Workgroup sum of v; every thread gets the same bits.
-__device__ __forceinline__ double block_sum1(double v, double (&part)[2][PW1], int &buf) {
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const double tot = lane63(wave_scan_dpp(v));
-    if (lane == 0) part[buf][w] = tot;
-    __syncthreads();
-    double all = 0.0;
-#pragma unroll
-    for (int k = 0; k < PW1; k++) all += part[buf][k];
-    buf ^= 1;
-    return all;
-}
-
-// Workgroup exclusive scan of the per-thread totals in thread order.
-__device__ __forceinline__ double block_excl_scan1(double tot, double (&part)[2][PW1], int &buf) {
+// Workgroup exclusive scan of the per-thread totals in thread order, and their
+// sum (the same bits in every thread).
+template <int W>
+__device__ __forceinline__ double block_excl_scan1(double tot, double (&part)[2][PW1], int &buf, double &sum) {
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const double inc = wave_scan_dpp(tot);
-    if (lane == 63) part[buf][w] = inc;
     const double exc = dpp_or_0<0x138>(inc);  // wave_shr:1: lane l - 1's inclusive sum, 0 at lane 0
+    if (W == 1) {
+        __syncthreads();
+        sum = lane63(inc);
+        return exc;
+    }
+    if (lane == 63) part[buf][w] = inc;
     __syncthreads();
-    double off = 0.0;
+    double off = 0.0, all = 0.0;
 #pragma unroll
-    for (int k = 0; k < PW1; k++)
-        if (k < w) off += part[buf][k];
+    for (int k = 0; k < W; k++) {
+        if (k == w) off = all;
+        all += part[buf][k];
+    }
     buf ^= 1;
+    sum = all;
     return off + exc;
 }
 
@@ -444,50 +456,34 @@ __device__ __forceinline__ void put_periodic(SmallLds &L, const double *val, int
     }
 }
 
-// One approximate solve of A out = in: S = exclusive prefix of
-// (-sum_{k>=1} in_k, in_1, in_2, ...), D = mean(S) - S (D_0 = 0), y = inclusive
-// prefix of D, c = M^-1 y - (M^-1 y)_0, and c_0 from row 0 of the matrix.
-template <int CH>
+// One approximate solve of A out = in: S_i = sum_{1<=k<i} in_k - tail (tail the
+// sum over k >= 1, S_0 = 0), d0 = mean(S), y_i = sum_{1<=k<=i} (d0 - S_k) = i d0 -
+// T_i with T the inclusive prefix of S, c = M^-1 y - (M^-1 y)_0, and c_0 from row
+// 0 of the matrix.  Each prefix sum's exchange also gives the sum.
+template <int CH, int W>
 __device__ void approx_one(const PoissonArgs &P, const double *in, double *out, SmallLds &L, int &buf) {
     const int N = P.fs.n_f;
     const int base = threadIdx.x * CH;
-    double loc = 0.0;
-#pragma unroll
-    for (int k = 0; k < CH; k++)
-        if (base + k >= 1 && base + k < N) loc += in[k];
-    const double tail = block_sum1(loc, L.part, buf);
-    double rp[CH], S[CH];
-    double tot = 0.0;
+    double rp[CH], tot = 0.0, tail, ssum;
 #pragma unroll
     for (int k = 0; k < CH; k++) {
-        const int i = base + k;
-        rp[k] = (i == 0) ? -tail : (i < N ? in[k] : 0.0);
+        rp[k] = base + k >= 1 && base + k < N ? in[k] : 0.0;
         tot += rp[k];
     }
-    double run = block_excl_scan1(tot, L.part, buf);
-    double ssum = 0.0;
-#pragma unroll
-    for (int k = 0; k < CH; k++) {
-        S[k] = run;
-        run += rp[k];
-        if (base + k < N) ssum += S[k];
-    }
-    const double d0 = block_sum1(ssum, L.part, buf) * P.invN;
-    double D[CH];
+    double run = block_excl_scan1<W>(tot, L.part, buf, tail);
+    run -= tail;
+    double y[CH];
     tot = 0.0;
 #pragma unroll
     for (int k = 0; k < CH; k++) {
-        const int i = base + k;
-        D[k] = (i == 0 || i >= N) ? 0.0 : d0 - S[k];
-        tot += D[k];
+        if (base + k >= 1 && base + k < N) tot += run;
+        y[k] = tot;
+        run += rp[k];
     }
-    run = block_excl_scan1(tot, L.part, buf);
-    double y[CH];
+    run = block_excl_scan1<W>(tot, L.part, buf, ssum);
+    const double d0 = ssum * P.invN;
 #pragma unroll
-    for (int k = 0; k < CH; k++) {
-        run += D[k];
-        y[k] = run;
-    }
+    for (int k = 0; k < CH; k++) y[k] = (double)(base + k) * d0 - (run + y[k]);
     // (every thread's reads of L.v before this solve came before its first
     // barrier above)
     put_periodic<CH>(L, y, N, base);
@@ -574,10 +570,11 @@ __device__ void residual_one(const PoissonArgs &P, const double *b, const double
     }
 }
 
-template <int CH>
-__global__ __launch_bounds__(PT1) void k_poisson_one(PoissonArgs P) {
+template <int CH, int W>
+__global__ __launch_bounds__(64 * W) void k_poisson_one(PoissonArgs P) {
     const vx_field_state &F = P.fs;
     const int N = F.n_f;
+    constexpr int PT1 = 64 * W;
     const int t = threadIdx.x, base = t * CH;
     __shared__ SmallLds L;
     int buf = 0;
@@ -617,12 +614,12 @@ __global__ __launch_bounds__(PT1) void k_poisson_one(PoissonArgs P) {
         b[k] = base + k < N ? L.at(base + k) : 0.0;
         x[k] = 0.0;
     }
-    // the approximate solve of b, then three rounds of refinement (residual r
+    // the approximate solve of b, then two rounds of refinement (residual r
     // of x, x += the approximate solve of r), as one loop: the kernel runs
     // once per field solve and its code is fetched cold, so one copy of each
     // step is fetched once and then reused
 #pragma nounroll
-    for (int it = 0; it < 4; it++) {
+    for (int it = 0; it < SOLVES; it++) {
         if (it > 0) {
             // the previous solve's last barrier ordered its reads of L.v
             residual_one<CH>(P, b, x, r, L);
@@ -632,7 +629,7 @@ __global__ __launch_bounds__(PT1) void k_poisson_one(PoissonArgs P) {
         }
         // the first barrier of the solve below orders the residual's reads of
         // L.v before the solve writes it
-        approx_one<CH>(P, r, c, L, buf);
+        approx_one<CH, W>(P, r, c, L, buf);
 #pragma unroll
         for (int k = 0; k < CH; k++) x[k] = it == 0 ? c[k] : x[k] + c[k];
     }
@@ -845,12 +842,18 @@ static int poisson(vx_ctx *ctx, const vx_field_state *fs, double *work) {
     P.C = C;
     P.invN = 1.0 / fs->n_f;
     LaunchTimer lt(ctx, "k_poisson");
-    const int ch = (fs->n_f + PT1 - 1) / PT1;
     if (fs->n_f <= SMALL_MAX) {
-        if (ch <= 1) k_poisson_one<1><<<1, PT1, 0, ctx->stream>>>(P);
-        else if (ch <= 2) k_poisson_one<2><<<1, PT1, 0, ctx->stream>>>(P);
-        else if (ch <= 4) k_poisson_one<4><<<1, PT1, 0, ctx->stream>>>(P);
-        else k_poisson_one<8><<<1, PT1, 0, ctx->stream>>>(P);
+        const int n = fs->n_f;
+        // entries a thread and wavefronts: the fewest wavefronts with an entry a
+        // thread, then a wavefront per SIMD, then two (us, 2 x 4 / 1 x 8 at 512: 7.1
+        // / 7.4; 4 x 4 / 2 x 8 at 1024: 8.7 / 9.1; 4 x 8 / 8 x 4 at 2048: 11.9 / 12.8)
+        if (n <= 64) k_poisson_one<1, 1><<<1, 64, 0, ctx->stream>>>(P);
+        else if (n <= 128) k_poisson_one<1, 2><<<1, 128, 0, ctx->stream>>>(P);
+        else if (n <= 256) k_poisson_one<1, 4><<<1, 256, 0, ctx->stream>>>(P);
+        else if (n <= 512) k_poisson_one<2, 4><<<1, 256, 0, ctx->stream>>>(P);
+        else if (n <= 1024) k_poisson_one<4, 4><<<1, 256, 0, ctx->stream>>>(P);
+        else if (n <= 2048) k_poisson_one<4, 8><<<1, 512, 0, ctx->stream>>>(P);
+        else k_poisson_one<8, 8><<<1, 512, 0, ctx->stream>>>(P);
         return check_launch(ctx, "k_poisson");
     }
     PoissonMB M;
