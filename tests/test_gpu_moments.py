@@ -2,7 +2,10 @@
 leave a partial workgroup, p-columns that end inside, at and just past a 64-cell
 chunk, patches with and without the logarithm table (above 2^19 cells), with and
 without nested cells (levels 3: relativeToBottom 1, 2 and 4), behind and ahead
-of a pulse.  The compensated sums agree with the ordered ones."""
+of a pulse.  The compensated sums agree with the ordered ones.  A table of
+another patch is never taken for this one's."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -10,6 +13,8 @@ import veritas_amd as va
 from _amr_cases import two_slab_laser
 from _oracle import OracleRun
 from test_gpu_parity import assert_same
+from test_gpu_staged_copies import Patch
+from test_zz_no_alloc import kernels
 
 pytestmark = pytest.mark.gpu
 
@@ -39,3 +44,55 @@ def test_moments_match_the_oracle(levels, nx, np_):
         assert np.abs(a - b).max() <= tol * np.abs(b).max()
     g.close()
     o.close()
+
+
+class Fields(ctypes.Structure):  # vx_fields
+    _fields_ = ([(n, ctypes.c_int32) for n in ("n_f", "n_prepad", "n_e", "pad")]
+                + [(n, ctypes.c_void_p) for n in ("E", "a2", "Ay1", "Az1", "E0", "a20")])
+
+
+def test_patches_of_different_heights_in_turn():
+    """Two patches above the table's size with one A^2, the second short enough
+    that its tables end inside the first one's entries: the first patch's moments
+    are the same before and after the second's."""
+    L = kernels()
+    L.vx_moments_patch.argtypes = [ctypes.c_void_p, ctypes.POINTER(Patch), ctypes.POINTER(Fields)]
+    ctx = ctypes.c_void_p()
+    assert L.vx_ctx_create(0, ctypes.byref(ctx)) == 0
+    bufs = []
+
+    def put(a):
+        d = ctypes.c_void_p()
+        a = np.ascontiguousarray(a)
+        assert L.vx_malloc(ctx, a.nbytes, ctypes.byref(d)) == 0
+        assert L.vx_memcpy_h2d(ctx, d, a.ctypes.data, a.nbytes) == 0
+        bufs.append(d)
+        return d
+
+    rng = np.random.default_rng(3)
+    made = []
+    for nx, np_ in ((480, 1100), (1760, 300)):
+        pitch = (np_ + 11) // 8 * 8
+        p = Patch(n_x=nx, n_p=np_, rtb=1, pitch=pitch, l=1, r=1, d=1, u=1, dx=1.0, dp=0.004, pmin=-0.002 * np_,
+                  q=-1.0, m=1.0, dx_inv=1.0, dp_inv=250.0, cc=9e16, mc2inv=1.1e-17)
+        f = rng.uniform(1.0, 2.0, (nx + 4, pitch))
+        planes = [put(f)] * 3 + [None] * 21 + [put(np.zeros(nx)), put(np.zeros(nx))]
+        p.planes[:] = [None if q is None else q.value for q in planes]
+        fl = Fields(n_f=nx, n_prepad=2, n_e=nx + 4)
+        a = put(np.full(nx + 4, 0.6))
+        fl.E = fl.a2 = fl.Ay1 = fl.Az1 = fl.E0 = fl.a20 = a.value
+        made.append((p, fl, planes[-2:], nx))
+
+    def run(k):
+        p, fl, out, nx = made[k]
+        assert L.vx_moments_patch(ctx, ctypes.byref(p), ctypes.byref(fl)) == 0, L.vx_last_error(ctx)
+        got = np.empty((2, nx))
+        for g, d in zip(got, out):
+            assert L.vx_memcpy_d2h(ctx, g.ctypes.data, d, g.nbytes) == 0
+        return got
+
+    first, _, again = run(0), run(1), run(0)
+    assert np.abs(first).min() > 0 and np.array_equal(first, again)
+    for d in bufs:
+        L.vx_free(ctx, d)
+    L.vx_ctx_destroy(ctx)

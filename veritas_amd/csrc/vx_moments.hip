@@ -39,11 +39,12 @@ struct MomArgs {
     double rel[3 * MAX_RTB];  // interpolatCoefsREL (Rectangle.cpp:103-110)
     // Two tables of logarithm terms, each for one value a0 of A^2: table 0 for
     // the patch's first sub-column (every column when A^2 is uniform), table 1
-    // for A^2 = 0 (the plasma ahead of a laser pulse).  Table q starts at
-    // tab + q (n_p + 3 + TAB_KEY): entries t in [0, n_p+2) hold
-    // c2 log(h(t)/h(t-1)) with h(j) = Gamma(p_j, a0) + c1 p_j, entry n_p+2 is 1
-    // once built, and the TAB_KEY entries after it what they were formed from
-    // (a0 first, then the p grid and the constants), so an unchanged table is
+    // for A^2 = 0 (the plasma ahead of a laser pulse).  Table q's entries t in
+    // [0, n_p+2) (tab_entries) hold c2 log(h(t)/h(t-1)) with h(j) = Gamma(p_j, a0)
+    // + c1 p_j; its head, at tab + q TAB_HEAD wherever the entries lie (so that a
+    // table of another n_p is never taken for this one), holds what they were
+    // formed from (a0 first, then the p grid and the constants) and at TAB_KEY 1
+    // once built, so an unchanged table is
     // not rebuilt.  A wavefront whose chains all have A^2 == a0 of a table
     // reads it (the same bits it would form itself); the others form their
     // logarithms per distinct A^2.
@@ -60,18 +61,18 @@ __device__ __forceinline__ double cell_a2(const vx_fields &fl, long i) {
 }
 
 
-__host__ __device__ inline long tab_stride(int n_p) { return (long)n_p + 3 + TAB_KEY; }
+constexpr int TAB_HEAD = 16;
+__host__ __device__ inline long tab_entries(int q, int n_p) { return 2 * TAB_HEAD + q * ((long)n_p + 3); }
 
 // Logarithm tables of one patch (see MomArgs::tab); workgroup q builds table q.
 template <int RTB>
 __global__ __launch_bounds__(1024) void k_moment_table(MomArgs A, double *tab) {
     const vx_patch &P = A.p;
     const int t = threadIdx.x;
-    tab += blockIdx.x * tab_stride(P.n_p);
     const double a0 = blockIdx.x == 0 ? P.q * P.q * cell_a2(A.fl, (long)P.x_pos * RTB) : 0.0;
     const double key[TAB_KEY] = {a0, P.pmin, P.dp, (double)P.p_pos, P.mc2inv, A.c1, A.c2, (double)P.n_p};
-    double *kt = tab + P.n_p + 3;
-    bool hit = tab[P.n_p + 2] == 1.0;
+    double *kt = tab + blockIdx.x * TAB_HEAD, *entry = tab + tab_entries((int)blockIdx.x, P.n_p);
+    bool hit = kt[TAB_KEY] == 1.0;
     for (int k = 0; k < TAB_KEY; k++) hit = hit && kt[k] == key[k];
     if (__syncthreads_or(hit ? 1 : 0) != 0) return;  // the same table is in place
     // (every thread read the same bits; the barrier also orders those reads
@@ -80,9 +81,9 @@ __global__ __launch_bounds__(1024) void k_moment_table(MomArgs A, double *tab) {
         double pm = momentum(P.pmin, P.dp, j, P.p_pos);
         return gamma_(pm, a0, P.mc2inv) + A.c1 * pm;
     };
-    for (int e = t; e < P.n_p + 2; e += blockDim.x) tab[e] = A.c2 * vx_log(h(e) / h(e - 1));
+    for (int e = t; e < P.n_p + 2; e += blockDim.x) entry[e] = A.c2 * vx_log(h(e) / h(e - 1));
     if (t < TAB_KEY) kt[t] = key[t];
-    if (t == 0) tab[P.n_p + 2] = 1.0;
+    if (t == 0) kt[TAB_KEY] = 1.0;
 }
 
 // Compensated wavefront sum of the lanes' (value, error) pairs (mixed-precision
@@ -192,16 +193,16 @@ __global__ __launch_bounds__(64 * (WCOL + 1)) void k_moments(MomArgs A) {
         for (int s = 0; s < RTB; s++) asq[s] = P.q * P.q * cell_a2(A.fl, (long)(ic + P.x_pos) * RTB + s);
         const double *tab = nullptr;
         for (int q = 1; q >= 0 && A.tab && !tab; q--) {
-            const double *tq = A.tab + q * tab_stride(P.n_p);
-            bool all = tq[P.n_p + 2] != 0.0;
+            const double *kt = A.tab + q * TAB_HEAD;
+            bool all = kt[TAB_KEY] != 0.0;
 #pragma unroll
-            for (int s = 0; s < RTB; s++) all = all && asq[s] == tq[P.n_p + 3];
-            if (all) tab = tq;
+            for (int s = 0; s < RTB; s++) all = all && asq[s] == kt[0];
+            if (all) tab = A.tab + tab_entries(q, P.n_p);
         }
         // Chunk k (jb = 64 k) loads entry r = jb + l of two sequences: the
         // column's f from p = -1 (f at p-cell jb - 1 + l; rows ic - 2 .. ic + 2
         // for the interpolation) and the logarithm table (entry jb + l), with r
-        // clamped to n_p + 2 (f at p-cell n_p + 1, the table's last entry), and
+        // clamped to n_p + 2 (f at p-cell n_p + 1, past the table's last), and
         // the nested flag of p-cell jb + l, clamped to the last; those clamped
         // entries serve skipped cells only.  The chunk's address is scalar, the
         // lane adds a 32-bit offset.
@@ -501,7 +502,7 @@ static int moments_patch(vx_ctx *ctx, const vx_patch *p, const vx_fields *fl, bo
     // 8000 x 256 27.8 / 33.7; columns with a pulse do not use it (500 x 512 at rtb
     // 4 21.1 / 19.1).
     if ((long)p->n_x * p->n_p > TAB_CELLS) {
-        const size_t need = 2 * (size_t)tab_stride(p->n_p);
+        const size_t need = (size_t)tab_entries(2, p->n_p);
         if (ctx->mom_table_n < need) {
             if (ctx->capturing) return fail(ctx, VX_EINVAL, "moments: table growth while a step graph is recorded");
             if (ctx->mom_table) (void)hipFree(ctx->mom_table);
