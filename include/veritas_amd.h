@@ -243,6 +243,9 @@ int vx_maxwell_stage(vx_ctx *ctx, const vx_field_state *fs, int step, double dt,
  * at every stage). */
 int vx_maxwell_stage_dev(vx_ctx *ctx, const vx_field_state *fs, int step, double dt,
                          const double *drive);
+/* E (n_f entries) and A^2 at the faces (n_f + 1) into E0 and a20: the fields of
+ * stage 0 that the later stages of a step read (vx_fields.E0, a20). */
+int vx_snapshot_fields(vx_ctx *ctx, const vx_field_state *fs, double *E0, double *a20);
 /* EMFieldSolver::EnforceChargeNeutralization tail (EMSolver.cpp:624-628):
  * J = 0, neutral = -charge. */
 int vx_neutralize(vx_ctx *ctx, const vx_field_state *fs);

@@ -700,8 +700,7 @@ void EMFieldSolver::AssembleRhoAndJ() {
 void EMFieldSolver::UpdatePotential() { dev->check(vx_poisson(dev->ctx, &fs), "poisson"); }
 
 void EMFieldSolver::SnapshotStage0Fields() {
-    dev->check(vx_memcpy_d2d(dev->ctx, (void *)fl.E0, fs.E, sizeof(double) * fs.n_f), "E0");
-    dev->check(vx_memcpy_d2d(dev->ctx, (void *)fl.a20, fs.a2, sizeof(double) * (fs.n_f + 1)), "a2_0");
+    dev->check(vx_snapshot_fields(dev->ctx, &fs, (double *)fl.E0, (double *)fl.a20), "snapshot");
 }
 
 // EMSolver.cpp:194-202; the hooks are evaluated at x = 0 and the stage time

@@ -667,7 +667,7 @@ struct MaxArgs {
 
 __device__ __forceinline__ int fidx(int ne, int i, int slot) { return slot * ne + i; }
 
-// A field stage is two launches (three, with the faces apart, took 12.6 us at
+// Above MX1 elements a field stage is two launches (three, with the faces apart, took 12.6 us at
 // 4096 elements on an MI355X, these 8.9): the right-hand sides, which read
 // slot 1 at the neighbouring elements and write slot step + 2, then the update
 // of slot 1 and A^2 at the faces from it.  A face's four potentials are formed
@@ -678,24 +678,21 @@ __device__ __forceinline__ int fidx(int ne, int i, int slot) { return slot * ne 
 
 // EMSolver.cpp:479-553; blockIdx.y = 0: By, Ez, Az; 1: Bz, Ey, Ay (each set
 // reads only itself)
-__device__ __forceinline__ void maxwell_last(double *y, int ne, int i, const double *b, double k5) {
+__device__ __forceinline__ double maxwell_last(const double *y, int ne, int i, const double *b, double k5) {
     double t = y[fidx(ne, i, 1)] + b[0] * y[fidx(ne, i, 2)];
 #pragma unroll
     for (int k = 1; k < 5; k++) t = t + b[k] * y[fidx(ne, i, k + 2)];
-    t = t + b[5] * k5;
-    y[fidx(ne, i, 0)] = t;
+    return t + b[5] * k5;
 }
 
-__global__ __launch_bounds__(256) void k_maxwell_rhs(MaxArgs A) {
+// The right-hand sides of element i of a set (z: By, Ez, Az; else Bz, Ey, Ay)
+__device__ __forceinline__ void maxwell_rhs(const MaxArgs &A, bool z, const double *B, const double *E, const double *V,
+                                            int i, double &rB, double &rE, double &rV) {
     const vx_field_state &F = A.fs;
     const int ne = F.n_e, npre = F.n_prepad, N = F.n_f;
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= ne) return;
-    const bool z = blockIdx.y == 0;  // By, Ez, Az; else Bz, Ey, Ay
-    double *B = z ? F.By : F.Bz, *E = z ? F.Ez : F.Ey, *V = z ? F.Az : F.Ay;
-    const int s = fidx(ne, i, A.step + 2), i1 = fidx(ne, i, 1);
+    const int i1 = fidx(ne, i, 1);
     const double dx_inv = A.dx_inv, db = z ? dx_inv : -dx_inv, de = z ? dx_inv : -dx_inv;
-    double rB = 0, rE = 0, rV = 0;
+    rB = rE = rV = 0;
     if (i == 0) {
         const double b0 = z ? (A.drive ? A.drive[0] : A.by0) : (A.drive ? A.drive[1] : A.bz0);
         rB = db * (E[i1 + 1] - E[i1]);
@@ -714,13 +711,25 @@ __global__ __launch_bounds__(256) void k_maxwell_rhs(MaxArgs A) {
              vx_eps0_inv * Jc * V[i1];
         rV = -E[i1];
     }
+}
+
+__global__ __launch_bounds__(256) void k_maxwell_rhs(MaxArgs A) {
+    const vx_field_state &F = A.fs;
+    const int ne = F.n_e;
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= ne) return;
+    const bool z = blockIdx.y == 0;
+    double *B = z ? F.By : F.Bz, *E = z ? F.Ez : F.Ey, *V = z ? F.Az : F.Ay;
+    double rB, rE, rV;
+    maxwell_rhs(A, z, B, E, V, i, rB, rE, rV);
+    const int s = fidx(ne, i, A.step + 2);
     B[s] = rB;
     E[s] = rE;
     V[s] = rV;
     if (A.step == 5) {
-        maxwell_last(B, ne, i, A.b, rB);
-        maxwell_last(E, ne, i, A.b, rE);
-        maxwell_last(V, ne, i, A.b, rV);
+        B[fidx(ne, i, 0)] = maxwell_last(B, ne, i, A.b, rB);
+        E[fidx(ne, i, 0)] = maxwell_last(E, ne, i, A.b, rE);
+        V[fidx(ne, i, 0)] = maxwell_last(V, ne, i, A.b, rV);
     }
 }
 
@@ -764,6 +773,68 @@ __global__ __launch_bounds__(MXT) void k_maxwell_update(MaxArgs A) {
     const double y = face_weno(ay[k], ay[k + 1], ay[k + 2], ay[k + 3]);
     const double z = face_weno(az[k], az[k + 1], az[k + 2], az[k + 3]);
     F.a2[face] = (y * y) + (z * z);
+}
+
+// The whole stage in one workgroup, for at most MX1 elements: a thread forms the
+// right-hand sides and new values of an element of its set from slot 1, which is
+// written only after a barrier has ordered every read of it, then A^2 at the
+// faces from the new potentials in LDS.  Bound by launch latency: one launch for
+// two.  us a stage on an MI355X, this / the two launches: 4.4 / 8.0 at 64 cells,
+// 4.5 to 5.2 / 8.0 at 256, 4.7 to 6.1 / 8.2 at 508; two elements a thread took 6.0
+// to 8.3 / 8.1 at 700, 7.1 to 10.6 / 8.1 at 1020.
+constexpr int MX1 = 512;
+__global__ __launch_bounds__(2 * MX1) void k_maxwell_one(MaxArgs A) {
+    const vx_field_state &F = A.fs;
+    const int ne = F.n_e;
+    const bool z = threadIdx.x < MX1;  // uniform per wavefront
+    const int i = (int)threadIdx.x & (MX1 - 1);
+    double *B = z ? F.By : F.Bz, *E = z ? F.Ez : F.Ey, *V = z ? F.Az : F.Ay;
+    __shared__ double pot[2][MX1];  // the new Ay, Az
+    double nB, nE, nV;
+    // slot 1 after the update, from the right-hand side and the slots before it
+    auto fresh = [&](const double *y, double r) {
+        if (A.step > 4) return maxwell_last(y, ne, i, A.b, r);
+        double v = y[fidx(ne, i, 0)];
+        for (int k = 0; k < A.step; k++) v = v + A.a[k] * y[fidx(ne, i, k + 2)];
+        return v + A.a[A.step] * r;
+    };
+    if (i < ne) {
+        double rB, rE, rV;
+        maxwell_rhs(A, z, B, E, V, i, rB, rE, rV);
+        nB = fresh(B, rB);
+        nE = fresh(E, rE);
+        nV = fresh(V, rV);
+        const int s = fidx(ne, i, A.step + 2);
+        B[s] = rB;
+        E[s] = rE;
+        V[s] = rV;
+        pot[z][i] = nV;
+    }
+    __syncthreads();
+    if (i < ne) {
+        const int s = fidx(ne, i, 1);
+        B[s] = nB;
+        E[s] = nE;
+        V[s] = nV;
+        if (A.step > 4) {
+            B[i] = nB;
+            E[i] = nE;
+            V[i] = nV;
+        }
+    }
+    const int face = threadIdx.x;
+    if (face >= F.n_f) return;
+    const int e = face + F.n_prepad - 2;
+    const double y = face_weno(pot[0][e], pot[0][e + 1], pot[0][e + 2], pot[0][e + 3]);
+    const double v = face_weno(pot[1][e], pot[1][e + 1], pot[1][e + 2], pot[1][e + 3]);
+    F.a2[face] = (y * y) + (v * v);
+}
+
+// a2_0 and E at the start of a step, in one launch
+__global__ __launch_bounds__(256) void k_snapshot(vx_field_state F, double *E0, double *a20) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i < F.n_f) E0[i] = F.E[i];
+    if (i <= F.n_f) a20[i] = F.a2[i];
 }
 
 __global__ void k_neutralize(vx_field_state F) {
@@ -925,6 +996,10 @@ static int maxwell_stage(vx_ctx *ctx, const vx_field_state *fs, int step, double
         a[5] = 0;
         for (int k = 0; k < 6; k++) A.b[k] = vx::rk_a[5][k] * dt - a[k];
     }
+    if (fs->n_e <= MX1) {
+        k_maxwell_one<<<1, 2 * MX1, 0, ctx->stream>>>(A);
+        return check_launch(ctx, "k_maxwell_one");
+    }
     unsigned g = (unsigned)((fs->n_e + MXT - 1) / MXT);
     k_maxwell_rhs<<<dim3(g, 2), MXT, 0, ctx->stream>>>(A);
     if ((rc = check_launch(ctx, "k_maxwell_rhs"))) return rc;
@@ -943,6 +1018,14 @@ int vx_maxwell_stage_dev(vx_ctx *ctx, const vx_field_state *fs, int step, double
                          const double *drive) {
     if (!drive) return fail(ctx, VX_EINVAL, "maxwell: null drive");
     return maxwell_stage(ctx, fs, step, dt, 0.0, 0.0, drive);
+}
+
+int vx_snapshot_fields(vx_ctx *ctx, const vx_field_state *fs, double *E0, double *a20) {
+    int rc = validate_fs(ctx, fs);
+    if (rc) return rc;
+    if (!E0 || !a20) return fail(ctx, VX_EINVAL, "snapshot: null output");
+    k_snapshot<<<(unsigned)((fs->n_f + 256) / 256), 256, 0, ctx->stream>>>(*fs, E0, a20);
+    return check_launch(ctx, "k_snapshot");
 }
 
 int vx_neutralize(vx_ctx *ctx, const vx_field_state *fs) {
