@@ -176,6 +176,9 @@ int vx_moments_patch(vx_ctx *ctx, const vx_patch *p, const vx_fields *fl);
  * mixed-precision form keeps the moment reductions FP64 and compensated; the
  * reference's sequential order is not kept; no counterpart in the reference). */
 int vx_moments_patch_compensated(vx_ctx *ctx, const vx_patch *p, const vx_fields *fl);
+/* The moments of n patches (of one or several species and levels; host array),
+ * compensated or not, with as few launches as their sizes allow. */
+int vx_moments_patches(vx_ctx *ctx, const vx_patch *patches, int32_t n, const vx_fields *fl, int compensated);
 /* Rectangle::CalculateEnergy (Rectangle.cpp:284-305): energyR[j * rtb + k]
  * (n_p * rtb doubles, device) = dx * sum over non-nested cells (i, j) of the
  * p-sub-cell value k, summed in increasing i (the reference's loop races on

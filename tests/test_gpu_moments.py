@@ -3,7 +3,8 @@ leave a partial workgroup, p-columns that end inside, at and just past a 64-cell
 chunk, patches with and without the logarithm table (above 2^19 cells), with and
 without nested cells (levels 3: relativeToBottom 1, 2 and 4), behind and ahead
 of a pulse.  The compensated sums agree with the ordered ones.  A table of
-another patch is never taken for this one's."""
+another patch is never taken for this one's, and several patches in one launch
+give each one's bits."""
 import ctypes
 
 import numpy as np
@@ -51,48 +52,92 @@ class Fields(ctypes.Structure):  # vx_fields
                 + [(n, ctypes.c_void_p) for n in ("E", "a2", "Ay1", "Az1", "E0", "a20")])
 
 
+class Case:
+    """Patches of the given (n_x, n_p, rtb, nested) in one context, with an A^2
+    that is 0, uniform or varies."""
+
+    def __init__(self, shapes, a):
+        L = self.L = kernels()
+        pp, pf = ctypes.POINTER(Patch), ctypes.POINTER(Fields)
+        L.vx_moments_patch.argtypes = L.vx_moments_patch_compensated.argtypes = [ctypes.c_void_p, pp, pf]
+        L.vx_moments_patches.argtypes = [ctypes.c_void_p, pp, ctypes.c_int32, pf, ctypes.c_int]
+        self.ctx, self.bufs = ctypes.c_void_p(), []
+        assert L.vx_ctx_create(0, ctypes.byref(self.ctx)) == 0
+        rng = np.random.default_rng(3)
+        n_f = max(nx * rtb for nx, _, rtb, _ in shapes)
+        self.p, self.out = (Patch * len(shapes))(), []
+        for k, (nx, np_, rtb, nested) in enumerate(shapes):
+            pitch = (np_ + 11) // 8 * 8
+            f = rng.uniform(1.0, 2.0, (nx + 4, pitch))
+            mask = (rng.random((nx + 4, pitch)) < 0.4).astype(np.uint8)
+            planes = [self.put(f)] * 3 + [None] * 20 + [self.put(mask) if nested else None]
+            self.out.append([self.put(np.zeros(nx * rtb)) for _ in range(2)])
+            self.p[k] = Patch(n_x=nx, n_p=np_, rtb=rtb, pitch=pitch, l=1, r=1, d=1, u=1, dx=1.0, dp=0.004,
+                                  pmin=-0.002 * np_, q=-1.0, m=1.0, dx_inv=1.0, dp_inv=250.0, cc=9e16, mc2inv=0.5)
+            self.p[k].planes[:] = [None if q is None else q.value for q in planes + self.out[-1]]
+        self.fl = Fields(n_f=n_f, n_prepad=2, n_e=n_f + 4)
+        x = np.arange(n_f + 4)
+        A = {"zero": 0.0 * x, "uniform": 0.6 + 0.0 * x, "pulse": np.maximum(0.0, np.sin(x / 40.0))}[a]
+        for name in ("E", "a2", "Ay1", "Az1", "E0", "a20"):
+            setattr(self.fl, name, self.put(A).value)
+
+    def put(self, a):
+        d = ctypes.c_void_p()
+        a = np.ascontiguousarray(a)
+        assert self.L.vx_malloc(self.ctx, a.nbytes, ctypes.byref(d)) == 0
+        assert self.L.vx_memcpy_h2d(self.ctx, d, a.ctypes.data, a.nbytes) == 0
+        self.bufs.append(d)
+        return d
+
+    def get(self, k):
+        """The charge and current of patch k, which are then cleared."""
+        got = []
+        for d in self.out[k]:
+            a = np.empty(self.p[k].n_x * self.p[k].rtb)
+            assert self.L.vx_memcpy_d2h(self.ctx, a.ctypes.data, d, a.nbytes) == 0
+            z = np.zeros_like(a)
+            assert self.L.vx_memcpy_h2d(self.ctx, d, z.ctypes.data, z.nbytes) == 0
+            got.append(a)
+        return got
+
+    def one(self, k, comp=False):
+        f = self.L.vx_moments_patch_compensated if comp else self.L.vx_moments_patch
+        assert f(self.ctx, ctypes.byref(self.p[k]), ctypes.byref(self.fl)) == 0, self.L.vx_last_error(self.ctx)
+        return self.get(k)
+
+    def free(self):
+        for d in self.bufs:
+            self.L.vx_free(self.ctx, d)
+        self.L.vx_ctx_destroy(self.ctx)
+
+
 def test_patches_of_different_heights_in_turn():
     """Two patches above the table's size with one A^2, the second short enough
     that its tables end inside the first one's entries: the first patch's moments
     are the same before and after the second's."""
-    L = kernels()
-    L.vx_moments_patch.argtypes = [ctypes.c_void_p, ctypes.POINTER(Patch), ctypes.POINTER(Fields)]
-    ctx = ctypes.c_void_p()
-    assert L.vx_ctx_create(0, ctypes.byref(ctx)) == 0
-    bufs = []
-
-    def put(a):
-        d = ctypes.c_void_p()
-        a = np.ascontiguousarray(a)
-        assert L.vx_malloc(ctx, a.nbytes, ctypes.byref(d)) == 0
-        assert L.vx_memcpy_h2d(ctx, d, a.ctypes.data, a.nbytes) == 0
-        bufs.append(d)
-        return d
-
-    rng = np.random.default_rng(3)
-    made = []
-    for nx, np_ in ((480, 1100), (1760, 300)):
-        pitch = (np_ + 11) // 8 * 8
-        p = Patch(n_x=nx, n_p=np_, rtb=1, pitch=pitch, l=1, r=1, d=1, u=1, dx=1.0, dp=0.004, pmin=-0.002 * np_,
-                  q=-1.0, m=1.0, dx_inv=1.0, dp_inv=250.0, cc=9e16, mc2inv=1.1e-17)
-        f = rng.uniform(1.0, 2.0, (nx + 4, pitch))
-        planes = [put(f)] * 3 + [None] * 21 + [put(np.zeros(nx)), put(np.zeros(nx))]
-        p.planes[:] = [None if q is None else q.value for q in planes]
-        fl = Fields(n_f=nx, n_prepad=2, n_e=nx + 4)
-        a = put(np.full(nx + 4, 0.6))
-        fl.E = fl.a2 = fl.Ay1 = fl.Az1 = fl.E0 = fl.a20 = a.value
-        made.append((p, fl, planes[-2:], nx))
-
-    def run(k):
-        p, fl, out, nx = made[k]
-        assert L.vx_moments_patch(ctx, ctypes.byref(p), ctypes.byref(fl)) == 0, L.vx_last_error(ctx)
-        got = np.empty((2, nx))
-        for g, d in zip(got, out):
-            assert L.vx_memcpy_d2h(ctx, g.ctypes.data, d, g.nbytes) == 0
-        return got
-
-    first, _, again = run(0), run(1), run(0)
+    c = Case([(480, 1100, 1, False), (1760, 300, 1, False)], "uniform")
+    first, _, again = c.one(0), c.one(1), c.one(0)
     assert np.abs(first).min() > 0 and np.array_equal(first, again)
-    for d in bufs:
-        L.vx_free(ctx, d)
-    L.vx_ctx_destroy(ctx)
+    c.free()
+
+
+@pytest.mark.parametrize("a", ["zero", "uniform", "pulse"])
+@pytest.mark.parametrize("comp", [False, True])
+def test_patches_together_match_each_alone(a, comp):
+    """More patches than one launch holds, of every relativeToBottom, with and
+    without nested cells, below and above the table's size (alone they read it,
+    together they form their logarithms) and one that keeps its own launch: the
+    same bits as each alone."""
+    c = Case([(2050, 1030, 1, False), (1030, 514, 1, False), (515, 1030, 2, True), (1100, 500, 4, True),
+              (1030, 514, 4, False), (7, 9, 1, False), (33, 64, 2, False), (5, 130, 4, True), (64, 65, 1, True),
+              (1, 8, 4, False), (130, 100, 2, True), (18, 192, 1, False), (40, 66, 4, False), (9, 127, 2, True),
+              (3, 1, 1, False)], a)
+    n = len(c.p)
+    alone = [c.one(k, comp) for k in range(n)]
+    for m in (n, 12, 13, 1):
+        assert c.L.vx_moments_patches(c.ctx, c.p, m, ctypes.byref(c.fl), comp) == 0, c.L.vx_last_error(c.ctx)
+        for k in range(n):
+            for x, y in zip(c.get(k), alone[k]):
+                assert np.array_equal(x, y if k < m else 0.0 * y), (k, m)
+    assert all(np.abs(y).max() > 0 for r in alone for y in r)
+    c.free()

@@ -458,10 +458,7 @@ void Rectangle::UnaliasSlots() {
 }
 
 void Rectangle::CalculateRhoAndJ() {
-    if (EMSolver->compensated_moments)
-        dev->check(vx_moments_patch_compensated(dev->ctx, &P, &EMSolver->fields()), "moments");
-    else
-        dev->check(vx_moments_patch(dev->ctx, &P, &EMSolver->fields()), "moments");
+    dev->check(vx_moments_patches(dev->ctx, &P, 1, &EMSolver->fields(), EMSolver->compensated_moments), "moments");
 }
 
 std::vector<double> Rectangle::DownloadSlot(int slot, int g) const {
@@ -691,9 +688,11 @@ void EMFieldSolver::RebuildMomentPlan() {
 
 // EMSolver.cpp:104-122
 void EMFieldSolver::AssembleRhoAndJ() {
+    std::vector<vx_patch> p;
     for (auto &m : meshes)
         for (auto &l : m->levels)
-            for (auto &r : l->rectangles) r->CalculateRhoAndJ();
+            for (auto &r : l->rectangles) p.push_back(r->desc());
+    dev->check(vx_moments_patches(dev->ctx, p.data(), (int32_t)p.size(), &fl, compensated_moments), "moments");
     dev->check(vx_moments_assemble(dev->ctx, plan, fs.charge, fs.J, charges_species), "assemble");
 }
 

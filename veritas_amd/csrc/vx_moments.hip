@@ -7,8 +7,9 @@
 // forms a column's summands, 64 consecutive p-cells in parallel (interpolants,
 // gamma factors, logarithms), and another adds them in order from LDS, one lane
 // per accumulation chain.
-#include <type_traits>
+#include <algorithm>
 #include <cstring>
+#include <type_traits>
 #include <vector>
 
 #include "vx_dev.h"
@@ -22,6 +23,7 @@ namespace {
 
 constexpr int MAX_RTB = 4;  // coarsest level of a 3-level hierarchy at ratio 2
 constexpr long TAB_CELLS = 1 << 19;  // a patch of more cells gets a logarithm table
+constexpr long BATCH_CELLS = 1 << 21;  // a patch of more cells has a launch (and a table) of its own
 constexpr int TAB_KEY = 8;  // A^2, pmin, dp, p_pos, mc2inv, c1, c2, n_p
 
 // Rectangle.cpp:76-89
@@ -30,13 +32,22 @@ __constant__ double kInterp[12] = {
     0.117647058823529, 0.029411764705882,  0.029411764705882, 0.117647058823529,
     -0.083333333333333, 0.166666666666667, -0.166666666666667, 0.083333333333334};
 
-struct MomArgs {
-    vx_patch p;
-    vx_fields fl;
-    double c1, c2, c3;     // m_inv*c_inv, 1/c1, 1/48
+// What the moments of one patch need
+struct MomPatch {
+    const double *f;
+    const uint8_t *nested;
+    double *chargeR, *currentR;
+    int n_x, n_p, x_pos, p_pos, rtb, pitch;
+    double dx, dp, pmin, q, mc2inv;
+    double c1, c2, c3;    // m_inv*c_inv, 1/c1, 1/48
     double inv_rtb;       // 1.0 / relativeToBottom
     double dpq, jscale;   // dp*q and -q*q/mass
     double rel[3 * MAX_RTB];  // interpolatCoefsREL (Rectangle.cpp:103-110)
+};
+
+struct MomArgs {
+    MomPatch p;
+    vx_fields fl;
     // Two tables of logarithm terms, each for one value a0 of A^2: table 0 for
     // the patch's first sub-column (every column when A^2 is uniform), table 1
     // for A^2 = 0 (the plasma ahead of a laser pulse).  Table q's entries t in
@@ -44,11 +55,18 @@ struct MomArgs {
     // + c1 p_j; its head, at tab + q TAB_HEAD wherever the entries lie (so that a
     // table of another n_p is never taken for this one), holds what they were
     // formed from (a0 first, then the p grid and the constants) and at TAB_KEY 1
-    // once built, so an unchanged table is
-    // not rebuilt.  A wavefront whose chains all have A^2 == a0 of a table
-    // reads it (the same bits it would form itself); the others form their
-    // logarithms per distinct A^2.
+    // once built, so an unchanged table is not rebuilt.  A wavefront whose chains
+    // all have A^2 == a0 of a table reads it (the same bits it would form itself);
+    // the others form their logarithms per distinct A^2.
     const double *tab;
+};
+
+// Several patches in one launch: patch k's workgroups start at start[k].
+constexpr int MOM_BATCH = 12;  // 3 KB of kernel arguments
+struct MomBatch {
+    vx_fields fl;
+    int n, start[MOM_BATCH + 1];
+    MomPatch p[MOM_BATCH];
 };
 
 // EMFieldSolver::GetCellAverageASquared (EMSolver.hpp:57-64)
@@ -67,10 +85,10 @@ __host__ __device__ inline long tab_entries(int q, int n_p) { return 2 * TAB_HEA
 // Logarithm tables of one patch (see MomArgs::tab); workgroup q builds table q.
 template <int RTB>
 __global__ __launch_bounds__(1024) void k_moment_table(MomArgs A, double *tab) {
-    const vx_patch &P = A.p;
+    const MomPatch &P = A.p;
     const int t = threadIdx.x;
     const double a0 = blockIdx.x == 0 ? P.q * P.q * cell_a2(A.fl, (long)P.x_pos * RTB) : 0.0;
-    const double key[TAB_KEY] = {a0, P.pmin, P.dp, (double)P.p_pos, P.mc2inv, A.c1, A.c2, (double)P.n_p};
+    const double key[TAB_KEY] = {a0, P.pmin, P.dp, (double)P.p_pos, P.mc2inv, P.c1, P.c2, (double)P.n_p};
     double *kt = tab + blockIdx.x * TAB_HEAD, *entry = tab + tab_entries((int)blockIdx.x, P.n_p);
     bool hit = kt[TAB_KEY] == 1.0;
     for (int k = 0; k < TAB_KEY; k++) hit = hit && kt[k] == key[k];
@@ -79,9 +97,9 @@ __global__ __launch_bounds__(1024) void k_moment_table(MomArgs A, double *tab) {
     // before the writes below)
     auto h = [&](int j) {
         double pm = momentum(P.pmin, P.dp, j, P.p_pos);
-        return gamma_(pm, a0, P.mc2inv) + A.c1 * pm;
+        return gamma_(pm, a0, P.mc2inv) + P.c1 * pm;
     };
-    for (int e = t; e < P.n_p + 2; e += blockDim.x) entry[e] = A.c2 * vx_log(h(e) / h(e - 1));
+    for (int e = t; e < P.n_p + 2; e += blockDim.x) entry[e] = P.c2 * vx_log(h(e) / h(e - 1));
     if (t < TAB_KEY) kt[t] = key[t];
     if (t == 0) kt[TAB_KEY] = 1.0;
 }
@@ -171,17 +189,19 @@ __device__ __forceinline__ double log_ratio(double a, double b) {
 // compensated (TwoSum) sums over the chunks and ends with one compensated
 // reduction across its lanes.
 // NEST: the patch has nested cells (their summands are -0.0).
+// tabs: the patch's logarithm tables, or null; blk: the workgroup's number in
+// the patch; lds: 2 x 2 x WCOL RTB rows of 65 (not used by COMP).
 template <int RTB, bool COMP, bool NEST>
-__global__ __launch_bounds__(64 * (WCOL + 1)) void k_moments(MomArgs A) {
+__device__ __forceinline__ void moments_columns(const MomPatch &P, const vx_fields &fl, const double *tabs, int blk,
+                                                double *lds) {
     constexpr int NR = RTB == 1 ? 1 : 5;  // rows of f that a column's values read
     constexpr int WDEPTH = RTB == 1 ? 4 : 2;
     constexpr int NCH = WCOL * RTB;
-    const vx_patch &P = A.p;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = (int)(threadIdx.x & 63);
-    const int i0 = (int)blockIdx.x * WCOL;
+    const int i0 = blk * WCOL;
     // buffer, charge/current, chain, p-cell of the chunk (rows of 65: the
     // consumer's lanes read one row each, in different LDS banks)
-    __shared__ double T[2][2][NCH][65];
+    double(*T)[2][NCH][65] = reinterpret_cast<double(*)[2][NCH][65]>(lds);
     const int nchunk = (P.n_p + 63) / 64;
     if (wave < WCOL) {
         const int i = i0 + wave;
@@ -190,14 +210,14 @@ __global__ __launch_bounds__(64 * (WCOL + 1)) void k_moments(MomArgs A) {
         // the sub-columns' A^2 and a logarithm table built for them, if there is one
         double asq[RTB];
 #pragma unroll
-        for (int s = 0; s < RTB; s++) asq[s] = P.q * P.q * cell_a2(A.fl, (long)(ic + P.x_pos) * RTB + s);
+        for (int s = 0; s < RTB; s++) asq[s] = P.q * P.q * cell_a2(fl, (long)(ic + P.x_pos) * RTB + s);
         const double *tab = nullptr;
-        for (int q = 1; q >= 0 && A.tab && !tab; q--) {
-            const double *kt = A.tab + q * TAB_HEAD;
+        for (int q = 1; q >= 0 && tabs && !tab; q--) {
+            const double *kt = tabs + q * TAB_HEAD;
             bool all = kt[TAB_KEY] != 0.0;
 #pragma unroll
             for (int s = 0; s < RTB; s++) all = all && asq[s] == kt[0];
-            if (all) tab = A.tab + tab_entries(q, P.n_p);
+            if (all) tab = tabs + tab_entries(q, P.n_p);
         }
         // Chunk k (jb = 64 k) loads entry r = jb + l of two sequences: the
         // column's f from p = -1 (f at p-cell jb - 1 + l; rows ic - 2 .. ic + 2
@@ -206,11 +226,11 @@ __global__ __launch_bounds__(64 * (WCOL + 1)) void k_moments(MomArgs A) {
         // the nested flag of p-cell jb + l, clamped to the last; those clamped
         // entries serve skipped cells only.  The chunk's address is scalar, the
         // lane adds a 32-bit offset.
-        const double *row = P.f[1] + pidx(P.pitch, RTB == 1 ? ic : ic - 2, -1);
+        const double *row = P.f + pidx(P.pitch, RTB == 1 ? ic : ic - 2, -1);
         const uint8_t *nrow = NEST ? P.nested + pidx(P.pitch, ic, 0) : nullptr;
         auto h = [&](int m, double a2) {
             const double pm = momentum(P.pmin, P.dp, m, P.p_pos);
-            return gamma_(pm, a2, P.mc2inv) + A.c1 * pm;
+            return gamma_(pm, a2, P.mc2inv) + P.c1 * pm;
         };
         // sub-cell values of a p-cell from its rows (Rectangle.cpp:76-110)
         auto values = [&](const double *f, double *v) __attribute__((always_inline)) {
@@ -227,10 +247,10 @@ __global__ __launch_bounds__(64 * (WCOL + 1)) void k_moments(MomArgs A) {
             double te = 0.0;
 #pragma unroll
             for (int s = 0; s < RTB; s++) {
-                v[s] = A.rel[3 * s] * a1 + A.rel[3 * s + 1] * a2 + A.rel[3 * s + 2] * a3 + f3;
+                v[s] = P.rel[3 * s] * a1 + P.rel[3 * s + 1] * a2 + P.rel[3 * s + 2] * a3 + f3;
                 te += v[s] + 0.0;  // the interpolant with a zero correction
             }
-            const double corr = f3 - A.inv_rtb * te;
+            const double corr = f3 - P.inv_rtb * te;
 #pragma unroll
             for (int s = 0; s < RTB; s++) v[s] = v[s] + corr;
         };
@@ -279,7 +299,7 @@ __global__ __launch_bounds__(64 * (WCOL + 1)) void k_moments(MomArgs A) {
                         continue;
                     }
                     const double hm = h(jb + lane, asq[s]), hs = shup1(hm);
-                    out[s] = A.c2 * log_ratio(hm, lane == 0 ? hl[s] : hs);
+                    out[s] = P.c2 * log_ratio(hm, lane == 0 ? hl[s] : hs);
                     hl[s] = __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(hm), 63),
                                              __builtin_amdgcn_readlane(__double2loint(hm), 63));
                 }
@@ -316,7 +336,7 @@ __global__ __launch_bounds__(64 * (WCOL + 1)) void k_moments(MomArgs A) {
                         double t0, tp;
                         next2_rot(lane, V[s], Vn[s], t0, tp);
                         const double tm = V[s], gm1 = L[s < NL ? s : 0];
-                        const double jv = t0 * gm + A.c3 * (gp1 - gm1) * (tp - tm);
+                        const double jv = t0 * gm + P.c3 * (gp1 - gm1) * (tp - tm);
                         const double tr = skip ? -0.0 : t0, tj = skip ? -0.0 : jv;
                         if (COMP) {
                             add_two(aR[s], cR[s], tr);
@@ -346,8 +366,8 @@ __global__ __launch_bounds__(64 * (WCOL + 1)) void k_moments(MomArgs A) {
                 wave_two_sum(aR[s], cR[s], sr, er);
                 wave_two_sum(aJ[s], cJ[s], sj, ej);
                 if (lane == 0 && col_ok) {
-                    P.chargeR[(long)i * RTB + s] = (sr + er) * A.dpq;
-                    P.currentR[(long)i * RTB + s] = (sj + ej) * A.jscale;
+                    P.chargeR[(long)i * RTB + s] = (sr + er) * P.dpq;
+                    P.currentR[(long)i * RTB + s] = (sj + ej) * P.jscale;
                 }
             }
         }
@@ -373,9 +393,35 @@ __global__ __launch_bounds__(64 * (WCOL + 1)) void k_moments(MomArgs A) {
         const int i = i0 + c / RTB;
         if (c < NCH && i < P.n_x) {
             const long e = (long)i * RTB + c % RTB;
-            if (lane < 32) P.chargeR[e] = acc * A.dpq;
-            else P.currentR[e] = acc * A.jscale;
+            if (lane < 32) P.chargeR[e] = acc * P.dpq;
+            else P.currentR[e] = acc * P.jscale;
         }
+    }
+}
+
+template <int RTB, bool COMP, bool NEST>
+__global__ __launch_bounds__(64 * (WCOL + 1)) void k_moments(MomArgs A) {
+    __shared__ double T[COMP ? 1 : 2 * 2 * WCOL * RTB * 65];
+    moments_columns<RTB, COMP, NEST>(A.p, A.fl, A.tab, (int)blockIdx.x, T);
+}
+
+// The patches of a hierarchy in one launch, without tables.  A patch's own launch
+// leaves most of the chip idle at its end (and, for a coarse patch, throughout).
+// Measured on an MI355X: MB_TXT
+template <bool COMP>
+__global__ __launch_bounds__(64 * (WCOL + 1)) void k_moments_batch(MomBatch A) {
+    __shared__ double T[COMP ? 1 : 2 * 2 * WCOL * MAX_RTB * 65];
+    int k = 0;
+    while (k + 1 < A.n && (int)blockIdx.x >= A.start[k + 1]) k++;
+    const MomPatch P = A.p[k];
+    const int blk = (int)blockIdx.x - A.start[k];
+    switch (P.rtb * 2 + (P.nested ? 1 : 0)) {
+        case 2: moments_columns<1, COMP, false>(P, A.fl, nullptr, blk, T); break;
+        case 3: moments_columns<1, COMP, true>(P, A.fl, nullptr, blk, T); break;
+        case 4: moments_columns<2, COMP, false>(P, A.fl, nullptr, blk, T); break;
+        case 5: moments_columns<2, COMP, true>(P, A.fl, nullptr, blk, T); break;
+        case 8: moments_columns<4, COMP, false>(P, A.fl, nullptr, blk, T); break;
+        default: moments_columns<4, COMP, true>(P, A.fl, nullptr, blk, T);
     }
 }
 
@@ -385,13 +431,12 @@ __global__ __launch_bounds__(64 * (WCOL + 1)) void k_moments(MomArgs A) {
 // energyR entries from several threads; the oracle and this kernel use the
 // sequential order).
 template <int RTB>
-__global__ __launch_bounds__(256) void k_energy(MomArgs A, double *energyR) {
-    const vx_patch &P = A.p;
+__global__ __launch_bounds__(256) void k_energy(MomPatch P, double *energyR) {
     const int e = blockIdx.x * blockDim.x + threadIdx.x;
     if (e >= P.n_p * RTB) return;
     const int j = e / RTB, k = e % RTB;
     const int pitch = P.pitch;
-    const double *g = P.f[1];
+    const double *g = P.f;
     double acc = 0.0;
     for (int i = 0; i < P.n_x; i++) {
         if (P.nested && P.nested[pidx(pitch, i, j)]) continue;
@@ -401,7 +446,7 @@ __global__ __launch_bounds__(256) void k_energy(MomArgs A, double *energyR) {
         double a1 = kInterp[0] * f1 + kInterp[1] * f2 + kInterp[2] * f4 + kInterp[3] * f5;
         double a2 = kInterp[4] * f1 + kInterp[5] * f2 + kInterp[6] * f4 + kInterp[7] * f5;
         double a3 = kInterp[8] * f1 + kInterp[9] * f2 + kInterp[10] * f4 + kInterp[11] * f5;
-        acc += A.rel[3 * k] * a1 + A.rel[3 * k + 1] * a2 + A.rel[3 * k + 2] * a3 + f3;
+        acc += P.rel[3 * k] * a1 + P.rel[3 * k + 1] * a2 + P.rel[3 * k + 2] * a3 + f3;
     }
     energyR[(long)j * RTB + k] = acc * P.dx;
 }
@@ -442,26 +487,25 @@ __global__ void k_assemble(const MomentSrc *src, const int *level_start, int n_s
     J[x] = jsum;
 }
 
-void fill_args(MomArgs &A, const vx_patch *p, const vx_fields *fl) {
-    A.p = *p;
-    if (fl) A.fl = *fl;
-    double m_inv = 1 / p->m;
-    A.c1 = m_inv * vx_c_inv;
-    A.c2 = 1 / A.c1;
-    A.c3 = 1 / 48.0;
-    double rtb = (double)p->rtb;
-    A.inv_rtb = 1.0 / rtb;
-    A.dpq = p->dp * p->q;
-    A.jscale = -p->q * p->q / p->m;
-    for (int i = 0; i < 3 * MAX_RTB; i++) A.rel[i] = 0.0;
-    for (int i = 0; i < p->rtb; i++) {  // Rectangle.cpp:103-110
+MomPatch mom_patch(const vx_patch &p) {
+    MomPatch M{p.f[1], p.nested, p.chargeR, p.currentR, p.n_x, p.n_p, p.x_pos, p.p_pos, p.rtb, p.pitch,
+               p.dx, p.dp, p.pmin, p.q, p.mc2inv};
+    double m_inv = 1 / p.m;
+    M.c1 = m_inv * vx_c_inv;
+    M.c2 = 1 / M.c1;
+    M.c3 = 1 / 48.0;
+    double rtb = (double)p.rtb;
+    M.inv_rtb = 1.0 / rtb;
+    M.dpq = p.dp * p.q;
+    M.jscale = -p.q * p.q / p.m;
+    for (int i = 0; i < std::min(p.rtb, MAX_RTB); i++) {  // Rectangle.cpp:103-110
         double tl = -0.5 + i / rtb;
         double tr = -0.5 + (i + 1.0) / rtb;
-        A.rel[3 * i] = (tl + tr) * 0.5;
-        A.rel[3 * i + 1] = (tl * tl + tl * tr + tr * tr) / 3.0 - (1.0 / 12);
-        A.rel[3 * i + 2] = (tl * tl * tl + tl * tl * tr + tl * tr * tr + tr * tr * tr) * 0.25;
+        M.rel[3 * i] = (tl + tr) * 0.5;
+        M.rel[3 * i + 1] = (tl * tl + tl * tr + tr * tr) / 3.0 - (1.0 / 12);
+        M.rel[3 * i + 2] = (tl * tl * tl + tl * tl * tr + tl * tr * tr + tr * tr * tr) * 0.25;
     }
-    A.tab = nullptr;
+    return M;
 }
 
 }  // namespace
@@ -472,8 +516,7 @@ int vx_energy_patch(vx_ctx *ctx, const vx_patch *p, double *energyR) {
     int rc = validate_patch(ctx, p);
     if (rc) return rc;
     if (!energyR) return fail(ctx, VX_EINVAL, "energy: null output");
-    MomArgs A{};
-    fill_args(A, p, nullptr);
+    const MomPatch A = mom_patch(*p);
     const unsigned nb = (unsigned)((p->n_p * p->rtb + 255) / 256);
     switch (p->rtb) {
         case 1: k_energy<1><<<nb, 256, 0, ctx->stream>>>(A, energyR); break;
@@ -486,16 +529,21 @@ int vx_energy_patch(vx_ctx *ctx, const vx_patch *p, double *energyR) {
 
 }  // extern "C"
 
-static int moments_patch(vx_ctx *ctx, const vx_patch *p, const vx_fields *fl, bool comp) {
+static int moments_check(vx_ctx *ctx, const vx_patch *p, const vx_fields *fl) {
     int rc = validate_patch(ctx, p);
     if (rc) return rc;
     if (p->rtb > MAX_RTB) return fail(ctx, VX_ENOTSUP, "moments: relativeToBottom %d > %d", p->rtb, MAX_RTB);
     if (!fl) return fail(ctx, VX_EINVAL, "moments: null fields");
     if ((rc = validate_span(ctx, p, fl->n_f))) return rc;
-    MomArgs A;
-    fill_args(A, p, fl);
     if (p->rtb != 1 && p->rtb != 2 && p->rtb != 4)
         return fail(ctx, VX_ENOTSUP, "moments: relativeToBottom %d not in {1,2,4}", p->rtb);
+    return VX_OK;
+}
+
+static int moments_patch(vx_ctx *ctx, const vx_patch *p, const vx_fields *fl, bool comp) {
+    int rc = moments_check(ctx, p, fl);
+    if (rc) return rc;
+    MomArgs A{mom_patch(*p), *fl, nullptr};
     // The table saves each column its logarithms but costs a launch (3.1 us).
     // us with / without it: 1024 x 512 at rtb 1 8.3 / 7.0, 1024 x 1024 11.2 / 10.7,
     // 2048 x 1024 12.1 / 15.4; 2000 x 64 at rtb 4 7.8 / 6.1, 512 x 512 11.4 / 12.4,
@@ -550,6 +598,37 @@ int vx_moments_patch(vx_ctx *ctx, const vx_patch *p, const vx_fields *fl) {
 
 int vx_moments_patch_compensated(vx_ctx *ctx, const vx_patch *p, const vx_fields *fl) {
     return moments_patch(ctx, p, fl, true);
+}
+
+int vx_moments_patches(vx_ctx *ctx, const vx_patch *patches, int32_t n, const vx_fields *fl, int compensated) {
+    if (n < 0 || (n > 0 && !patches)) return fail(ctx, VX_EINVAL, "moments: bad patch list");
+    int rc;
+    for (int k = 0; k < n; k++)
+        if ((rc = moments_check(ctx, patches + k, fl))) return rc;
+    MomBatch B;
+    B.n = 0;
+    // the last patches first (a hierarchy lists its levels finest first, and a
+    // coarse patch's workgroups run longest)
+    for (int k = n; k-- > 0;) {
+        const vx_patch &p = patches[k];
+        const bool alone = n == 1 || (long)p.n_x * p.n_p > BATCH_CELLS;
+        if (alone) {
+            if ((rc = moments_patch(ctx, &p, fl, compensated != 0))) return rc;
+        } else {
+            if (B.n == 0) B.start[0] = 0;
+            B.p[B.n++] = mom_patch(p);
+            B.start[B.n] = B.start[B.n - 1] + (p.n_x + WCOL - 1) / WCOL;
+        }
+        if (B.n == MOM_BATCH || (k == 0 && B.n > 0)) {
+            B.fl = *fl;
+            LaunchTimer lt(ctx, "k_moments");
+            if (compensated) k_moments_batch<true><<<(unsigned)B.start[B.n], 64 * WCOL, 0, ctx->stream>>>(B);
+            else k_moments_batch<false><<<(unsigned)B.start[B.n], 64 * (WCOL + 1), 0, ctx->stream>>>(B);
+            if ((rc = check_launch(ctx, "k_moments_batch"))) return rc;
+            B.n = 0;
+        }
+    }
+    return VX_OK;
 }
 
 int vx_moment_plan_create(vx_ctx *ctx, const vx_patch *patches, const vx_moment_layout *lay,
