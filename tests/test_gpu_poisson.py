@@ -1,5 +1,5 @@
 """vx_poisson at the edges of its forms (wavefronts, entries a thread, sub-chunks
-of 64, chunks of 512 and the two solvers' border at 4096), through the C ABI, against the
+of 64, chunks of 192 and 512, the solvers' borders at 4096 and 36864), through the C ABI, against the
 oracle's solve of the same right-hand side: both converge to the correctly
 rounded solution (a near-tie may differ by 1 ulp), E and Ex0 follow from phi.
 Smooth, random and zero charges; a second call repeats the first's bits."""
@@ -16,7 +16,8 @@ from test_zz_no_alloc import State, kernels
 pytestmark = pytest.mark.gpu
 
 SIZES = [8, 10, 16, 34, 64, 66, 128, 130, 256, 258, 512, 514, 1024, 1026, 2048, 2050, 4094, 4096,
-         4098, 4114, 4160, 4162, 4606, 4608, 4610, 4628, 8190, 8192, 10000, 20002, 40000, 65536, 70000]
+         4098, 4114, 4160, 4162, 4224, 4226, 4606, 4608, 4610, 4628, 8190, 8192, 10000, 20002, 36864, 36866,
+         40000, 65536, 70000]
 EPS0_INV = 1.1294e+11
 
 

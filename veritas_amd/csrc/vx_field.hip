@@ -80,9 +80,8 @@ __device__ __forceinline__ void dd_sub(double &sh, double &sl, double a, double 
 }
 
 // ------------------------------------------------ multi-workgroup solve, n_f > 4096
-// Workgroup b owns the chunk of CHUNK consecutive entries [b CHUNK, (b + 1)
-// CHUNK), wavefront w of it the sub-chunk w of 64 entries.  One approximate
-// solve of A c = v and the residual of the next round are one launch:
+// Workgroup b owns the chunk of 64 MW consecutive entries [64 MW b, 64 MW (b +
+// 1)), wavefront w of it the sub-chunk w of 64 entries.  One approximate solve of A c = v and the residual of the next round are one launch:
 //   S_i = sum_{k<i} v'_k with v'_0 = -tail, tail = sum_{k>=1} v_k,
 //   d0 = mean(S), D_i = d0 - S_i (D_0 = 0), y_i = sum_{k<=i} D_k,
 //   c = M^-1 y - (M^-1 y)_0 with c_0 from row 0, x (+)= c, then either the
@@ -102,16 +101,22 @@ __device__ __forceinline__ void dd_sub(double &sh, double &sl, double a, double 
 // Ex0).  x and r alternate between two buffers: a launch reads one and writes
 // the other.
 // Bound by launch latency and each launch's chain (sums, two scans,
-// convolution, residual, sums).  32768 entries on an MI355X: 77 us as 13
-// launches (the two scans and the convolution apart), 42 us as 5.
-constexpr int SUB = 64, MW = 8, CHUNK = SUB * MW;
-constexpr int MT = 64 * (MW + 5);  // k_pm_solve: a wavefront per sub-chunk that it forms
+// convolution, residual, sums), and by FP64 issue where a CU has many
+// wavefronts: five more than the chunk's form y.  MW = 3 gives a SIMD two of the
+// eight and 32768 entries 171 CUs; above PM_SMALL the sums over the chunks weigh
+// more, and MW = 8 has fewer.  us on an MI355X at 8192, 32768 and 100000 entries: MW =
+// 2 29, 33, 97; 3 28, 31, 65; 4 32, 34, 56; 8 39, 38, 44.  32768 entries took 77 us
+// as 13 launches (the two scans and the convolution apart), 42 us as 5 with MW = 8 and
+// each launch's reads one behind the other.
+constexpr int PM_SMALL = 192 * 192;  // largest n_f with MW = 3: three chunks a lane
+__host__ __device__ constexpr int pm_mw(int n) { return n <= PM_SMALL ? 3 : 8; }
+constexpr int SUB = 64;
 constexpr int HALO = 2;
 constexpr int CW = NG - 1 + HALO;  // y window margin: convolution reach + halo
 constexpr int NSPEC = 6;           // entries N-3, N-2, N-1, 0, 1, 2
 constexpr int YS = NSPEC + 2 * (NG - 1);  // y window of those entries
 
-__host__ __device__ constexpr int pm_chunks(int n) { return (n + CHUNK - 1) / CHUNK; }
+__host__ __device__ constexpr int pm_chunks(int n) { return (n + SUB * pm_mw(n) - 1) / (SUB * pm_mw(n)); }
 
 // M and P of a chunk or sub-chunk, double-double
 struct PmSum {
@@ -125,7 +130,7 @@ struct PmWork {
     PmSum *sums[2];
 };
 __host__ __device__ inline PmWork pm_work(double *w, int n) {
-    const size_t N = n, ns = (size_t)pm_chunks(n) * (1 + MW);
+    const size_t N = n, ns = (size_t)pm_chunks(n) * (1 + pm_mw(n));
     PmWork W;
     W.b = w;
     W.xa = w + N;
@@ -189,9 +194,17 @@ __device__ __forceinline__ DD wave_dd_sum(DD v) {
     return {lane63(v.h), lane63(v.l)};
 }
 
+// sum over lanes 0..7, in lane 7 (wave_scan_dpp's first steps)
+__device__ __forceinline__ DD row_dd_sum8(DD v) {
+    v = dd_step<0x111, 0xf>(v);
+    v = dd_step<0x112, 0xf>(v);
+    return dd_step<0x114, 0xf>(v);
+}
+
 // M and P of a wavefront's 64 entries v (entry 0 and entries past N passed as
 // 0) and of the workgroup's chunk of n_own entries, into out.  P is the sum of v_l
 // (n - 1 - l), n the wavefront's entries below N.
+template <int MW>
 __device__ __forceinline__ void pm_store_sums(double v, int n_own, PmSum *out, int nb, PmSum *ms) {
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, blk = blockIdx.x;
     const int n = min(SUB, n_own - w * SUB);
@@ -209,15 +222,17 @@ __device__ __forceinline__ void pm_store_sums(double v, int n_own, PmSum *out, i
             M = {ms[lane].mh, ms[lane].ml};
             P = dd_add({ms[lane].ph, ms[lane].pl}, dd_mul(M, (double)(n_own - end)));
         }
-        M = wave_dd_sum(M);
-        P = wave_dd_sum(P);
-        if (lane == 0) out[blk] = {M.h, M.l, P.h, P.l};
+        M = row_dd_sum8(M);
+        P = row_dd_sum8(P);
+        if (lane == 7) out[blk] = {M.h, M.l, P.h, P.l};
     }
 }
 
 // b = dx^2 eps0_inv (charge + neutral) (EMSolver.cpp:157-167), its sums over
 // entries >= 1, and the entry value of Ex0
-__global__ __launch_bounds__(CHUNK) void k_pm_rhs(PoissonMB P) {
+template <int MW>
+__global__ __launch_bounds__(SUB *MW) void k_pm_rhs(PoissonMB P) {
+    constexpr int CHUNK = SUB * MW;
     __shared__ PmSum ms[MW];
     const vx_field_state &F = P.fs;
     const int N = F.n_f, i = blockIdx.x * CHUNK + threadIdx.x;
@@ -227,14 +242,15 @@ __global__ __launch_bounds__(CHUNK) void k_pm_rhs(PoissonMB P) {
         v *= F.dx2;
         P.W.b[i] = v;
     }
-    pm_store_sums(i >= 1 ? v : 0.0, min(CHUNK, N - (int)blockIdx.x * CHUNK), P.sums_out, P.nb, ms);
+    pm_store_sums<MW>(i >= 1 ? v : 0.0, min(CHUNK, N - (int)blockIdx.x * CHUNK), P.sums_out, P.nb, ms);
     if (i == 0) *P.W.ex0 = *F.Ex0;
 }
 
 // MODE 0: first solve (x = c); 1: refinement (x += c); both then form the next
 // residual.  MODE 2: last refinement, writes phi (x_out), Ex0 and E.
-template <int MODE>
-__global__ __launch_bounds__(MT) void k_pm_solve(PoissonMB P) {
+template <int MODE, int MW>
+__global__ __launch_bounds__(64 * (MW + 5)) void k_pm_solve(PoissonMB P) {
+    constexpr int CHUNK = SUB * MW, MT = 64 * (MW + 5);
     __shared__ double yw[CHUNK + 2 * CW];
     __shared__ double ys[YS];
     __shared__ double xw[CHUNK + 2 * HALO];
@@ -249,6 +265,12 @@ __global__ __launch_bounds__(MT) void k_pm_solve(PoissonMB P) {
     const bool own = j >= HALO && j < n_own + HALO, have = j < n_own + 2 * HALO;
     const double xo = MODE > 0 && have ? P.x_in[gi] : 0.0;
     const double bv = MODE < 2 && j < n_own ? P.W.b[lo + j] : 0.0;
+    double ps[NSPEC], ex0 = 0.0;  // MODE 2: x around entry 0, then phi; Ex0 on entry
+    if (MODE == 2) {
+#pragma unroll
+        for (int k = 0; k < NSPEC; k++) ps[k] = P.x_in[wrap(k - 3, N)];
+        ex0 = *P.W.ex0;
+    }
     const PmSum *C = P.sums, *U = C + nb;  // chunks, sub-chunks
     // (sum v, sum v (pos - 1 - i)) of item q that ends at `end`, seen from pos
     auto item = [](const PmSum &q, int pos, int end, DD &t, DD &g) {
@@ -256,22 +278,34 @@ __global__ __launch_bounds__(MT) void k_pm_solve(PoissonMB P) {
         t = dd_add(t, m);
         g = dd_add(g, dd_add(dd_mul(m, (double)(pos - end)), {q.ph, q.pl}));
     };
-    // over every chunk: tail and d0
-    DD t{0.0, 0.0}, g{0.0, 0.0};
-    for (int q = lane; q < nb; q += 64) item(C[q], N, min((q + 1) * CHUNK, N), t, g);
+    // the wavefront's sub-chunk: the chunk's, the neighbours' and those around entry
+    // 0 (the last one may be shorter than the window, hence the one before it too);
+    // none for some (s < 0 or s >= ns)
+    const int ns = (N + SUB - 1) / SUB, s0 = blk * MW;
+    const int s = w < MW ? s0 + w : w == MW ? s0 - 1 : w == MW + 1 ? s0 + MW : w == MW + 2 ? 0 : ns - (w - MW - 2);
+    const int b = s / MW, i0 = s * SUB, i = i0 + lane;
+    const bool sub = s >= 0 && s < ns;
+    // what the steps below read from memory, all in flight at once
+    const double in = sub && i < N ? P.in[i] : 0.0, in0 = P.in[0];
+    PmSum u{0.0, 0.0, 0.0, 0.0};
+    if (sub && lane < s - b * MW) u = U[b * MW + lane];
+    // tail and d0 over every chunk (t, g), S and the sum of D before the sub-chunk (a, h)
+    DD t{0.0, 0.0}, g{0.0, 0.0}, a{0.0, 0.0}, h{0.0, 0.0};
+    for (int q = lane; q < nb; q += 64) {
+        const PmSum c = C[q];
+        item(c, N, min((q + 1) * CHUNK, N), t, g);
+        if (q < b) item(c, i0, (q + 1) * CHUNK, a, h);
+    }
+    item(u, i0, (b * MW + lane + 1) * SUB, a, h);
     const DD tail = wave_dd_sum(t);
-    g = dd_add(wave_dd_sum(g), dd_mul(tail, -(double)(N - 1)));
+    g = wave_dd_sum(g);
+    a = wave_dd_sum(a);
+    h = wave_dd_sum(h);
+    g = dd_add(g, dd_mul(tail, -(double)(N - 1)));
     const double d0 = (g.h + g.l) * P.invN, tl = tail.h + tail.l;
-    // y of sub-chunk s, into the windows it reaches
-    auto sub_y = [&](int s) {
-        const int b = s / MW, i0 = s * SUB, i = i0 + lane;
-        const double in = i < N ? P.in[i] : 0.0;
-        // S and the sum of D before the sub-chunk
-        DD a{0.0, 0.0}, h{0.0, 0.0};
-        for (int q = lane; q < b; q += 64) item(C[q], i0, (q + 1) * CHUNK, a, h);
-        if (lane < s - b * MW) item(U[b * MW + lane], i0, (b * MW + lane + 1) * SUB, a, h);
-        a = dd_add(wave_dd_sum(a), dd_neg(tail));
-        h = dd_add(wave_dd_sum(h), dd_mul(tail, -(double)(i0 - 1)));
+    if (sub) {  // y, into the windows it reaches
+        a = dd_add(a, dd_neg(tail));
+        h = dd_add(h, dd_mul(tail, -(double)(i0 - 1)));
         h = dd_add(dd_mul({d0, 0.0}, (double)(i0 - 1)), dd_neg(h));
         // (entry 0: S = 0, D = 0)
         const double S = s == 0 ? 0.0 : a.h + a.l, Y = s == 0 ? 0.0 : h.h + h.l;
@@ -279,29 +313,28 @@ __global__ __launch_bounds__(MT) void k_pm_solve(PoissonMB P) {
         const double Si = S + dpp_or_0<0x138>(wave_scan_dpp(v));
         const double Di = (i == 0 || i >= N) ? 0.0 : d0 - Si;
         const double y = Y + wave_scan_dpp(Di);
-        if (i >= N) return;
-        for (int img = -N; img <= N; img += N) {
-            const int p = i + img - lo + CW;
-            if (p >= 0 && p < n_own + 2 * CW) yw[p] = y;
+        if (i < N) {
+            for (int img = -N; img <= N; img += N) {
+                const int p = i + img - lo + CW;
+                if (p >= 0 && p < n_own + 2 * CW) yw[p] = y;
+            }
+            const int e = i < N - i ? i + 3 + NG - 1 : i - N + 3 + NG - 1;
+            if (e >= 0 && e < YS) ys[e] = y;
         }
-        const int e = i < N - i ? i + 3 + NG - 1 : i - N + 3 + NG - 1;
-        if (e >= 0 && e < YS) ys[e] = y;
-    };
-    // the chunk's sub-chunks, the neighbours' and those around entry 0 (the last
-    // one may be shorter than the window, hence the one before it too)
-    const int ns = (N + SUB - 1) / SUB, s0 = blk * MW;
-    const int sub = w < MW ? s0 + w : w == MW ? s0 - 1 : w == MW + 1 ? s0 + MW : w == MW + 2 ? 0 : ns - (w - MW - 2);
-    if (sub >= 0 && sub < ns) sub_y(sub);
+    }
     __syncthreads();
-    if (threadIdx.x < NSPEC) cs[threadIdx.x] = conv_at(ys, threadIdx.x + NG - 1, P.g);
+    // M^-1 y at this thread's entry, and (by the last wavefront) around entry 0
+    const double my = have ? conv_at(yw, j + NG - 1, P.g) : 0.0;
+    const int e0 = (int)threadIdx.x - (MT - 64);
+    if (e0 >= 0 && e0 < NSPEC) cs[e0] = conv_at(ys, e0 + NG - 1, P.g);
     __syncthreads();
     const double cp0 = cs[3];  // (M^-1 y)_0
     // row 0 (the approximate solve's last step): c_0 from c_1, c_2, c_{N-2}, c_{N-1}
-    const double c0 = P.in[0] - (((P.w1 * (cs[4] - cp0) + P.w2 * (cs[5] - cp0)) + P.w2 * (cs[1] - cp0)) +
-                                 P.w1 * (cs[2] - cp0));
+    const double c0 = in0 - (((P.w1 * (cs[4] - cp0) + P.w2 * (cs[5] - cp0)) + P.w2 * (cs[1] - cp0)) +
+                             P.w1 * (cs[2] - cp0));
     // x on the chunk and its halo
     if (have) {
-        const double c = gi == 0 ? c0 : conv_at(yw, j + NG - 1, P.g) - cp0;
+        const double c = gi == 0 ? c0 : my - cp0;
         const double xn = MODE == 0 ? c : xo + c;
         xw[j] = xn;
         if (own) P.x_out[gi] = xn;
@@ -327,16 +360,13 @@ __global__ __launch_bounds__(MT) void k_pm_solve(PoissonMB P) {
             r = sh + sl;
             P.r_out[i] = r;
         }
-        pm_store_sums(i >= 1 ? r : 0.0, n_own, P.sums_out, nb, ms);
+        pm_store_sums<MW>(i >= 1 ? r : 0.0, n_own, P.sums_out, nb, ms);
     } else {
         // EMSolver.cpp:191: Ex0 += -(E(-1) + E(0)) * 0.5 with the entry Ex0, from phi
         // at N-3..N-1, 0..2 (recomputed here with the owners' operations)
-        double ps[NSPEC];
 #pragma unroll
-        for (int k = 0; k < NSPEC; k++) {
-            ps[k] = P.x_in[wrap(k - 3, N)] + (k == 3 ? c0 : cs[k] - cp0);
-        }
-        const double ex0 = *P.W.ex0, fc = F.field_coef;
+        for (int k = 0; k < NSPEC; k++) ps[k] = ps[k] + (k == 3 ? c0 : cs[k] - cp0);
+        const double fc = F.field_coef;
         const double e_m1 = -fc * (8 * (ps[3] - ps[1]) - ps[4] + ps[0]) + ex0;
         const double e_0 = -fc * (8 * (ps[4] - ps[2]) - ps[5] + ps[1]) + ex0;
         const double ex0n = ex0 + -(e_m1 + e_0) * 0.5;
@@ -852,10 +882,13 @@ __global__ void k_neutralize(vx_field_state F) {
 // device current (scratch_address, at context creation).
 __host__ __device__ constexpr size_t pm_work_elems(int n) { return 7 * (size_t)n + 2 * (((size_t)n + 1023) / 1024) + 1; }
 constexpr size_t NOALLOC_WORK = pm_work_elems(VX_POISSON_NOALLOC_MAX_NF);
-// pm_work's 5 n + 1 doubles and 72 per chunk of sums fit for
-// every n that the multi-workgroup solve serves
-static_assert(5 * 4097 + 1 + pm_chunks(4097) * 2 * 4 * (1 + MW) <= pm_work_elems(4097), "work array");
-static_assert(2 * CHUNK > 2 * 4 * (1 + MW), "sums per chunk against 2 doubles per entry");
+// pm_work's 5 n + 1 doubles and 8 (1 + MW) per chunk of sums fit for every n that
+// the multi-workgroup solve serves
+constexpr bool pm_fits(int n) {
+    return 5 * (size_t)n + 1 + (size_t)pm_chunks(n) * 2 * 4 * (1 + pm_mw(n)) <= pm_work_elems(n);
+}
+static_assert(pm_fits(4097) && pm_fits(PM_SMALL) && pm_fits(PM_SMALL + 1), "work array");
+static_assert(2 * SUB > 2 * 4 * 2, "sums per sub-chunk (and its share of its chunk's) against 2 doubles per entry");
 static __device__ __align__(256) double scratch[NOALLOC_WORK];
 constexpr int MAX_DEVICES = 64;
 static std::mutex scratch_mu;
@@ -940,7 +973,9 @@ static int poisson(vx_ctx *ctx, const vx_field_state *fs, double *work) {
     const PmWork &W = M.W;
     const unsigned nb = (unsigned)M.nb;
     M.sums_out = W.sums[0];
-    k_pm_rhs<<<nb, CHUNK, 0, ctx->stream>>>(M);
+    const bool small = pm_mw(fs->n_f) == 3;
+    if (small) k_pm_rhs<3><<<nb, SUB * 3, 0, ctx->stream>>>(M);
+    else k_pm_rhs<8><<<nb, SUB * 8, 0, ctx->stream>>>(M);
     // four approximate solves: of b (x = c), then of three residuals (x += c)
     const double *in[4] = {W.b, W.ra, W.rb, W.ra};
     double *r_out[4] = {W.ra, W.rb, W.ra, nullptr};
@@ -953,9 +988,15 @@ static int poisson(vx_ctx *ctx, const vx_field_state *fs, double *work) {
         M.x_out = x_out[s];
         M.sums = W.sums[s & 1];
         M.sums_out = W.sums[~s & 1];
-        if (s == 0) k_pm_solve<0><<<nb, MT, 0, ctx->stream>>>(M);
-        else if (s < 3) k_pm_solve<1><<<nb, MT, 0, ctx->stream>>>(M);
-        else k_pm_solve<2><<<nb, MT, 0, ctx->stream>>>(M);
+        if (small) {
+            if (s == 0) k_pm_solve<0, 3><<<nb, 64 * 8, 0, ctx->stream>>>(M);
+            else if (s < 3) k_pm_solve<1, 3><<<nb, 64 * 8, 0, ctx->stream>>>(M);
+            else k_pm_solve<2, 3><<<nb, 64 * 8, 0, ctx->stream>>>(M);
+        } else {
+            if (s == 0) k_pm_solve<0, 8><<<nb, 64 * 13, 0, ctx->stream>>>(M);
+            else if (s < 3) k_pm_solve<1, 8><<<nb, 64 * 13, 0, ctx->stream>>>(M);
+            else k_pm_solve<2, 8><<<nb, 64 * 13, 0, ctx->stream>>>(M);
+        }
     }
     return check_launch(ctx, "k_poisson");
 }

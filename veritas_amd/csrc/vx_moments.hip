@@ -407,7 +407,8 @@ __global__ __launch_bounds__(64 * (WCOL + 1)) void k_moments(MomArgs A) {
 
 // The patches of a hierarchy in one launch, without tables.  A patch's own launch
 // leaves most of the chip idle at its end (and, for a coarse patch, throughout).
-// Measured on an MI355X: MB_TXT
+// Three patches of 1.27, 0.34 and 1.05 M cells on an MI355X: 43 us, apart 42 us and two
+// checks of the tables, 4.5 us each; 22 steps of the laser run 40.9 -> 39.9 ms.
 template <bool COMP>
 __global__ __launch_bounds__(64 * (WCOL + 1)) void k_moments_batch(MomBatch A) {
     __shared__ double T[COMP ? 1 : 2 * 2 * WCOL * MAX_RTB * 65];
