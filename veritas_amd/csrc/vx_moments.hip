@@ -22,7 +22,7 @@ using namespace vxd;
 namespace {
 
 constexpr int MAX_RTB = 4;  // coarsest level of a 3-level hierarchy at ratio 2
-constexpr long TAB_CELLS = 1 << 19;  // a patch of more cells gets a logarithm table
+constexpr long TAB_CELLS = 1 << 20;  // a patch of more cells gets a logarithm table
 constexpr long BATCH_CELLS = 1 << 21;  // a patch of more cells has a launch (and a table) of its own
 constexpr int TAB_KEY = 8;  // A^2, pmin, dp, p_pos, mc2inv, c1, c2, n_p
 
@@ -546,10 +546,11 @@ static int moments_patch(vx_ctx *ctx, const vx_patch *p, const vx_fields *fl, bo
     if (rc) return rc;
     MomArgs A{mom_patch(*p), *fl, nullptr};
     // The table saves each column its logarithms but costs a launch (3.1 us).
-    // us with / without it: 1024 x 512 at rtb 1 8.3 / 7.0, 1024 x 1024 11.2 / 10.7,
+    // us with / without it: 1024 x 512 at rtb 1 8.3 / 7.0, 1024 x 1024 11.9 / 10.7,
     // 2048 x 1024 12.1 / 15.4; 2000 x 64 at rtb 4 7.8 / 6.1, 512 x 512 11.4 / 12.4,
     // 8000 x 256 27.8 / 33.7; columns with a pulse do not use it (500 x 512 at rtb
-    // 4 21.1 / 19.1).
+    // 4 21.1 / 19.1).  A wavefront that forms the terms for its workgroup's columns
+    // instead: 9.2 at 1024 x 1024, but 52 at 4096 x 4096, 46 with the table.
     if ((long)p->n_x * p->n_p > TAB_CELLS) {
         const size_t need = (size_t)tab_entries(2, p->n_p);
         if (ctx->mom_table_n < need) {
