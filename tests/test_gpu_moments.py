@@ -1,6 +1,7 @@
 """The p-moments (k_moments) against the oracle, bit for bit: column counts that
 leave a partial workgroup, p-columns that end inside, at and just past a 64-cell
-chunk, patches with and without the logarithm table (above 2^20 cells), with and
+chunk, tall columns (8 a workgroup from 2048 p-cells on), patches with and without the
+logarithm table (above 2^20 cells), with and
 without nested cells (levels 3: relativeToBottom 1, 2 and 4), behind and ahead
 of a pulse.  The compensated sums agree with the ordered ones.  A table of
 another patch is never taken for this one's, and several patches in one launch
@@ -20,6 +21,7 @@ from test_zz_no_alloc import kernels
 pytestmark = pytest.mark.gpu
 
 SHAPES = [(1, 8, 8), (1, 10, 62), (1, 34, 64), (1, 30, 66), (1, 12, 128), (1, 1026, 1022), (1, 1026, 1030),
+          (1, 10, 2046), (1, 10, 2048), (1, 14, 2050), (1, 522, 2050),
           (3, 128, 64), (3, 126, 66), (3, 1026, 514)]
 
 

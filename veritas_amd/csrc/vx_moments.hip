@@ -153,7 +153,7 @@ __device__ __forceinline__ void add_two(double &acc, double &cmp, double v) {
 // / 9.8 / 11.4, 500 x 512 at RTB 4 with a pulse 20.5 / 20.9 / 27.1.  One
 // wavefront per 4 sub-columns that adds its own chunk took 64.9, 35.4, 66.9, 27.1
 // and 30.0; two of them, a producer and a consumer, 92.3, 34.8, 80.4, 22.4, 27.5.
-constexpr int WCOL = 4;
+constexpr int MCOL = 4, MCOL_TALL = 8;
 
 // Whole-wavefront rotation by one lane (DPP wave_rol:1): lane l receives the
 // value of lane (l + 1) mod 64.
@@ -191,7 +191,7 @@ __device__ __forceinline__ double log_ratio(double a, double b) {
 // NEST: the patch has nested cells (their summands are -0.0).
 // tabs: the patch's logarithm tables, or null; blk: the workgroup's number in
 // the patch; lds: 2 x 2 x WCOL RTB rows of 65 (not used by COMP).
-template <int RTB, bool COMP, bool NEST>
+template <int RTB, int WCOL, bool COMP, bool NEST>
 __device__ __forceinline__ void moments_columns(const MomPatch &P, const vx_fields &fl, const double *tabs, int blk,
                                                 double *lds) {
     constexpr int NR = RTB == 1 ? 1 : 5;  // rows of f that a column's values read
@@ -399,10 +399,10 @@ __device__ __forceinline__ void moments_columns(const MomPatch &P, const vx_fiel
     }
 }
 
-template <int RTB, bool COMP, bool NEST>
+template <int RTB, bool COMP, bool NEST, int WCOL = MCOL>
 __global__ __launch_bounds__(64 * (WCOL + 1)) void k_moments(MomArgs A) {
     __shared__ double T[COMP ? 1 : 2 * 2 * WCOL * RTB * 65];
-    moments_columns<RTB, COMP, NEST>(A.p, A.fl, A.tab, (int)blockIdx.x, T);
+    moments_columns<RTB, WCOL, COMP, NEST>(A.p, A.fl, A.tab, (int)blockIdx.x, T);
 }
 
 // The patches of a hierarchy in one launch, without tables.  A patch's own launch
@@ -410,19 +410,20 @@ __global__ __launch_bounds__(64 * (WCOL + 1)) void k_moments(MomArgs A) {
 // Three patches of 1.27, 0.34 and 1.05 M cells on an MI355X: 43 us, apart 42 us and two
 // checks of the tables, 4.5 us each; 22 steps of the laser run 40.9 -> 39.9 ms.
 template <bool COMP>
-__global__ __launch_bounds__(64 * (WCOL + 1)) void k_moments_batch(MomBatch A) {
+__global__ __launch_bounds__(64 * (MCOL + 1)) void k_moments_batch(MomBatch A) {
+    constexpr int WCOL = MCOL;
     __shared__ double T[COMP ? 1 : 2 * 2 * WCOL * MAX_RTB * 65];
     int k = 0;
     while (k + 1 < A.n && (int)blockIdx.x >= A.start[k + 1]) k++;
     const MomPatch P = A.p[k];
     const int blk = (int)blockIdx.x - A.start[k];
     switch (P.rtb * 2 + (P.nested ? 1 : 0)) {
-        case 2: moments_columns<1, COMP, false>(P, A.fl, nullptr, blk, T); break;
-        case 3: moments_columns<1, COMP, true>(P, A.fl, nullptr, blk, T); break;
-        case 4: moments_columns<2, COMP, false>(P, A.fl, nullptr, blk, T); break;
-        case 5: moments_columns<2, COMP, true>(P, A.fl, nullptr, blk, T); break;
-        case 8: moments_columns<4, COMP, false>(P, A.fl, nullptr, blk, T); break;
-        default: moments_columns<4, COMP, true>(P, A.fl, nullptr, blk, T);
+        case 2: moments_columns<1, WCOL, COMP, false>(P, A.fl, nullptr, blk, T); break;
+        case 3: moments_columns<1, WCOL, COMP, true>(P, A.fl, nullptr, blk, T); break;
+        case 4: moments_columns<2, WCOL, COMP, false>(P, A.fl, nullptr, blk, T); break;
+        case 5: moments_columns<2, WCOL, COMP, true>(P, A.fl, nullptr, blk, T); break;
+        case 8: moments_columns<4, WCOL, COMP, false>(P, A.fl, nullptr, blk, T); break;
+        default: moments_columns<4, WCOL, COMP, true>(P, A.fl, nullptr, blk, T);
     }
 }
 
@@ -574,7 +575,17 @@ static int moments_patch(vx_ctx *ctx, const vx_patch *p, const vx_fields *fl, bo
         if ((rc = check_launch(ctx, "k_moment_table"))) return rc;
     }
     LaunchTimer lt(ctx, "k_moments");
+    // 8 columns a workgroup for tall columns: one consumer for more of them, and
+    // enough chunks for its start.  us, 8 / 4 columns, without and with a pulse: 8190
+    // x 1024 30.1 / 31.6, 53.5 / 46.5; 4096 x 2048 25.4 / 27.5, 45.8 / 47.3; 4096 x 4096
+    // 39.8 / 47.1, 84.0 / 90.8.
+    const bool tall = !comp && p->rtb == 1 && !p->nested && p->n_p >= 2048;
+    const int WCOL = tall ? MCOL_TALL : MCOL;
     const dim3 g((unsigned)((p->n_x + WCOL - 1) / WCOL)), b(64 * (comp ? WCOL : WCOL + 1));
+    if (tall) {
+        k_moments<1, false, false, MCOL_TALL><<<g, b, 0, ctx->stream>>>(A);
+        return check_launch(ctx, "k_moments");
+    }
     switch (p->rtb * 4 + (comp ? 2 : 0) + (p->nested ? 1 : 0)) {
         case 4: k_moments<1, false, false><<<g, b, 0, ctx->stream>>>(A); break;
         case 5: k_moments<1, false, true><<<g, b, 0, ctx->stream>>>(A); break;
@@ -619,13 +630,13 @@ int vx_moments_patches(vx_ctx *ctx, const vx_patch *patches, int32_t n, const vx
         } else {
             if (B.n == 0) B.start[0] = 0;
             B.p[B.n++] = mom_patch(p);
-            B.start[B.n] = B.start[B.n - 1] + (p.n_x + WCOL - 1) / WCOL;
+            B.start[B.n] = B.start[B.n - 1] + (p.n_x + MCOL - 1) / MCOL;
         }
         if (B.n == MOM_BATCH || (k == 0 && B.n > 0)) {
             B.fl = *fl;
             LaunchTimer lt(ctx, "k_moments");
-            if (compensated) k_moments_batch<true><<<(unsigned)B.start[B.n], 64 * WCOL, 0, ctx->stream>>>(B);
-            else k_moments_batch<false><<<(unsigned)B.start[B.n], 64 * (WCOL + 1), 0, ctx->stream>>>(B);
+            if (compensated) k_moments_batch<true><<<(unsigned)B.start[B.n], 64 * MCOL, 0, ctx->stream>>>(B);
+            else k_moments_batch<false><<<(unsigned)B.start[B.n], 64 * (MCOL + 1), 0, ctx->stream>>>(B);
             if ((rc = check_launch(ctx, "k_moments_batch"))) return rc;
             B.n = 0;
         }
