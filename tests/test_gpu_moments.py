@@ -113,6 +113,30 @@ class Case:
         self.L.vx_ctx_destroy(self.ctx)
 
 
+@pytest.mark.parametrize("comp", [False, True])
+@pytest.mark.parametrize("shape", [(37, 70, 1, False), (20, 2050, 1, False), (9, 130, 4, True), (16, 64, 2, False)])
+def test_whole_patch_writes_the_assembled_moments(shape, comp):
+    """0.0 + the patch's own moments, as the assembly forms them, in charge, J and the
+    species' charge; columns without particles give +0.0."""
+    c = Case([shape], "pulse")
+    L, n = c.L, shape[0] * shape[2]
+    L.vx_moments_whole.argtypes = [ctypes.c_void_p, ctypes.POINTER(Patch), ctypes.POINTER(Fields), ctypes.c_int] + \
+        [ctypes.c_void_p] * 3
+    c.p[0].planes[1] = c.put(np.where(np.arange(shape[0] + 4)[:, None] < 8, 0.0, 1.5)
+                             * np.ones((1, c.p[0].pitch))).value
+    q, j = c.one(0, comp)
+    assert np.signbit(q[0]) and q[0] == 0.0
+    out = [c.put(np.full(n, 7.0)) for _ in range(3)]
+    assert L.vx_moments_whole(c.ctx, ctypes.byref(c.p[0]), ctypes.byref(c.fl), comp, *out) == 0
+    for d, want in zip(out, (q, j, q)):
+        a = np.empty(n)
+        assert L.vx_memcpy_d2h(c.ctx, a.ctypes.data, d, a.nbytes) == 0
+        assert np.array_equal(a.view(np.int64), (0.0 + want).view(np.int64))
+    c.p[0].x_pos = 1
+    assert L.vx_moments_whole(c.ctx, ctypes.byref(c.p[0]), ctypes.byref(c.fl), comp, *out) != 0
+    c.free()
+
+
 def test_patches_of_different_heights_in_turn():
     """Two patches above the table's size with one A^2, the second short enough
     that its tables end inside the first one's entries: the first patch's moments

@@ -692,6 +692,12 @@ void EMFieldSolver::AssembleRhoAndJ() {
     for (auto &m : meshes)
         for (auto &l : m->levels)
             for (auto &r : l->rectangles) p.push_back(r->desc());
+    // one patch over the whole grid: its moments are the assembled ones
+    if (p.size() == 1 && meshes.size() == 1 && p[0].x_pos == 0 && p[0].n_x * p[0].rtb == fs.n_f) {
+        dev->check(vx_moments_whole(dev->ctx, p.data(), &fl, compensated_moments, fs.charge, fs.J, charges_species),
+                   "moments");
+        return;
+    }
     dev->check(vx_moments_patches(dev->ctx, p.data(), (int32_t)p.size(), &fl, compensated_moments), "moments");
     dev->check(vx_moments_assemble(dev->ctx, plan, fs.charge, fs.J, charges_species), "assemble");
 }

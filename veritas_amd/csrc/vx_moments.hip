@@ -43,6 +43,11 @@ struct MomPatch {
     double inv_rtb;       // 1.0 / relativeToBottom
     double dpq, jscale;   // dp*q and -q*q/mass
     double rel[3 * MAX_RTB];  // interpolatCoefsREL (Rectangle.cpp:103-110)
+    // A patch that is the whole assembly by itself: the assembly's 0.0 + (which
+    // makes -0.0 +0.0; -0.0 otherwise, which changes nothing) and the place of its
+    // species' charge (null otherwise)
+    double zero;
+    double *species;
 };
 
 struct MomArgs {
@@ -183,6 +188,12 @@ __device__ __forceinline__ double log_ratio(double a, double b) {
     const double R = vx_log_r(z);
     const double hfsq = 0.5 * f * f;
     return f - (hfsq - s * (hfsq + R));
+}
+
+__device__ __forceinline__ void put_charge(const MomPatch &P, long e, double v) {
+    v = P.zero + v;
+    P.chargeR[e] = v;
+    if (P.species) P.species[e] = v;
 }
 
 // COMP (mixed-precision form): no consumer; each producer keeps its lanes'
@@ -366,8 +377,8 @@ __device__ __forceinline__ void moments_columns(const MomPatch &P, const vx_fiel
                 wave_two_sum(aR[s], cR[s], sr, er);
                 wave_two_sum(aJ[s], cJ[s], sj, ej);
                 if (lane == 0 && col_ok) {
-                    P.chargeR[(long)i * RTB + s] = (sr + er) * P.dpq;
-                    P.currentR[(long)i * RTB + s] = (sj + ej) * P.jscale;
+                    put_charge(P, (long)i * RTB + s, (sr + er) * P.dpq);
+                    P.currentR[(long)i * RTB + s] = P.zero + (sj + ej) * P.jscale;
                 }
             }
         }
@@ -393,8 +404,8 @@ __device__ __forceinline__ void moments_columns(const MomPatch &P, const vx_fiel
         const int i = i0 + c / RTB;
         if (c < NCH && i < P.n_x) {
             const long e = (long)i * RTB + c % RTB;
-            if (lane < 32) P.chargeR[e] = acc * P.dpq;
-            else P.currentR[e] = acc * P.jscale;
+            if (lane < 32) put_charge(P, e, acc * P.dpq);
+            else P.currentR[e] = P.zero + acc * P.jscale;
         }
     }
 }
@@ -507,6 +518,8 @@ MomPatch mom_patch(const vx_patch &p) {
         M.rel[3 * i + 1] = (tl * tl + tl * tr + tr * tr) / 3.0 - (1.0 / 12);
         M.rel[3 * i + 2] = (tl * tl * tl + tl * tl * tr + tl * tr * tr + tr * tr * tr) * 0.25;
     }
+    M.zero = -0.0;
+    M.species = nullptr;
     return M;
 }
 
@@ -542,10 +555,16 @@ static int moments_check(vx_ctx *ctx, const vx_patch *p, const vx_fields *fl) {
     return VX_OK;
 }
 
-static int moments_patch(vx_ctx *ctx, const vx_patch *p, const vx_fields *fl, bool comp) {
+// species: where the patch's moments are the assembled ones, the place of its
+// species' charge.
+static int moments_patch(vx_ctx *ctx, const vx_patch *p, const vx_fields *fl, bool comp, double *species = nullptr) {
     int rc = moments_check(ctx, p, fl);
     if (rc) return rc;
     MomArgs A{mom_patch(*p), *fl, nullptr};
+    if (species) {
+        A.p.zero = 0.0;
+        A.p.species = species;
+    }
     // The table saves each column its logarithms but costs a launch (3.1 us).
     // us with / without it: 1024 x 512 at rtb 1 8.3 / 7.0, 1024 x 1024 11.9 / 10.7,
     // 2048 x 1024 12.1 / 15.4; 2000 x 64 at rtb 4 7.8 / 6.1, 512 x 512 11.4 / 12.4,
@@ -611,6 +630,19 @@ int vx_moments_patch(vx_ctx *ctx, const vx_patch *p, const vx_fields *fl) {
 
 int vx_moments_patch_compensated(vx_ctx *ctx, const vx_patch *p, const vx_fields *fl) {
     return moments_patch(ctx, p, fl, true);
+}
+
+int vx_moments_whole(vx_ctx *ctx, const vx_patch *p, const vx_fields *fl, int compensated, double *charge, double *J,
+                     double *charges_species) {
+    int rc = moments_check(ctx, p, fl);
+    if (rc) return rc;
+    if (!charge || !J || !charges_species) return fail(ctx, VX_EINVAL, "moments: null output");
+    if (p->x_pos != 0 || p->n_x * p->rtb != fl->n_f)
+        return fail(ctx, VX_EINVAL, "moments: the patch does not cover the %d finest cells", fl->n_f);
+    vx_patch w = *p;
+    w.chargeR = charge;
+    w.currentR = J;
+    return moments_patch(ctx, &w, fl, compensated != 0, charges_species);
 }
 
 int vx_moments_patches(vx_ctx *ctx, const vx_patch *patches, int32_t n, const vx_fields *fl, int compensated) {
