@@ -1,7 +1,7 @@
 // CPU ORACLE -- test infrastructure only.
 //
 // A plain FP64 restatement of the reference's Vlasov-Maxwell time advance
-// (Libbum/Veritas).  It is the checker for the GPU framework: only tests/,
+// (Libbum/Veritas).  It is what the GPU framework is compared with: only tests/,
 // __graft_entry__.smoke() and bench.py's CPU-baseline leg may load it, and
 // never as the thing that is measured or shipped.
 //

@@ -1,11 +1,11 @@
 """The p-moments (k_moments) against the oracle, bit for bit: column counts that
 leave a partial workgroup, p-columns that end inside, at and just past a 64-cell
-chunk, tall columns (8 a workgroup from 2048 p-cells on), patches with and without the
-logarithm table (above 2^20 cells), with and
-without nested cells (levels 3: relativeToBottom 1, 2 and 4), behind and ahead
-of a pulse.  The compensated sums agree with the ordered ones.  A table of
-another patch is never taken for this one's, and several patches in one launch
-give each one's bits."""
+chunk, tall columns (8 a workgroup from 2048 p-cells on), patches with and
+without the logarithm table (above 2^20 cells), with and without nested cells
+(levels 3: relativeToBottom 1, 2 and 4), behind and ahead of a pulse.  The
+compensated sums agree with the ordered ones.  A table of another patch is never
+taken for this one's, several patches in one launch give each one's bits, and a
+patch that is the whole grid writes what the assembly would."""
 import ctypes
 
 import numpy as np

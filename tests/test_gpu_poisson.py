@@ -1,8 +1,9 @@
 """vx_poisson at the edges of its forms (wavefronts, entries a thread, sub-chunks
-of 64, chunks of 192 and 512, the solvers' borders at 4096 and 36864), through the C ABI, against the
-oracle's solve of the same right-hand side: both converge to the correctly
-rounded solution (a near-tie may differ by 1 ulp), E and Ex0 follow from phi.
-Smooth, random and zero charges; a second call repeats the first's bits."""
+of 64, chunks of 192 and 512, the solvers' borders at 4096 and 36864), through
+the C ABI, against the oracle's solve of the same right-hand side: both converge
+to the correctly rounded solution (a near-tie may differ by 1 ulp), E and Ex0
+follow from phi.  Smooth, random and zero charges; a second call repeats the
+first's bits."""
 import ctypes
 
 import numpy as np

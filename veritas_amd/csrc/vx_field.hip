@@ -80,8 +80,9 @@ __device__ __forceinline__ void dd_sub(double &sh, double &sl, double a, double 
 }
 
 // ------------------------------------------------ multi-workgroup solve, n_f > 4096
-// Workgroup b owns the chunk of 64 MW consecutive entries [64 MW b, 64 MW (b +
-// 1)), wavefront w of it the sub-chunk w of 64 entries.  One approximate solve of A c = v and the residual of the next round are one launch:
+// Workgroup b owns the chunk of 64 MW consecutive entries from 64 MW b on,
+// wavefront w of it the sub-chunk w of 64 entries.  One approximate solve of
+// A c = v and the residual of the next round are one launch:
 //   S_i = sum_{k<i} v'_k with v'_0 = -tail, tail = sum_{k>=1} v_k,
 //   d0 = mean(S), D_i = d0 - S_i (D_0 = 0), y_i = sum_{k<=i} D_k,
 //   c = M^-1 y - (M^-1 y)_0 with c_0 from row 0, x (+)= c, then either the
