@@ -87,7 +87,7 @@ struct Sub0Tiles {
 // it writes.
 // Measured (three patches of 5.6 M cells, MI355X): stages 0..5 145, 184, 197,
 // 215, 278, 179 us with both sides' WENO parts formed per face, scaled
-// divisions and A^2 read behind the plane loads; 92, 130, 150, 174, 252, 110 us
+// divisions and A^2 read behind the plane loads; 95, 114, 138, 161, 244, 109 us
 // now.  Bound by FP64 issue at stages 0-2 and 5, by the stored planes (120 and
 // 136 B a position, 154 us at the copy rate for stage 4) at 3 and 4.
 // IN: every reference loop-range test holds for every lane and march row
@@ -390,7 +390,10 @@ __device__ __forceinline__ void lo_predictor(const vx_patch &P, double aSum, int
 // Bound by memory: 72 B a position with COR, 82 us at the copy rate for three
 // patches of 5.6 M cells, measured 104 us (116 before the loads were free of
 // branches, the extrema of f^n and f^td shared between neighbours and the
-// ratios divided only where one is below 1).
+// ratios divided only where one is below 1).  With COR R and C are stored past
+// the caches: the launch itself takes as long, but the next stages find f and
+// the fluxes there (sub-step 0 at stages 1..4 129, 150, 177, 251 -> 114, 138, 161,
+// 244 us; streaming the loads of f^td and the fluxes too gave nothing).
 constexpr int LIMW = 56;  // positions per limiter wavefront (7 x 64 bytes)
 
 struct LimTiles {
@@ -476,8 +479,7 @@ __device__ __forceinline__ void limiter_stream(const vx_patch &P, const LimTiles
             const long idx = pidx(pitch, i, j);
             if (own && i < i1 && i >= -1 && i < nx + 1 && r_j) {
                 // only the cross-patch C sync reads R again (at patch edges):
-                // streamed past the caches, which keep C and the fluxes that
-                // the corrector reads next
+                // streamed past the caches, which keep what the next launches read
                 __builtin_nontemporal_store(rp, &P.Rp[idx]);
                 __builtin_nontemporal_store(rm, &P.Rm[idx]);
             }
@@ -488,8 +490,13 @@ __device__ __forceinline__ void limiter_stream(const vx_patch &P, const LimTiles
                 cp = p_c > 0.0 ? valmin(rp, Rm_l) : valmin(Rp_l, rm);
             }
             if (own && i < i1) {
-                P.Cx[idx] = cx;
-                P.Cp[idx] = cp;
+                if (COR) {  // only the C sync and its corrections read C again
+                    __builtin_nontemporal_store(cx, &P.Cx[idx]);
+                    __builtin_nontemporal_store(cp, &P.Cp[idx]);
+                } else {
+                    P.Cx[idx] = cx;
+                    P.Cp[idx] = cp;
+                }
             }
         }
         if (COR) {
