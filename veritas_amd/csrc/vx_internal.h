@@ -108,9 +108,12 @@ inline int fail(vx_ctx *ctx, int code, const char *fmt, ...) {
     return code;
 }
 
+// (a refused call's error is taken from the runtime too, or the next launch's
+// check would report it)
 inline int check_hip(vx_ctx *ctx, hipError_t e, const char *what) {
-    if (e != hipSuccess) return fail(ctx, VX_EHIP, "%s: %s", what, hipGetErrorString(e));
-    return VX_OK;
+    if (e == hipSuccess) return VX_OK;
+    (void)hipGetLastError();
+    return fail(ctx, VX_EHIP, "%s: %s", what, hipGetErrorString(e));
 }
 
 inline int check_launch(vx_ctx *ctx, const char *what) {

@@ -122,6 +122,25 @@ int vx_stage_init(vx_ctx *ctx) {
     return rc;
 }
 
+// Whether the staging kernels may copy n doubles at dev: they lie inside one
+// allocation of the context's device.  Whatever else a caller passes (null, a
+// count past the allocation, another device's memory) goes to HIP's own copy,
+// which refuses it or knows how to reach it; a kernel would fault on it.
+static bool staged_dev(const vx_ctx *ctx, const double *dev, size_t n) {
+    if (!dev || (uintptr_t)dev % sizeof(double) != 0) return false;
+    hipPointerAttribute_t at;
+    hipDeviceptr_t base = nullptr;
+    size_t size = 0;
+    if (hipPointerGetAttributes(&at, dev) != hipSuccess ||
+        hipMemGetAddressRange(&base, &size, (hipDeviceptr_t)dev) != hipSuccess) {
+        (void)hipGetLastError();  // (an address that HIP does not know)
+        return false;
+    }
+    const size_t off = (size_t)((const char *)dev - (const char *)base);
+    return at.type == hipMemoryTypeDevice && at.device == ctx->device && off <= size &&
+           n <= (size - off) / sizeof(double);
+}
+
 // h rows of w doubles between a pitched device array and pageable host memory,
 // through the context's two pinned buffers: a kernel packs one (or unpacks it)
 // over the link while the host copies the other.  hipMemcpy2DAsync on pageable
@@ -165,7 +184,7 @@ static int staged_rows(vx_ctx *ctx, double *dev, size_t pitch, double *host, siz
 static int host_copy(vx_ctx *ctx, void *dev, void *host, size_t bytes, bool up, const char *what) {
     if (bytes == 0) return vx_sync(ctx);
     constexpr size_t W = 1024;  // doubles a "row" of a contiguous array
-    if (bytes % sizeof(double) == 0 && (uintptr_t)dev % sizeof(double) == 0) {
+    if (bytes % sizeof(double) == 0 && host && staged_dev(ctx, (const double *)dev, bytes / sizeof(double))) {
         const size_t n = bytes / sizeof(double), h = n / W, rest = n % W;
         double *d = (double *)dev, *p = (double *)host;
         int rc = h ? staged_rows(ctx, d, W, p, W, h, up, what) : VX_OK;
@@ -345,7 +364,10 @@ static int patch_copy(vx_ctx *ctx, const vx_patch *p, int slot, int ghosts, doub
     const size_t w = (size_t)(p->n_p + 2 * ghosts), h = (size_t)(p->n_x + 2 * ghosts);
     double *dev = p->f[slot] + (size_t)(2 - ghosts) * p->pitch + (2 - ghosts);
     const char *what = up ? "patch upload" : "patch download";
-    if (w * sizeof(double) <= vx_ctx::STAGE_BYTES) return staged_rows(ctx, dev, p->pitch, host, w, h, up, what);
+    // (a shape without rows, or with rows that lap over each other, is HIP's to refuse too)
+    const bool rows = p->n_x + 2 * ghosts > 0 && w <= (size_t)p->pitch && w * sizeof(double) <= vx_ctx::STAGE_BYTES;
+    if (rows && staged_dev(ctx, dev, (h - 1) * p->pitch + w))
+        return staged_rows(ctx, dev, p->pitch, host, w, h, up, what);
     hipError_t e = up ? hipMemcpy2DAsync(dev, sizeof(double) * p->pitch, host, sizeof(double) * w,
                                          sizeof(double) * w, h, hipMemcpyHostToDevice, ctx->stream)
                       : hipMemcpy2DAsync(host, sizeof(double) * w, dev, sizeof(double) * p->pitch,
