@@ -1,6 +1,7 @@
 """Copies that reach outside what they may touch: HIP's own copies refuse a null
 address and a count past the allocation, and so do the copies through the
-pinned buffers, with VX_EHIP and nothing written."""
+pinned buffers, with VX_EHIP and nothing written.  A shape without cells copies
+nothing."""
 import ctypes
 
 import numpy as np
@@ -51,4 +52,15 @@ def test_patch_copies_stay_inside_the_allocation(lib, block, nx, np_, pitch):
     h = np.full((nx + 4) * (np_ + 4), -1.0)
     assert L.vx_patch_upload(ctx, ctypes.byref(p), 0, 2, h.ctypes.data) == VX_EHIP
     assert L.vx_patch_download(ctx, ctypes.byref(p), 0, 2, h.ctypes.data) == VX_EHIP
+    assert (h == -1.0).all()
+
+
+@pytest.mark.parametrize("nx,np_,g", [(4, 0, 0), (0, 4, 0), (0, 0, 0), (4, -2, 1), (-4, 4, 2)])
+def test_an_empty_patch_copies_nothing(lib, block, nx, np_, g):
+    L, ctx = lib
+    p = Patch(n_x=nx, n_p=np_, rtb=1, pitch=8)
+    p.planes[0] = block
+    h = np.full(64, -1.0)
+    assert L.vx_patch_upload(ctx, ctypes.byref(p), 0, g, h.ctypes.data) == 0
+    assert L.vx_patch_download(ctx, ctypes.byref(p), 0, g, h.ctypes.data) == 0
     assert (h == -1.0).all()

@@ -364,8 +364,8 @@ static int patch_copy(vx_ctx *ctx, const vx_patch *p, int slot, int ghosts, doub
     const size_t w = (size_t)(p->n_p + 2 * ghosts), h = (size_t)(p->n_x + 2 * ghosts);
     double *dev = p->f[slot] + (size_t)(2 - ghosts) * p->pitch + (2 - ghosts);
     const char *what = up ? "patch upload" : "patch download";
-    // (a shape without rows, or with rows that lap over each other, is HIP's to refuse too)
-    const bool rows = p->n_x + 2 * ghosts > 0 && w <= (size_t)p->pitch && w * sizeof(double) <= vx_ctx::STAGE_BYTES;
+    // (an empty shape copies nothing, rows that lap over each other are HIP's to refuse too)
+    const bool rows = p->n_x + 2 * ghosts > 0 && w > 0 && w <= (size_t)p->pitch && w * sizeof(double) <= vx_ctx::STAGE_BYTES;
     if (rows && staged_dev(ctx, dev, (h - 1) * p->pitch + w))
         return staged_rows(ctx, dev, p->pitch, host, w, h, up, what);
     hipError_t e = up ? hipMemcpy2DAsync(dev, sizeof(double) * p->pitch, host, sizeof(double) * w,
