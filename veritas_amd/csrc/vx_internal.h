@@ -6,6 +6,7 @@
 #include <cstdarg>
 #include <cstdio>
 #include <array>
+#include <mutex>
 #include <string>
 #include <unordered_map>
 #include <vector>
@@ -51,7 +52,9 @@ struct vx_ctx {
     hipEvent_t ring_ev[RING] = {};
     bool ring_pending[RING] = {};
     int ring_next = 0;
-    // two pinned buffers of the copies to and from pageable host memory
+    // two pinned buffers of the copies to and from pageable host memory, held by
+    // one thread's copy at a time
+    std::mutex stage_mu;
     static constexpr size_t STAGE_BYTES = (size_t)2 << 20;
     double *stage = nullptr;
     hipEvent_t stage_ev[2] = {};
@@ -59,7 +62,7 @@ struct vx_ctx {
 
 // vx_field.hip: looks up this device's fixed work array (ctx->device current)
 int vx_noalloc_scratch_init(vx_ctx *ctx);
-// vx_runtime.hip: makes sure that ctx->stage is there
+// vx_runtime.hip: makes sure that ctx->stage is there (with ctx->stage_mu held)
 int vx_stage_init(vx_ctx *ctx);
 
 struct vx_graph {

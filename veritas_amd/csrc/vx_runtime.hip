@@ -109,9 +109,19 @@ __global__ __launch_bounds__(256) void k_rows_in(double *dev, const double *host
     if (e < n) dev[(e / w) * pitch + e % w] = host[e];
 }
 
-// The pinned buffers, allocated on first use (40 us).
+// The pinned buffers, allocated on first use (40 us), with their events on the
+// context's device, whichever device the calling thread has current.
 int vx_stage_init(vx_ctx *ctx) {
     if (ctx->stage) return VX_OK;
+    struct Device {
+        int was = -1;
+        explicit Device(int d) {
+            if (hipGetDevice(&was) != hipSuccess || was == d || hipSetDevice(d) != hipSuccess) was = -1;
+        }
+        ~Device() {
+            if (was >= 0) (void)hipSetDevice(was);
+        }
+    } device(ctx->device);
     void *p = nullptr;
     int rc = check_hip(ctx, hipHostMalloc(&p, 2 * vx_ctx::STAGE_BYTES), "pinned staging");
     if (rc) return rc;
@@ -146,9 +156,11 @@ static bool staged_dev(const vx_ctx *ctx, const double *dev, size_t n) {
 // over the link while the host copies the other.  hipMemcpy2DAsync on pageable
 // memory goes row by row: 64 x 256 doubles 490 us, 1024 x 1024 8.7 ms, 4096 x
 // 4096 54 ms on an MI355X; these 16 us, 0.17 ms and 2.7 ms.  Waits for the copy.
+// Threads that copy at once on one context take the buffers in turn.
 static int staged_rows(vx_ctx *ctx, double *dev, size_t pitch, double *host, size_t w, size_t h, bool up,
                        const char *what) {
     constexpr size_t BUF = vx_ctx::STAGE_BYTES / sizeof(double);
+    std::lock_guard<std::mutex> lock(ctx->stage_mu);
     int rc = vx_stage_init(ctx);
     if (rc) return rc;
     const size_t rows = BUF / w;  // (the caller checked w <= BUF)
