@@ -1,5 +1,7 @@
 """Threads that copy to and from the device on one context at once, each its own
-arrays: every thread gets its own values, whole."""
+arrays: every thread gets its own values, whole.  The CFL bound, whose maxima come
+through the same pinned buffers, is the same beside copies, and it refuses field
+arrays that it cannot read."""
 import ctypes
 import threading
 
@@ -7,6 +9,7 @@ import numpy as np
 import pytest
 
 from test_gpu_staged_copies import P, Patch, lib
+from test_zz_no_alloc import D, FieldState, State
 
 pytestmark = pytest.mark.gpu
 
@@ -56,3 +59,53 @@ def test_threads_copy_patches_and_arrays_of_one_context(lib, nx, np_):
     together(4, work)
     for d in dev:
         L.vx_free(ctx, d)
+
+
+def bound(L, ctx, fs):
+    """vx_cfl_bound of one electron species: (return code, bound)."""
+    L.vx_cfl_bound.argtypes = [P, ctypes.POINTER(FieldState), ctypes.c_int] + [ctypes.POINTER(D)] * 4
+    q, m, dp, out = D(-1.60217657e-19), D(9.10938291e-31), D(1e-24), D(-1.0)
+    rc = L.vx_cfl_bound(ctx, ctypes.byref(fs), 1, ctypes.byref(q), ctypes.byref(m), ctypes.byref(dp), ctypes.byref(out))
+    return rc, out.value
+
+
+@pytest.fixture
+def fields(lib):
+    L, ctx = lib
+    s = State(L, ctx, 3000, np.zeros(3000), np.zeros(3000), 0.0, work=False)
+    rng = np.random.default_rng(5)
+    for name, amp in (("Ay", 1e-3), ("Az", 1e-3), ("By", 1e4), ("Bz", 1e4), ("E", 1e12)):
+        s.put(name, amp * rng.standard_normal(3000))
+    yield s
+    s.free()
+
+
+def test_the_cfl_bound_beside_copies_of_the_same_context(lib, fields):
+    L, ctx = lib
+    rc, want = bound(L, ctx, fields.fs)
+    assert rc == 0 and want > 0
+    a = np.full(200_000, 1e300)  # (a bound from these values would be 0)
+    d = P()
+    assert L.vx_malloc(ctx, a.nbytes, ctypes.byref(d)) == 0
+
+    def work(k):
+        got = np.empty_like(a)
+        for _ in range(20):
+            if k == 0:
+                assert bound(L, ctx, fields.fs) == (0, want)
+            else:
+                assert L.vx_memcpy_h2d(ctx, d, a.ctypes.data, a.nbytes) == 0
+                assert L.vx_memcpy_d2h(ctx, got.ctypes.data, d, a.nbytes) == 0
+                assert np.array_equal(got, a)
+    together(2, work)
+    L.vx_free(ctx, d)
+
+
+@pytest.mark.parametrize("name", ["Ay", "Az", "By", "Bz", "E"])
+def test_the_cfl_bound_refuses_arrays_that_are_not_there(lib, fields, name):
+    L, ctx = lib
+    was = getattr(fields.fs, name)
+    setattr(fields.fs, name, None)
+    assert bound(L, ctx, fields.fs) == (-2, -1.0)
+    setattr(fields.fs, name, was)
+    assert bound(L, ctx, fields.fs)[0] == 0

@@ -64,6 +64,7 @@ struct vx_ctx {
 int vx_noalloc_scratch_init(vx_ctx *ctx);
 // vx_runtime.hip: makes sure that ctx->stage is there (with ctx->stage_mu held)
 int vx_stage_init(vx_ctx *ctx);
+bool vx_device_range(const vx_ctx *ctx, const double *dev, size_t n);
 
 struct vx_graph {
     hipGraphExec_t exec = nullptr;

@@ -132,11 +132,11 @@ int vx_stage_init(vx_ctx *ctx) {
     return rc;
 }
 
-// Whether the staging kernels may copy n doubles at dev: they lie inside one
-// allocation of the context's device.  Whatever else a caller passes (null, a
+// Whether n doubles at dev lie inside one allocation of the context's device, so
+// that a kernel may read and write them.  Whatever else a caller passes (null, a
 // count past the allocation, another device's memory) goes to HIP's own copy,
 // which refuses it or knows how to reach it; a kernel would fault on it.
-static bool staged_dev(const vx_ctx *ctx, const double *dev, size_t n) {
+bool vx_device_range(const vx_ctx *ctx, const double *dev, size_t n) {
     if (!dev || (uintptr_t)dev % sizeof(double) != 0) return false;
     hipPointerAttribute_t at;
     hipDeviceptr_t base = nullptr;
@@ -196,7 +196,7 @@ static int staged_rows(vx_ctx *ctx, double *dev, size_t pitch, double *host, siz
 static int host_copy(vx_ctx *ctx, void *dev, void *host, size_t bytes, bool up, const char *what) {
     if (bytes == 0) return vx_sync(ctx);
     constexpr size_t W = 1024;  // doubles a "row" of a contiguous array
-    if (bytes % sizeof(double) == 0 && host && staged_dev(ctx, (const double *)dev, bytes / sizeof(double))) {
+    if (bytes % sizeof(double) == 0 && host && vx_device_range(ctx, (const double *)dev, bytes / sizeof(double))) {
         const size_t n = bytes / sizeof(double), h = n / W, rest = n % W;
         double *d = (double *)dev, *p = (double *)host;
         int rc = h ? staged_rows(ctx, d, W, p, W, h, up, what) : VX_OK;
@@ -378,7 +378,7 @@ static int patch_copy(vx_ctx *ctx, const vx_patch *p, int slot, int ghosts, doub
     const char *what = up ? "patch upload" : "patch download";
     // (an empty shape copies nothing, rows that lap over each other are HIP's to refuse too)
     const bool rows = p->n_x + 2 * ghosts > 0 && w > 0 && w <= (size_t)p->pitch && w * sizeof(double) <= vx_ctx::STAGE_BYTES;
-    if (rows && staged_dev(ctx, dev, (h - 1) * p->pitch + w))
+    if (rows && vx_device_range(ctx, dev, (h - 1) * p->pitch + w))
         return staged_rows(ctx, dev, p->pitch, host, w, h, up, what);
     hipError_t e = up ? hipMemcpy2DAsync(dev, sizeof(double) * p->pitch, host, sizeof(double) * w,
                                          sizeof(double) * w, h, hipMemcpyHostToDevice, ctx->stream)
