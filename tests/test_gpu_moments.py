@@ -4,7 +4,7 @@ chunk, tall columns (8 a workgroup from 2048 p-cells on), patches with and
 without the logarithm table (above 2^20 cells), with and without nested cells
 (levels 3: relativeToBottom 1, 2 and 4), behind and ahead of a pulse.  The
 compensated sums agree with the ordered ones.  A table of another patch is never
-taken for this one's, several patches in one launch give each one's bits, and a
+taken for this one's, a recorded launch keeps its own, several patches in one launch give each one's bits, and a
 patch that is the whole grid writes what the assembly would."""
 import ctypes
 
@@ -166,4 +166,34 @@ def test_patches_together_match_each_alone(a, comp):
             for x, y in zip(c.get(k), alone[k]):
                 assert np.array_equal(x, y if k < m else 0.0 * y), (k, m)
     assert all(np.abs(y).max() > 0 for r in alone for y in r)
+    c.free()
+
+
+def test_a_recorded_launch_outlives_its_logarithm_table():
+    """A graph recorded with one table, replayed after a taller patch of the same
+    context needed a larger one, between eager calls of both."""
+    c = Case([(1030, 1030, 1, False), (300, 4100, 1, False), (200, 8200, 1, False)], "uniform")
+    L = c.L
+    L.vx_graph_begin.argtypes, L.vx_graph_destroy.argtypes = [ctypes.c_void_p], [ctypes.c_void_p]
+    L.vx_graph_end.argtypes = [ctypes.c_void_p, ctypes.POINTER(ctypes.c_void_p)]
+    L.vx_graph_launch.argtypes = [ctypes.c_void_p, ctypes.c_void_p]
+    want, g = c.one(0), ctypes.c_void_p()
+    assert L.vx_graph_begin(c.ctx) == 0
+    assert L.vx_moments_patch(c.ctx, ctypes.byref(c.p[0]), ctypes.byref(c.fl)) == 0
+    assert L.vx_graph_end(c.ctx, ctypes.byref(g)) == 0
+    tall = {}
+    for k in (1, 1, 2, 1, 2, 0):
+        got = c.one(k)
+        assert np.array_equal(got, tall.setdefault(k, got))
+        assert L.vx_graph_launch(c.ctx, g) == 0
+        assert np.array_equal(c.get(0), want)
+        # memory taken now, which a freed table's place would serve, keeps its values
+        q = np.full(4096, 3.0)
+        d, back = c.put(q), np.empty(4096)
+        assert L.vx_graph_launch(c.ctx, g) == 0
+        assert np.array_equal(c.get(0), want)
+        assert L.vx_memcpy_d2h(c.ctx, back.ctypes.data, d, back.nbytes) == 0
+        assert np.array_equal(back, q)
+    assert np.array_equal(tall[0], want) and np.abs(want).min() > 0
+    L.vx_graph_destroy(g)
     c.free()

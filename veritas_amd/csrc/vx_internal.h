@@ -26,6 +26,7 @@ struct vx_ctx {
     // p-moment logarithm table of the patch being reduced (vx_moments_patch)
     double *mom_table = nullptr;
     size_t mom_table_n = 0;
+    std::vector<double *> mom_old;  // smaller ones before it, which recorded graphs may hold
     // strip heights of the fused stage chosen per patch shape and stage:
     // {n_x, n_p, rows, mixed, stage}
     std::vector<std::array<int, 5>> ti_cache;

@@ -572,17 +572,24 @@ static int moments_patch(vx_ctx *ctx, const vx_patch *p, const vx_fields *fl, bo
     // 4 21.1 / 19.1).  A wavefront that forms the terms for its workgroup's columns
     // instead: 9.2 at 1024 x 1024, but 52 at 4096 x 4096, 46 with the table.
     if ((long)p->n_x * p->n_p > TAB_CELLS) {
-        const size_t need = (size_t)tab_entries(2, p->n_p);
+        size_t need = (size_t)tab_entries(2, p->n_p);
         if (ctx->mom_table_n < need) {
             if (ctx->capturing) return fail(ctx, VX_EINVAL, "moments: table growth while a step graph is recorded");
-            if (ctx->mom_table) (void)hipFree(ctx->mom_table);
-            ctx->mom_table = nullptr;
-            ctx->mom_table_n = 0;
-            if (hipMalloc(&ctx->mom_table, sizeof(double) * need) != hipSuccess)
+            // The outgrown table stays until the context ends: a graph recorded
+            // with it writes and reads it when it is replayed.  Each table has at
+            // least twice the entries of the one before, so that all of them
+            // together are less than two of the largest.
+            need = std::max(need, 2 * ctx->mom_table_n);
+            double *table = nullptr;
+            if (hipMalloc(&table, sizeof(double) * need) != hipSuccess)
                 return fail(ctx, VX_ENOMEM, "moments: logarithm table");
             // no table in place yet (flag 0)
-            if (hipMemsetAsync(ctx->mom_table, 0, sizeof(double) * need, ctx->stream) != hipSuccess)
+            if (hipMemsetAsync(table, 0, sizeof(double) * need, ctx->stream) != hipSuccess) {
+                (void)hipFree(table);
                 return fail(ctx, VX_EHIP, "moments: logarithm table clear");
+            }
+            if (ctx->mom_table) ctx->mom_old.push_back(ctx->mom_table);
+            ctx->mom_table = table;
             ctx->mom_table_n = need;
         }
         A.tab = ctx->mom_table;

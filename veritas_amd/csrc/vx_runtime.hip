@@ -42,6 +42,7 @@ void vx_ctx_destroy(vx_ctx *ctx) {
         if (e) (void)hipEventDestroy(e);
     for (auto &e : ctx->tev) (void)hipEventDestroy(e);
     if (ctx->mom_table) (void)hipFree(ctx->mom_table);
+    for (double *t : ctx->mom_old) (void)hipFree(t);
     if (ctx->batch_ring && ctx->batch_ring_free) ctx->batch_ring_free(ctx->batch_ring);
     if (ctx->xev) (void)hipEventDestroy(ctx->xev);
     if (ctx->cfl_ev) (void)hipEventDestroy(ctx->cfl_ev);
