@@ -702,7 +702,7 @@ int table_rebuild(vx_ctx *ctx, vx_patch_table *t) {
 
 // The strip policies of a table's batched flux (kind 0) and limiter (kind 1)
 // launches, chosen by timing on the table's first launch of each kind: every
-// candidate policy runs the launch three times (the launches are idempotent:
+// candidate policy runs the launch three times (the launches timed are idempotent:
 // they read f, the stored fluxes of earlier stages and f^n, and write only
 // their own outputs, the same values under any policy), the fastest is kept
 // (a later candidate must be 3 % faster), and the choice is kept per device
@@ -839,7 +839,8 @@ int sub0_fluxes_table(vx_ctx *ctx, vx_patch_table *t, int step, double dt, const
     A.step = step;
     rk_coefficients(step, dt, A.a, A.ns, A.aSum);
     for (int k = 0; k < 6; k++) A.b5[k] = vx::rk_a[5][k] * dt;  // as stage 5 forms its a[k]
-    if (!t->sub0_tuned[mp] && !ctx->capturing) {
+    // (not timed on stage 5, which writes its fluxes over the partial sum it reads)
+    if (!t->sub0_tuned[mp] && !ctx->capturing && step < 5) {
         rc = tune_policy(ctx, t, 0, mp, {-2048, 128, 64, 32, 16, 8}, [&] {
             if (mp) launch_sub0s_batch<true>(ctx, t, step, A);
             else launch_sub0s_batch<false>(ctx, t, step, A);
