@@ -180,8 +180,8 @@ int vx_moments_patch_compensated(vx_ctx *ctx, const vx_patch *p, const vx_fields
  * compensated or not, with as few launches as their sizes allow. */
 int vx_moments_patches(vx_ctx *ctx, const vx_patch *patches, int32_t n, const vx_fields *fl, int compensated);
 /* The moments of the only patch of a run (x_pos 0, n_x * rtb = n_f), written as
- * vx_moments_assemble would: charge, J and its species' charge, n_f each.  The
- * patch's own chargeR and currentR are not written. */
+ * vx_moments_assemble would: charge, J and its species' charge, n_f each; its own
+ * chargeR and currentR are written too (if they are not null). */
 int vx_moments_whole(vx_ctx *ctx, const vx_patch *p, const vx_fields *fl, int compensated, double *charge, double *J,
                      double *charges_species);
 /* Rectangle::CalculateEnergy (Rectangle.cpp:284-305): energyR[j * rtb + k]

@@ -197,3 +197,21 @@ def test_a_recorded_launch_outlives_its_logarithm_table():
     assert np.array_equal(tall[0], want) and np.abs(want).min() > 0
     L.vx_graph_destroy(g)
     c.free()
+
+
+@pytest.mark.parametrize("comp", [False, True])
+@pytest.mark.parametrize("shape", [(37, 70, 1, False), (20, 2050, 1, False), (9, 130, 4, True)])
+def test_whole_patch_keeps_its_own_moments(shape, comp):
+    """The patch's chargeR and currentR after the call that assembles them: those of
+    the patch's own call; a patch without them is accepted."""
+    c = Case([shape], "pulse")
+    c.L.vx_moments_whole.argtypes = [ctypes.c_void_p, ctypes.POINTER(Patch), ctypes.POINTER(Fields), ctypes.c_int] + \
+        [ctypes.c_void_p] * 3
+    want, out = c.one(0, comp), [c.put(np.zeros(shape[0] * shape[2])) for _ in range(3)]
+    args = c.ctx, ctypes.byref(c.p[0]), ctypes.byref(c.fl), comp, *out
+    assert c.L.vx_moments_whole(*args) == 0
+    for got, ref in zip(c.get(0), want):
+        assert np.array_equal(got, ref) and np.abs(ref).max() > 0
+    c.p[0].planes[24] = c.p[0].planes[25] = None
+    assert c.L.vx_moments_whole(*args) == 0
+    c.free()

@@ -43,11 +43,10 @@ struct MomPatch {
     double inv_rtb;       // 1.0 / relativeToBottom
     double dpq, jscale;   // dp*q and -q*q/mass
     double rel[3 * MAX_RTB];  // interpolatCoefsREL (Rectangle.cpp:103-110)
-    // A patch that is the whole assembly by itself: the assembly's 0.0 + (which
-    // makes -0.0 +0.0; -0.0 otherwise, which changes nothing) and the place of its
-    // species' charge (null otherwise)
-    double zero;
-    double *species;
+    // A patch that is the whole assembly by itself: the places of the assembled
+    // charge, current and species' charge (null otherwise), each 0.0 + the patch's
+    // (the assembly's sum, which makes -0.0 +0.0)
+    double *charge, *J, *species;
 };
 
 struct MomArgs {
@@ -191,9 +190,12 @@ __device__ __forceinline__ double log_ratio(double a, double b) {
 }
 
 __device__ __forceinline__ void put_charge(const MomPatch &P, long e, double v) {
-    v = P.zero + v;
-    P.chargeR[e] = v;
-    if (P.species) P.species[e] = v;
+    if (P.chargeR) P.chargeR[e] = v;
+    if (P.charge) P.charge[e] = P.species[e] = 0.0 + v;
+}
+__device__ __forceinline__ void put_current(const MomPatch &P, long e, double v) {
+    if (P.currentR) P.currentR[e] = v;
+    if (P.J) P.J[e] = 0.0 + v;
 }
 
 // COMP (mixed-precision form): no consumer; each producer keeps its lanes'
@@ -378,7 +380,7 @@ __device__ __forceinline__ void moments_columns(const MomPatch &P, const vx_fiel
                 wave_two_sum(aJ[s], cJ[s], sj, ej);
                 if (lane == 0 && col_ok) {
                     put_charge(P, (long)i * RTB + s, (sr + er) * P.dpq);
-                    P.currentR[(long)i * RTB + s] = P.zero + (sj + ej) * P.jscale;
+                    put_current(P, (long)i * RTB + s, (sj + ej) * P.jscale);
                 }
             }
         }
@@ -405,7 +407,7 @@ __device__ __forceinline__ void moments_columns(const MomPatch &P, const vx_fiel
         if (c < NCH && i < P.n_x) {
             const long e = (long)i * RTB + c % RTB;
             if (lane < 32) put_charge(P, e, acc * P.dpq);
-            else P.currentR[e] = P.zero + acc * P.jscale;
+            else put_current(P, e, acc * P.jscale);
         }
     }
 }
@@ -518,8 +520,7 @@ MomPatch mom_patch(const vx_patch &p) {
         M.rel[3 * i + 1] = (tl * tl + tl * tr + tr * tr) / 3.0 - (1.0 / 12);
         M.rel[3 * i + 2] = (tl * tl * tl + tl * tl * tr + tl * tr * tr + tr * tr * tr) * 0.25;
     }
-    M.zero = -0.0;
-    M.species = nullptr;
+    M.charge = M.J = M.species = nullptr;
     return M;
 }
 
@@ -555,15 +556,17 @@ static int moments_check(vx_ctx *ctx, const vx_patch *p, const vx_fields *fl) {
     return VX_OK;
 }
 
-// species: where the patch's moments are the assembled ones, the place of its
-// species' charge.
-static int moments_patch(vx_ctx *ctx, const vx_patch *p, const vx_fields *fl, bool comp, double *species = nullptr) {
+// whole: where the patch's moments are the assembled ones, the places of the charge,
+// the current and its species' charge.
+static int moments_patch(vx_ctx *ctx, const vx_patch *p, const vx_fields *fl, bool comp,
+                         double *const *whole = nullptr) {
     int rc = moments_check(ctx, p, fl);
     if (rc) return rc;
     MomArgs A{mom_patch(*p), *fl, nullptr};
-    if (species) {
-        A.p.zero = 0.0;
-        A.p.species = species;
+    if (whole) {
+        A.p.charge = whole[0];
+        A.p.J = whole[1];
+        A.p.species = whole[2];
     }
     // The table saves each column its logarithms but costs a launch (3.1 us).
     // us with / without it: 1024 x 512 at rtb 1 8.3 / 7.0, 1024 x 1024 11.9 / 10.7,
@@ -646,10 +649,8 @@ int vx_moments_whole(vx_ctx *ctx, const vx_patch *p, const vx_fields *fl, int co
     if (!charge || !J || !charges_species) return fail(ctx, VX_EINVAL, "moments: null output");
     if (p->x_pos != 0 || p->n_x * p->rtb != fl->n_f)
         return fail(ctx, VX_EINVAL, "moments: the patch does not cover the %d finest cells", fl->n_f);
-    vx_patch w = *p;
-    w.chargeR = charge;
-    w.currentR = J;
-    return moments_patch(ctx, &w, fl, compensated != 0, charges_species);
+    double *const whole[] = {charge, J, charges_species};
+    return moments_patch(ctx, p, fl, compensated != 0, whole);
 }
 
 int vx_moments_patches(vx_ctx *ctx, const vx_patch *patches, int32_t n, const vx_fields *fl, int compensated) {
