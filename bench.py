@@ -451,7 +451,8 @@ def main():
                    "wall_s": wall, "graph_ms_per_step": graph_ms,
                    "ms_per_step_driver_loop": driver_ms,
                    "tile_rows": run.tile_rows() if a.mode == "fused" else None,
-                   "tile_waves": run.tile_waves() if a.mode == "fused" else None},
+                   "tile_waves": run.tile_waves() if a.mode == "fused" else None,
+                   "tile_code": run.tile_code() if a.mode == "fused" else None},
         "roofline": {"bound": "hbm", "kernel": kernel, "achieved": achieved / 1e9,
                      "peak": HBM_PEAK / 1e9, "unit": "GB/s", "frac": achieved / HBM_PEAK,
                      "traffic": measured_traffic(kernel, params.nx, params.np),

@@ -159,6 +159,10 @@ int vx_stage_tile_rows(vx_ctx *ctx, int32_t n_x, int32_t n_p, int step, int mixe
  * (the other), 0 before the first call; all forms give the same bits.  No
  * counterpart in the reference. */
 int vx_stage_tile_waves(vx_ctx *ctx, int32_t n_x, int32_t n_p, int step, int mixed);
+/* The choice as VX_TILE_ROWS takes it: rows, + 4096 for the four-wave form, + 8192
+ * for the form with a wavefront per row; 0 before the first call.  No counterpart
+ * in the reference. */
+int vx_stage_tile_code(vx_ctx *ctx, int32_t n_x, int32_t n_p, int step, int mixed);
 int vx_fct_stage_fused_available(void);
 
 /* Ghost fill of slot `slot` of a patch whose neighbours are all the domain-edge

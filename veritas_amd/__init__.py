@@ -72,6 +72,7 @@ def host_lib():
         L.vxh_graph_stats.argtypes = [vp, ctypes.POINTER(ctypes.c_int)]
         L.vxh_tile_rows.argtypes = [vp, i, i, i]
         L.vxh_tile_waves.argtypes = [vp, i, i, i]
+        L.vxh_tile_code.argtypes = [vp, i, i, i]
         L.vxh_signatures.restype = i
         L.vxh_signatures.argtypes = [vp, i, i, i, vp, i]
         L.vxh_server_create.restype = vp
@@ -231,6 +232,13 @@ class Run:
         n_x = self.params.nx if n_x is None else n_x
         n_p = self.params.np if n_p is None else n_p
         return [host_lib().vxh_tile_waves(self.h, n_x, n_p, s) for s in range(6)]
+
+    def tile_code(self, n_x=None, n_p=None):
+        """The choice of each RK stage as VX_TILE_ROWS takes it: ",".join of these
+        pins a run to it (rows, + 4096 four-wave form, + 8192 a wavefront per row)."""
+        n_x = self.params.nx if n_x is None else n_x
+        n_p = self.params.np if n_p is None else n_p
+        return [host_lib().vxh_tile_code(self.h, n_x, n_p, s) for s in range(6)]
 
     def graph_stats(self):
         out = (ctypes.c_int * 2)()

@@ -1244,4 +1244,8 @@ int vx_stage_tile_waves(vx_ctx *ctx, int32_t n_x, int32_t n_p, int step, int mix
     return c == 0 ? 0 : (c >= W4_FORM ? 4 : 3);
 }
 
+int vx_stage_tile_code(vx_ctx *ctx, int32_t n_x, int32_t n_p, int step, int mixed) {
+    return tile_choice(ctx, n_x, n_p, step, mixed);
+}
+
 }  // extern "C"
