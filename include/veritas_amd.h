@@ -160,8 +160,9 @@ int vx_stage_tile_rows(vx_ctx *ctx, int32_t n_x, int32_t n_p, int step, int mixe
  * counterpart in the reference. */
 int vx_stage_tile_waves(vx_ctx *ctx, int32_t n_x, int32_t n_p, int step, int mixed);
 /* The choice as VX_TILE_ROWS takes it: rows, + 4096 for the four-wave form, + 8192
- * for the form with a wavefront per row; 0 before the first call.  No counterpart
- * in the reference. */
+ * for the form with a wavefront per row; 0 before the first call.  With n_x = n_p =
+ * 0: the choice of the context's last vx_fct_stage_fused_batch for that stage and
+ * precision.  No counterpart in the reference. */
 int vx_stage_tile_code(vx_ctx *ctx, int32_t n_x, int32_t n_p, int step, int mixed);
 int vx_fct_stage_fused_available(void);
 

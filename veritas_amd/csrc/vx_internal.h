@@ -30,6 +30,7 @@ struct vx_ctx {
     // strip heights of the fused stage chosen per patch shape and stage:
     // {n_x, n_p, rows, mixed, stage}
     std::vector<std::array<int, 5>> ti_cache;
+    int batch_tile[2][6] = {};  // those of the last shared launch, per precision and stage
     // device bytes held through vx_malloc (vx_ctx_live_bytes)
     std::unordered_map<void *, size_t> allocs;
     size_t live_bytes = 0;

@@ -892,27 +892,33 @@ int stage_blocks_per_cu(int step, bool mp) {
     return e == hipSuccess ? n : 0;
 }
 
+// VX_TILE_ROWS pins the choice of every launch, shared ones among them (one value,
+// or six comma-separated values, one per RK stage; rows + 4096 for the four-wave
+// form, + 8192 for the row form), e.g. to profile the configuration a timed run
+// chose.  The value of a stage, 0 without one.
+int pinned_tile(int step) {
+    const char *env = std::getenv("VX_TILE_ROWS");
+    if (!env) return 0;
+    int v[6], n = 0;
+    for (const char *q = env; *q && n < 6;) {
+        v[n++] = std::atoi(q);
+        while (*q && *q != ',') q++;
+        if (*q == ',') q++;
+    }
+    const int ti = n == 6 ? v[step] : (n >= 1 ? v[0] : 0);
+    const bool ok = (ti >= 1 && ti <= 1024) || (ti > W4_FORM && ti <= W4_FORM + 1024) ||
+                    (ti > 2 * W4_FORM && ti <= 2 * W4_FORM + ROWS_MAX);
+    return ok ? ti : 0;
+}
+
 int tile_rows(vx_ctx *ctx, const StageArgs &A0, bool mp) {
     const int nx = A0.p.n_x, np = A0.p.n_p;
     for (auto &c : ctx->ti_cache)
         if (c[0] == nx && c[1] == np && c[3] == (int)mp && c[4] == A0.step) return c[2];
     static const int cand[] = {64, 32, 16, 8, 4, 2};
-    // VX_TILE_ROWS pins the choice for this context (one value, or six
-    // comma-separated values, one per RK stage; rows + 4096 for the four-wave
-    // form), e.g. to profile the configuration a timed run chose
-    if (const char *env = std::getenv("VX_TILE_ROWS")) {
-        int v[6], n = 0;
-        for (const char *q = env; *q && n < 6;) {
-            v[n++] = std::atoi(q);
-            while (*q && *q != ',') q++;
-            if (*q == ',') q++;
-        }
-        const int ti = n == 6 ? v[A0.step] : (n >= 1 ? v[0] : 0);
-        if ((ti >= 1 && ti <= 1024) || (ti > W4_FORM && ti <= W4_FORM + 1024) ||
-            (ti > 2 * W4_FORM && ti <= 2 * W4_FORM + ROWS_MAX)) {
-            ctx->ti_cache.push_back({nx, np, ti, (int)mp, A0.step});  // this context only
-            return ti;
-        }
+    if (const int pin = pinned_tile(A0.step)) {
+        ctx->ti_cache.push_back({nx, np, pin, (int)mp, A0.step});  // this context only
+        return pin;
     }
     if (const int known = tile_lookup(ctx->device, nx, np, (int)mp, A0.step)) {
         ctx->ti_cache.push_back({nx, np, known, (int)mp, A0.step});
@@ -1113,9 +1119,10 @@ static void batch_ring_free(void *r) {
 // us as strips, 96 to 122 as rows; four mixed ones of 24 rows 38 to 55 as
 // strips, 34 to 61 as rows; a 1024 x 1024 patch of 18 rows 39 to 60 as strips,
 // 31 to 45 as rows); above: the strip height of the least rounds x (rows + 6), a round being
-// the resident wavefronts (three a SIMD) walking a strip each.
+// the resident wavefronts (three a SIMD) walking a strip each.  VX_TILE_ROWS pins it
+// (strips have one form here, held to three waves per SIMD).
 constexpr int BATCH_ROWS = 20;
-static void batch_form(vx_ctx *ctx, std::vector<StageArgs> &A) {
+static void batch_form(vx_ctx *ctx, std::vector<StageArgs> &A, int step, bool mp) {
     const double simds = 4.0 * ctx->n_cu;
     auto waves = [&](int ti) {
         double w = 0;
@@ -1123,7 +1130,10 @@ static void batch_form(vx_ctx *ctx, std::vector<StageArgs> &A) {
         return w;
     };
     int form = 2, ti = ROWS_MAX;
-    if (waves(1) > BATCH_ROWS * simds) {
+    if (const int pin = pinned_tile(step)) {
+        form = pin / W4_FORM == 2 ? 2 : 0;
+        ti = pin % W4_FORM;
+    } else if (waves(1) > BATCH_ROWS * simds) {
         form = 0;
         double best = 1e300;
         for (int t = 96; t >= 8; t -= 4) {
@@ -1139,13 +1149,14 @@ static void batch_form(vx_ctx *ctx, std::vector<StageArgs> &A) {
         a.TI = ti;
         a.nstrip = (a.p.n_x + ti - 1) / ti;
     }
+    ctx->batch_tile[mp][step] = form * W4_FORM + ti;
 }
 
 static int batch_launch(vx_ctx *ctx, std::vector<StageArgs> &A, int step, bool mp) {
     if (A.empty()) return VX_OK;
-    batch_form(ctx, A);
-    const bool rows = A[0].form == 2;
     if (ctx->capturing) return fail(ctx, VX_EINVAL, "stage batch while a step graph is recorded");
+    batch_form(ctx, A, step, mp);
+    const bool rows = A[0].form == 2;
     if (!ctx->batch_ring) {
         BatchRing *b = new BatchRing;
         ctx->batch_ring = b;
@@ -1180,7 +1191,7 @@ static int batch_launch(vx_ctx *ctx, std::vector<StageArgs> &A, int step, bool m
     if (rc) return rc;
     const StageArgs *dA = (const StageArgs *)d;
     const int *dS = (const int *)(d + sizeof(StageArgs) * BATCH_MAX);
-    const int wf = rows ? ROWS_MAX + 4 : 4;
+    const int wf = rows ? A[0].TI + 4 : 4;
     const size_t lds = rows ? sizeof(double) * 64 * RT_ARRAYS * wf : 0;
     dim3 grid((unsigned)total), block(64 * wf);
 #define VX_BATCH(S)                                                                                   \
@@ -1245,6 +1256,7 @@ int vx_stage_tile_waves(vx_ctx *ctx, int32_t n_x, int32_t n_p, int step, int mix
 }
 
 int vx_stage_tile_code(vx_ctx *ctx, int32_t n_x, int32_t n_p, int step, int mixed) {
+    if (n_x == 0 && n_p == 0) return step >= 0 && step <= 5 ? ctx->batch_tile[mixed ? 1 : 0][step] : 0;
     return tile_choice(ctx, n_x, n_p, step, mixed);
 }
 
