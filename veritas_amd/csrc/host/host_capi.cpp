@@ -34,8 +34,11 @@ int dl(Run *r, const double *d, size_t n, double *out, int room) {
     return (int)n;
 }
 
-// a plane of patch p with g ghost layers, likewise
-int dl_plane(const vxh::Rectangle &p, const double *plane, int g, double *out, int room) {
+// plane w of patch p with g ghost layers, likewise: 0 to 2 layers, and less than the
+// interior (g < 0) of a plane that is no f slot
+int dl_plane(const vxh::Rectangle &p, const std::string &w, const double *plane, int g, double *out, int room) {
+    if (g > 2 || (g < 0 && slot_of(w) >= 0) || p.n_x + 2 * g < 0 || p.n_p + 2 * g < 0)
+        throw vxh::Error("plane " + w + " with " + std::to_string(g) + " ghost layers");
     const int n = (p.n_x + 2 * g) * (p.n_p + 2 * g);
     if (out && room >= n) p.Download(plane, g, out);
     return n;
@@ -258,7 +261,7 @@ int vxh_patch_get(void *h, int sp, int lvl, int idx, const char *what, int ghost
         vxh::Rectangle &p = *levels[lvl]->rectangles[idx];
         const double *pl = p.Plane(what);
         if (!pl) return -2;
-        return dl_plane(p, pl, ghosts, out, n);
+        return dl_plane(p, what, pl, ghosts, out, n);
     } catch (std::exception &e) {
         r->err = e.what();
         return -1;
@@ -375,7 +378,7 @@ int vxh_get(void *h, const char *what, int ghosts, double *out, int n) {
     try {
         std::string w(what);
         vxh::Rectangle &p = base(r);
-        if (const double *pl = p.Plane(w)) return dl_plane(p, pl, ghosts, out, n);
+        if (const double *pl = p.Plane(w)) return dl_plane(p, w, pl, ghosts, out, n);
         const vx_field_state &fs = r->sm->EMSolver->state();
         int N = fs.n_f;
         size_t ne8 = (size_t)8 * fs.n_e;

@@ -473,8 +473,15 @@ std::vector<double> Rectangle::Download(const double *plane, int g) const {
     return out;
 }
 
-// any plane as slot 0 of a patch of this shape
+// any plane as slot 0 of a patch of this shape; g < 0 leaves -g rows and columns of
+// the interior's edge out
 void Rectangle::Download(const double *plane, int g, double *out) const {
+    if (g < 0) {
+        const std::vector<double> in = Download(plane, 0);
+        const int w = n_p + 2 * g;
+        for (int i = -g; i < n_x + g; i++, out += w) std::copy_n(in.data() + (size_t)i * n_p - g, w, out);
+        return;
+    }
     vx_patch p = P;
     p.f[0] = const_cast<double *>(plane);
     dev->check(vx_patch_download(dev->ctx, &p, 0, g, out), "download");
