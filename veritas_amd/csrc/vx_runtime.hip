@@ -152,11 +152,22 @@ bool vx_device_range(const vx_ctx *ctx, const double *dev, size_t n) {
            n <= (size - off) / sizeof(double);
 }
 
+// Whether HIP does not know the host address: pinned memory takes HIP's own copy,
+// which reaches it without a second copy on the host (1024 x 1024 doubles of a
+// patch 155 us, 240 up and 360 down through the buffers).
+static bool pageable(const void *host) {
+    hipPointerAttribute_t at;
+    if (hipPointerGetAttributes(&at, host) == hipSuccess) return at.type == hipMemoryTypeUnregistered;
+    (void)hipGetLastError();
+    return true;
+}
+
 // h rows of w doubles between a pitched device array and pageable host memory,
 // through the context's two pinned buffers: a kernel packs one (or unpacks it)
 // over the link while the host copies the other.  hipMemcpy2DAsync on pageable
-// memory goes row by row: 64 x 256 doubles 490 us, 1024 x 1024 8.7 ms, 4096 x
-// 4096 54 ms on an MI355X; these 16 us, 0.17 ms and 2.7 ms.  Waits for the copy.
+// memory goes row by row: 64 x 256 doubles up 600 us, down 430, 1024 x 1024 9.6 and
+// 7.2 ms, 4096 x 4096 40 and 37 ms on an MI355X; these 16 and 17 us, 0.24 and 0.35
+// ms, 4.7 and 4.4 ms.  Waits for the copy.
 // Threads that copy at once on one context take the buffers in turn.
 static int staged_rows(vx_ctx *ctx, double *dev, size_t pitch, double *host, size_t w, size_t h, bool up,
                        const char *what) {
@@ -193,17 +204,18 @@ static int staged_rows(vx_ctx *ctx, double *dev, size_t pitch, double *host, siz
     return check_hip(ctx, hipStreamSynchronize(ctx->stream), what);
 }
 
-// A contiguous copy: whole doubles through the staging buffers, else HIP's own.
+// A contiguous copy: HIP's own, but for downloads of whole doubles of up to 16 KB
+// or from 2 MB on to pageable memory, which the staging buffers take in less time.
+// us on an MI355X, HIP's / staged: downloads 4 KB 21.7 / 13.1, 16 KB 22.0 / 13.8, 24
+// KB 10.3 / 13.9, 256 KB 20 / 23, 1 MB 62 / 63, 2 MB 122 / 115, 8 MB 482 / 363, 64 MB
+// 3870 / 2370; uploads 4 KB 13.7 / 13.4, 64 KB 10.8 / 14.5, 1 MB 39 / 43, 64 MB
+// 2360 / 2470.
 static int host_copy(vx_ctx *ctx, void *dev, void *host, size_t bytes, bool up, const char *what) {
     if (bytes == 0) return vx_sync(ctx);
-    constexpr size_t W = 1024;  // doubles a "row" of a contiguous array
-    if (bytes % sizeof(double) == 0 && host && vx_device_range(ctx, (const double *)dev, bytes / sizeof(double))) {
-        const size_t n = bytes / sizeof(double), h = n / W, rest = n % W;
-        double *d = (double *)dev, *p = (double *)host;
-        int rc = h ? staged_rows(ctx, d, W, p, W, h, up, what) : VX_OK;
-        if (!rc && rest) rc = staged_rows(ctx, d + h * W, rest, p + h * W, rest, 1, up, what);
-        return rc;
-    }
+    const size_t n = bytes / sizeof(double);
+    const bool size = bytes % sizeof(double) == 0 && (bytes <= (16 << 10) || bytes >= (2 << 20));
+    if (!up && size && host && vx_device_range(ctx, (const double *)dev, n) && pageable(host))
+        return staged_rows(ctx, (double *)dev, 1, (double *)host, 1, n, false, what);
     int rc = check_hip(ctx, up ? hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, ctx->stream)
                                : hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, ctx->stream), what);
     return rc ? rc : vx_sync(ctx);
@@ -379,7 +391,7 @@ static int patch_copy(vx_ctx *ctx, const vx_patch *p, int slot, int ghosts, doub
     const char *what = up ? "patch upload" : "patch download";
     // (an empty shape copies nothing, rows that lap over each other are HIP's to refuse too)
     const bool rows = p->n_x + 2 * ghosts > 0 && w > 0 && w <= (size_t)p->pitch && w * sizeof(double) <= vx_ctx::STAGE_BYTES;
-    if (rows && vx_device_range(ctx, dev, (h - 1) * p->pitch + w))
+    if (rows && vx_device_range(ctx, dev, (h - 1) * p->pitch + w) && pageable(host))
         return staged_rows(ctx, dev, p->pitch, host, w, h, up, what);
     hipError_t e = up ? hipMemcpy2DAsync(dev, sizeof(double) * p->pitch, host, sizeof(double) * w,
                                          sizeof(double) * w, h, hipMemcpyHostToDevice, ctx->stream)
