@@ -215,3 +215,44 @@ def test_whole_patch_keeps_its_own_moments(shape, comp):
     c.p[0].planes[24] = c.p[0].planes[25] = None
     assert c.L.vx_moments_whole(*args) == 0
     c.free()
+
+
+@pytest.mark.parametrize("a", ["zero", "uniform", "pulse"])
+@pytest.mark.parametrize("comp", [False, True])
+def test_tall_patches_around_the_rules(a, comp):
+    """Heights on either side of those from which a small patch has a table, alone
+    (with it) and in one launch with another (without); full launches of tall columns
+    (8 a workgroup) with a ragged last workgroup, against a part of their columns."""
+    tall = [(10, 1022, 1, False), (9, 1026, 1, False), (6, 1088, 2, True), (10, 1536, 1, False), (11, 1538, 1, False),
+            (7, 1602, 4, False), (5, 1600, 1, True), (70, 2050, 1, False)]
+    c = Case(tall + [(2050, 2050, 1, False), (1030, 2050, 1, False)], a)
+    n = len(tall)
+    alone = [c.one(k, comp) for k in range(n)]
+    assert c.L.vx_moments_patches(c.ctx, c.p, n, ctypes.byref(c.fl), comp) == 0
+    for k in range(n):
+        for x, y in zip(c.get(k), alone[k]):
+            assert np.array_equal(x, y) and np.abs(y).max() > 0, k
+    full = c.one(n, comp)
+    c.p[n + 1].planes[1] = c.p[n].planes[1]  # the first columns of the same f
+    for x, y in zip(c.one(n + 1, comp), full):
+        assert np.array_equal(x, y[:1030]) and np.abs(y).min() > 0
+    c.free()
+
+
+def test_a_tall_patch_recorded_before_there_is_a_table():
+    c = Case([(10, 1602, 1, False)], "uniform")
+    L, g = c.L, ctypes.c_void_p()
+    L.vx_graph_begin.argtypes, L.vx_graph_destroy.argtypes = [ctypes.c_void_p], [ctypes.c_void_p]
+    L.vx_graph_end.argtypes = [ctypes.c_void_p, ctypes.POINTER(ctypes.c_void_p)]
+    L.vx_graph_launch.argtypes = [ctypes.c_void_p, ctypes.c_void_p]
+    assert L.vx_graph_begin(c.ctx) == 0
+    assert L.vx_moments_patch(c.ctx, ctypes.byref(c.p[0]), ctypes.byref(c.fl)) == 0
+    assert L.vx_graph_end(c.ctx, ctypes.byref(g)) == 0
+    want = c.one(0)
+    for _ in range(3):
+        assert L.vx_graph_launch(c.ctx, g) == 0
+        for x, y in zip(c.get(0), want):
+            assert np.array_equal(x, y) and np.abs(y).min() > 0
+        c.one(0)
+    L.vx_graph_destroy(g)
+    c.free()

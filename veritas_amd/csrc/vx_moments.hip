@@ -22,7 +22,7 @@ using namespace vxd;
 namespace {
 
 constexpr int MAX_RTB = 4;  // coarsest level of a 3-level hierarchy at ratio 2
-constexpr long TAB_CELLS = 1 << 20;  // a patch of more cells gets a logarithm table
+constexpr long TAB_CELLS = 1 << 20;  // a patch of more cells gets a logarithm table (and a tall one)
 constexpr long BATCH_CELLS = 1 << 21;  // a patch of more cells has a launch (and a table) of its own
 constexpr int TAB_KEY = 8;  // A^2, pmin, dp, p_pos, mc2inv, c1, c2, n_p
 
@@ -272,13 +272,17 @@ __device__ __forceinline__ void moments_columns(const MomPatch &P, const vx_fiel
         // and its ring of chunks in flight is unrolled: slot d holds chunk
         // k0 + d in fixed registers and is reloaded with chunk k0 + d + WDEPTH
         // once its values are formed (a rotating copy would wait for the loads
-        // in flight).
+        // in flight).  COMP with a table, a loop of few instructions, has no exit
+        // inside it (the chunks past the last are skipped cells) and reloads a slot
+        // behind the chunk's sums: 4096 x 4096 29.0 us against 32.6, 2048 x 4096 18.3
+        // and 20.9.
         double aR[RTB], cR[RTB], aJ[RTB], cJ[RTB];  // COMP: the lanes' sums
 #pragma unroll
         for (int s = 0; s < RTB; s++) aR[s] = cR[s] = aJ[s] = cJ[s] = 0.0;
         auto run = [&](auto tab_c) __attribute__((always_inline)) {
             constexpr bool TAB = decltype(tab_c)::value;
             constexpr int NL = TAB ? 1 : RTB;  // logarithm sequences
+            constexpr bool WHOLE = COMP && TAB;  // whole rounds of the ring, loads behind the sums
             double pv[WDEPTH][NR], pt[WDEPTH];
             int pn[WDEPTH];
             auto load = [&](int k, int d) __attribute__((always_inline)) {
@@ -327,7 +331,7 @@ __device__ __forceinline__ void moments_columns(const MomPatch &P, const vx_fiel
                 logs(0, L);
             }
             int nf = NEST ? pn[0] : 0;
-            for (int k0 = 0;; k0 += WDEPTH) {
+            for (int k0 = 0; !WHOLE || k0 < nchunk; k0 += WDEPTH) {
 #pragma unroll
                 for (int d = 0; d < WDEPTH; d++) {
                     // chunk k, its values in V and L (the only branch leaves
@@ -335,8 +339,10 @@ __device__ __forceinline__ void moments_columns(const MomPatch &P, const vx_fiel
                     // the slots loaded after it)
                     const int k = k0 + d, dn = (d + 1) % WDEPTH;  // dn: chunk k + 1
                     const int jb = 64 * k;
-                    load(k + WDEPTH, d);
-                    __builtin_amdgcn_sched_barrier(0);
+                    if (!WHOLE) {
+                        load(k + WDEPTH, d);
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
                     double Vn[RTB], Ln[NL];
                     values(pv[dn], Vn);
                     if (TAB) Ln[0] = pt[dn];
@@ -364,9 +370,10 @@ __device__ __forceinline__ void moments_columns(const MomPatch &P, const vx_fiel
 #pragma unroll
                     for (int s = 0; s < NL; s++) L[s] = Ln[s];
                     if (NEST) nf = pn[dn];
+                    if (WHOLE) load(k + WDEPTH, d);
                     __builtin_amdgcn_sched_barrier(0);
                     if (!COMP) __syncthreads();
-                    if (k + 1 == nchunk) return;
+                    if (!WHOLE && k + 1 == nchunk) return;
                 }
             }
         };
@@ -574,8 +581,13 @@ static int moments_patch(vx_ctx *ctx, const vx_patch *p, const vx_fields *fl, bo
     // 8000 x 256 27.8 / 33.7; columns with a pulse do not use it (500 x 512 at rtb
     // 4 21.1 / 19.1).  A wavefront that forms the terms for its workgroup's columns
     // instead: 9.2 at 1024 x 1024, but 52 at 4096 x 4096, 46 with the table.
-    if ((long)p->n_x * p->n_p > TAB_CELLS) {
-        size_t need = (size_t)tab_entries(2, p->n_p);
+    // In launches that do not fill the device a column's chain of chunks counts: any
+    // up to 512 columns, of 1280 p-cells 12.4 / 11.8, 1536 13.6 / 13.7, 2048 16.2 / 17.4,
+    // 4096 27.3 / 31.7; compensated, of 1024 8.7 / 9.5, 2048 10.6 / 15.8, 4096 15 / 28.
+    // (They go without where a graph is recorded before there is a table.)
+    size_t need = (size_t)tab_entries(2, p->n_p);
+    const bool tall = p->n_p > (comp ? 1024 : 1536) && !(ctx->capturing && ctx->mom_table_n < need);
+    if (tall || (long)p->n_x * p->n_p > TAB_CELLS) {
         if (ctx->mom_table_n < need) {
             if (ctx->capturing) return fail(ctx, VX_EINVAL, "moments: table growth while a step graph is recorded");
             // The outgrown table stays until the context ends: a graph recorded
@@ -604,15 +616,18 @@ static int moments_patch(vx_ctx *ctx, const vx_patch *p, const vx_fields *fl, bo
         if ((rc = check_launch(ctx, "k_moment_table"))) return rc;
     }
     LaunchTimer lt(ctx, "k_moments");
-    // 8 columns a workgroup for tall columns: one consumer for more of them, and
-    // enough chunks for its start.  us, 8 / 4 columns, without and with a pulse: 8190
-    // x 1024 30.1 / 31.6, 53.5 / 46.5; 4096 x 2048 25.4 / 27.5, 45.8 / 47.3; 4096 x 4096
-    // 39.8 / 47.1, 84.0 / 90.8.
-    const bool tall = !comp && p->rtb == 1 && !p->nested && p->n_p >= 2048;
-    const int WCOL = tall ? MCOL_TALL : MCOL;
+    // 8 columns a workgroup where both the columns are tall and the workgroups fill
+    // the device: one consumer for more of them, and enough chunks for its start.  us,
+    // 8 / 4 columns, without and with a pulse: 8190 x 1024 30.1 / 31.6, 53.5 / 46.5; 4096 x
+    // 2048 27.2 / 27.1, 43.8 / 45.8; 4096 x 4096 34.2 / 40.7, 75.9 / 83.1; compensated 18.0 /
+    // 22.6 and 29.0 / 30.3 without.  Where they do not: 1024 x 2048 with a pulse 26.5 / 20.2,
+    // 64 x 4096 without a table 44.3 / 31.6.
+    const bool wide = p->rtb == 1 && !p->nested && p->n_p >= 2048 && p->n_x >= MCOL_TALL * ctx->n_cu;
+    const int WCOL = wide ? MCOL_TALL : MCOL;
     const dim3 g((unsigned)((p->n_x + WCOL - 1) / WCOL)), b(64 * (comp ? WCOL : WCOL + 1));
-    if (tall) {
-        k_moments<1, false, false, MCOL_TALL><<<g, b, 0, ctx->stream>>>(A);
+    if (wide) {
+        if (comp) k_moments<1, true, false, MCOL_TALL><<<g, b, 0, ctx->stream>>>(A);
+        else k_moments<1, false, false, MCOL_TALL><<<g, b, 0, ctx->stream>>>(A);
         return check_launch(ctx, "k_moments");
     }
     switch (p->rtb * 4 + (comp ? 2 : 0) + (p->nested ? 1 : 0)) {
