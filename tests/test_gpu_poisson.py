@@ -59,3 +59,9 @@ def test_poisson_matches_the_oracle(lib, n_f):
             assert s.get("Ex0", 1)[0] == ex0
             assert np.array_equal(s.get("E", n_f), -fc * d + ex0)
         s.free()
+
+
+@pytest.mark.parametrize("n_f", [131070, 131072, 131074, 200002, 263170])
+def test_poisson_of_many_cells_matches_the_oracle(lib, n_f):
+    """Either side of the border at 131072 cells, where each compute unit has a chunk."""
+    test_poisson_matches_the_oracle(lib, n_f)

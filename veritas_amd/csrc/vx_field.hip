@@ -79,7 +79,7 @@ __device__ __forceinline__ void dd_sub(double &sh, double &sl, double a, double 
     sh = tt;
 }
 
-// ------------------------------------------------ multi-workgroup solve, n_f > 4096
+// ------------------------------------------------ multi-workgroup solve, 4096 < n_f <= PM_MAX
 // Workgroup b owns the chunk of 64 MW consecutive entries from 64 MW b on,
 // wavefront w of it the sub-chunk w of 64 entries.  One approximate solve of
 // A c = v and the residual of the next round are one launch:
@@ -110,6 +110,7 @@ __device__ __forceinline__ void dd_sub(double &sh, double &sl, double a, double 
 // as 13 launches (the two scans and the convolution apart), 42 us as 5 with MW = 8 and
 // each launch's reads one behind the other.
 constexpr int PM_SMALL = 192 * 192;  // largest n_f with MW = 3: three chunks a lane
+constexpr int PM_MAX = 512 * 256;      // largest n_f of this form: a chunk for every compute unit
 __host__ __device__ constexpr int pm_mw(int n) { return n <= PM_SMALL ? 3 : 8; }
 constexpr int SUB = 64;
 constexpr int HALO = 2;
@@ -374,6 +375,256 @@ __global__ __launch_bounds__(64 * (MW + 5)) void k_pm_solve(PoissonMB P) {
         if (blk == 0 && threadIdx.x == 0) *F.Ex0 = ex0n;
         const int c = j + HALO;
         if (j < n_own) F.E[lo + j] = -fc * (8 * (xw[c + 1] - xw[c - 1]) - xw[c + 2] + xw[c - 2]) + ex0n;
+    }
+}
+
+// ------------------------------------------------ multi-workgroup solve, n_f > PM_MAX
+// The same steps with the sums, the scans and the convolution in launches of their
+// own, 13 in all; chunks of 1024 entries:
+//   k_pl_scan_s  S and the chunks' sums of S;
+//   k_pl_scan_y  d0, D and y;
+//   k_pl_conv    c, x, then the next residual and the chunks' sums of it, or phi, Ex0
+//                and E.
+// A sum across workgroups is formed from per-chunk partials that every workgroup
+// reads and adds in the same order, so all of them hold the same bits.  The form in
+// five launches forms sums over all chunks in every wavefront and a sub-chunk's y
+// up to three times, which costs more than the launches it saves once a compute unit
+// has more than one chunk: us on an MI355X, 5 / 13 launches, 131072 entries 45 / 71,
+// 200000 88 / 77, 1000000 711 / 167, 4000000 8500 / 640.
+constexpr int PL_T = 256, PL_PER = 4, PL_CHUNK = PL_T * PL_PER;
+__host__ __device__ constexpr int pl_chunks(int n) { return (n + PL_CHUNK - 1) / PL_CHUNK; }
+
+// Work layout (doubles): b | xa | xb | ra | rb | S | y | Pa[nb] | Pb[nb] | Ex0 on entry
+struct PlWork {
+    double *b, *xa, *xb, *ra, *rb, *S, *y, *Pa, *Pb, *ex0;
+};
+__host__ __device__ inline PlWork pl_work(double *w, int n) {
+    const size_t N = n;
+    const int nb = pl_chunks(n);
+    PlWork W;
+    W.b = w;
+    W.xa = w + N;
+    W.xb = w + 2 * N;
+    W.ra = w + 3 * N;
+    W.rb = w + 4 * N;
+    W.S = w + 5 * N;
+    W.y = w + 6 * N;
+    W.Pa = w + 7 * N;
+    W.Pb = W.Pa + nb;
+    W.ex0 = W.Pb + nb;
+    return W;
+}
+
+struct PoissonLong {
+    vx_field_state fs;
+    double w1, w2, w3;
+    double g[NG];
+    double invN;
+    int nb;
+    PlWork W;
+    const double *in;    // right-hand side of this solve (b, then residuals)
+    const double *x_in;  // x before this solve's correction
+    double *x_out;       // x after it
+    double *r_out;       // next residual
+};
+
+__device__ __forceinline__ double wave_incl_scan(double v) {
+    const int lane = threadIdx.x & 63;
+    for (int off = 1; off < 64; off <<= 1) {
+        double t = __shfl_up(v, off, 64);
+        if (lane >= off) v += t;
+    }
+    return v;
+}
+
+__device__ __forceinline__ double wave_sum(double v) {
+    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+    return v;
+}
+
+// sum of v[lo..hi) in a fixed order; every lane of every wave gets the same bits
+__device__ __forceinline__ double wave_range_sum(const double *v, int lo, int hi) {
+    double s = 0.0;
+    for (int k = lo + (threadIdx.x & 63); k < hi; k += 64) s += v[k];
+    return wave_sum(s);
+}
+
+__device__ __forceinline__ double pl_sum(double v, double *lds) {
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    v = wave_sum(v);
+    if (lane == 0) lds[w] = v;
+    __syncthreads();
+    double r = ((lds[0] + lds[1]) + lds[2]) + lds[3];
+    __syncthreads();
+    return r;
+}
+
+// exclusive prefix of the per-thread totals over the workgroup
+__device__ __forceinline__ double pl_offset(double tot, double *lds) {
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    double inc = wave_incl_scan(tot);
+    double exc = __shfl_up(inc, 1, 64);
+    if (lane == 0) exc = 0.0;
+    if (lane == 63) lds[w] = inc;
+    __syncthreads();
+    double off = 0.0;
+    for (int k = 0; k < w; k++) off += lds[k];
+    __syncthreads();
+    return off + exc;
+}
+
+// b = dx^2 eps0_inv (charge + neutral) (EMSolver.cpp:157-167), its chunk sums
+// over entries >= 1, and the entry value of Ex0
+__global__ __launch_bounds__(PL_T) void k_pl_rhs(PoissonLong P) {
+    __shared__ double lds[PL_T / 64];
+    const vx_field_state &F = P.fs;
+    const int N = F.n_f, base = blockIdx.x * PL_CHUNK + threadIdx.x * PL_PER;
+    const double te = vx_eps0_inv;
+    double s = 0.0;
+#pragma unroll
+    for (int k = 0; k < PL_PER; k++) {
+        const int i = base + k;
+        if (i < N) {
+            double v = te * (F.charge[i] + F.neutral[i]);
+            v *= F.dx2;
+            P.W.b[i] = v;
+            if (i >= 1) s += v;
+        }
+    }
+    const double tot = pl_sum(s, lds);
+    if (threadIdx.x == 0) {
+        P.W.Pa[blockIdx.x] = tot;
+        if (blockIdx.x == 0) *P.W.ex0 = *F.Ex0;
+    }
+}
+
+__global__ __launch_bounds__(PL_T) void k_pl_scan_s(PoissonLong P) {
+    __shared__ double lds[PL_T / 64];
+    const int N = P.fs.n_f, blk = blockIdx.x, base = blk * PL_CHUNK + threadIdx.x * PL_PER;
+    const double tail = wave_range_sum(P.W.Pa, 0, P.nb);
+    // S at the chunk's first entry: v'_0 = -tail plus the entries >= 1 before the chunk
+    const double start = blk == 0 ? 0.0 : -tail + wave_range_sum(P.W.Pa, 0, blk);
+    double e[PL_PER], tot = 0.0;
+#pragma unroll
+    for (int k = 0; k < PL_PER; k++) {
+        const int i = base + k;
+        e[k] = (i == 0) ? -tail : (i < N ? P.in[i] : 0.0);
+        tot += e[k];
+    }
+    double run = start + pl_offset(tot, lds);
+    double ssum = 0.0;
+#pragma unroll
+    for (int k = 0; k < PL_PER; k++) {
+        const int i = base + k;
+        if (i < N) {
+            P.W.S[i] = run;
+            ssum += run;
+        }
+        run += e[k];
+    }
+    const double t2 = pl_sum(ssum, lds);
+    if (threadIdx.x == 0) P.W.Pb[blk] = t2;
+}
+
+__global__ __launch_bounds__(PL_T) void k_pl_scan_y(PoissonLong P) {
+    __shared__ double lds[PL_T / 64];
+    const int N = P.fs.n_f, blk = blockIdx.x, base = blk * PL_CHUNK + threadIdx.x * PL_PER;
+    const double d0 = wave_range_sum(P.W.Pb, 0, P.nb) * P.invN;
+    // sum of D over the earlier chunks: (entries - [chunk 0]) * d0 - (chunk sum of S)
+    double sd = 0.0;
+    for (int k = threadIdx.x & 63; k < blk; k += 64) {
+        const int n = min(PL_CHUNK, N - k * PL_CHUNK) - (k == 0 ? 1 : 0);
+        sd += (double)n * d0 - P.W.Pb[k];
+    }
+    const double offD = wave_sum(sd);
+    double D[PL_PER], tot = 0.0;
+#pragma unroll
+    for (int k = 0; k < PL_PER; k++) {
+        const int i = base + k;
+        D[k] = (i == 0 || i >= N) ? 0.0 : d0 - P.W.S[i];
+        tot += D[k];
+    }
+    double run = offD + pl_offset(tot, lds);
+#pragma unroll
+    for (int k = 0; k < PL_PER; k++) {
+        const int i = base + k;
+        run += D[k];
+        if (i < N) P.W.y[i] = run;
+    }
+}
+
+// MODE 0: first solve (x = c); 1: refinement (x += c); both then form the next
+// residual.  MODE 2: last refinement, writes phi (x_out), Ex0 and E.
+template <int MODE>
+__global__ __launch_bounds__(PL_T) void k_pl_conv(PoissonLong P) {
+    __shared__ double yw[PL_CHUNK + 2 * CW];
+    __shared__ double ys[NSPEC + 2 * (NG - 1)];
+    __shared__ double xw[PL_CHUNK + 2 * HALO];
+    __shared__ double cs[NSPEC];
+    __shared__ double lds[PL_T / 64];
+    const vx_field_state &F = P.fs;
+    const int N = F.n_f, blk = blockIdx.x, lo = blk * PL_CHUNK;
+    const int n_own = min(PL_CHUNK, N - lo);
+    const double *y = P.W.y;
+    for (int j = threadIdx.x; j < n_own + 2 * CW; j += PL_T) yw[j] = y[wrap(lo - CW + j, N)];
+    for (int j = threadIdx.x; j < NSPEC + 2 * (NG - 1); j += PL_T) ys[j] = y[wrap(-3 - (NG - 1) + j, N)];
+    __syncthreads();
+    if (threadIdx.x < NSPEC) cs[threadIdx.x] = conv_at(ys, threadIdx.x + NG - 1, P.g);
+    __syncthreads();
+    const double cp0 = cs[3];  // (M^-1 y)_0
+    // row 0 (the approximate solve's last step): c_0 from c_1, c_2, c_{N-2}, c_{N-1}
+    const double c0 = P.in[0] - (((P.w1 * (cs[4] - cp0) + P.w2 * (cs[5] - cp0)) + P.w2 * (cs[1] - cp0)) +
+                                 P.w1 * (cs[2] - cp0));
+    // x on the chunk and its halo
+    for (int j = threadIdx.x; j < n_own + 2 * HALO; j += PL_T) {
+        const int gi = wrap(lo - HALO + j, N);
+        const double c = (gi == 0) ? c0 : conv_at(yw, j + NG - 1, P.g) - cp0;
+        const double xn = MODE == 0 ? c : P.x_in[gi] + c;
+        xw[j] = xn;
+        if (j >= HALO && j < n_own + HALO) P.x_out[gi] = xn;
+    }
+    __syncthreads();
+    if (MODE < 2) {
+        // r = b - A x in double-double, rounded once (term order as the oracle's)
+        double s = 0.0;
+        for (int j = threadIdx.x; j < n_own; j += PL_T) {
+            const int i = lo + j, c = j + HALO;
+            double sh = P.W.b[i], sl = 0.0;
+            auto sub = [&](double a, double xv) { dd_sub(sh, sl, a, xv); };
+            if (i == 0) {
+                sub(1.0, xw[c]); sub(P.w1, xw[c + 1]); sub(P.w2, xw[c + 2]); sub(P.w2, xw[c - 2]);
+                sub(P.w1, xw[c - 1]);
+            } else {
+                const double cf[5] = {P.w2, P.w1, P.w3, P.w1, P.w2};
+                for (int d = -2; d <= 2; d++) {
+                    if (wrap(i + d, N) == 0) continue;
+                    sub(cf[d + 2], xw[c + d]);
+                }
+            }
+            const double r = sh + sl;
+            P.r_out[i] = r;
+            if (i >= 1) s += r;
+        }
+        const double tot = pl_sum(s, lds);
+        if (threadIdx.x == 0) P.W.Pa[blk] = tot;
+    } else {
+        // EMSolver.cpp:191: Ex0 += -(E(-1) + E(0)) * 0.5 with the entry Ex0, from phi
+        // at N-3..N-1, 0..2 (recomputed here with the owners' operations)
+        double ps[NSPEC];
+#pragma unroll
+        for (int k = 0; k < NSPEC; k++) {
+            const int gi = wrap(k - 3, N);
+            ps[k] = P.x_in[gi] + (k == 3 ? c0 : cs[k] - cp0);
+        }
+        const double ex0 = *P.W.ex0, fc = F.field_coef;
+        const double e_m1 = -fc * (8 * (ps[3] - ps[1]) - ps[4] + ps[0]) + ex0;
+        const double e_0 = -fc * (8 * (ps[4] - ps[2]) - ps[5] + ps[1]) + ex0;
+        const double ex0n = ex0 + -(e_m1 + e_0) * 0.5;
+        if (blk == 0 && threadIdx.x == 0) *F.Ex0 = ex0n;
+        for (int j = threadIdx.x; j < n_own; j += PL_T) {
+            const int c = j + HALO;
+            F.E[lo + j] = -fc * (8 * (xw[c + 1] - xw[c - 1]) - xw[c + 2] + xw[c - 2]) + ex0n;
+        }
     }
 }
 
@@ -883,12 +1134,12 @@ __global__ void k_neutralize(vx_field_state F) {
 // device current (scratch_address, at context creation).
 __host__ __device__ constexpr size_t pm_work_elems(int n) { return 7 * (size_t)n + 2 * (((size_t)n + 1023) / 1024) + 1; }
 constexpr size_t NOALLOC_WORK = pm_work_elems(VX_POISSON_NOALLOC_MAX_NF);
-// pm_work's 5 n + 1 doubles and 8 (1 + MW) per chunk of sums fit for every n that
-// the multi-workgroup solve serves
+// pl_work's layout, whose size pm_work's 5 n + 1 doubles and 8 (1 + MW) per chunk of
+// sums stay below for every n that they serve
 constexpr bool pm_fits(int n) {
     return 5 * (size_t)n + 1 + (size_t)pm_chunks(n) * 2 * 4 * (1 + pm_mw(n)) <= pm_work_elems(n);
 }
-static_assert(pm_fits(4097) && pm_fits(PM_SMALL) && pm_fits(PM_SMALL + 1), "work array");
+static_assert(pm_fits(4097) && pm_fits(PM_SMALL) && pm_fits(PM_SMALL + 1) && pm_fits(PM_MAX), "work array");
 static_assert(2 * SUB > 2 * 4 * 2, "sums per sub-chunk (and its share of its chunk's) against 2 doubles per entry");
 static __device__ __align__(256) double scratch[NOALLOC_WORK];
 constexpr int MAX_DEVICES = 64;
@@ -928,6 +1179,38 @@ extern "C" {
 
 size_t vx_field_work_elems(int32_t n_f) { return pm_work_elems(n_f); }
 
+static int poisson_long(vx_ctx *ctx, const PoissonArgs &P, double *work) {
+    PoissonLong M;
+    M.fs = P.fs;
+    M.w1 = P.w1;
+    M.w2 = P.w2;
+    M.w3 = P.w3;
+    for (int k = 0; k < NG; k++) M.g[k] = P.g[k];
+    M.invN = P.invN;
+    M.nb = pl_chunks(P.fs.n_f);
+    M.W = pl_work(work, P.fs.n_f);
+    const PlWork &W = M.W;
+    const unsigned nb = (unsigned)M.nb;
+    k_pl_rhs<<<nb, PL_T, 0, ctx->stream>>>(M);
+    // four approximate solves: of b (x = c), then of three residuals (x += c)
+    const double *in[4] = {W.b, W.ra, W.rb, W.ra};
+    double *r_out[4] = {W.ra, W.rb, W.ra, nullptr};
+    const double *x_in[4] = {nullptr, W.xa, W.xb, W.xa};
+    double *x_out[4] = {W.xa, W.xb, W.xa, P.fs.phi};
+    for (int s = 0; s < 4; s++) {
+        M.in = in[s];
+        M.r_out = r_out[s];
+        M.x_in = x_in[s];
+        M.x_out = x_out[s];
+        k_pl_scan_s<<<nb, PL_T, 0, ctx->stream>>>(M);
+        k_pl_scan_y<<<nb, PL_T, 0, ctx->stream>>>(M);
+        if (s == 0) k_pl_conv<0><<<nb, PL_T, 0, ctx->stream>>>(M);
+        else if (s < 3) k_pl_conv<1><<<nb, PL_T, 0, ctx->stream>>>(M);
+        else k_pl_conv<2><<<nb, PL_T, 0, ctx->stream>>>(M);
+    }
+    return check_launch(ctx, "k_poisson");
+}
+
 static int poisson(vx_ctx *ctx, const vx_field_state *fs, double *work) {
     int rc = validate_fs(ctx, fs);
     if (rc) return rc;
@@ -961,6 +1244,8 @@ static int poisson(vx_ctx *ctx, const vx_field_state *fs, double *work) {
         else k_poisson_one<8, 8><<<1, 512, 0, ctx->stream>>>(P);
         return check_launch(ctx, "k_poisson");
     }
+    if (!work) return fail(ctx, VX_EINVAL, "poisson: no work array for n_f = %d", fs->n_f);
+    if (fs->n_f > PM_MAX) return poisson_long(ctx, P, work);
     PoissonMB M;
     M.fs = *fs;
     M.w1 = P.w1;
@@ -969,7 +1254,6 @@ static int poisson(vx_ctx *ctx, const vx_field_state *fs, double *work) {
     for (int k = 0; k < NG; k++) M.g[k] = P.g[k];
     M.invN = P.invN;
     M.nb = pm_chunks(fs->n_f);
-    if (!work) return fail(ctx, VX_EINVAL, "poisson: no work array for n_f = %d", fs->n_f);
     M.W = pm_work(work, fs->n_f);
     const PmWork &W = M.W;
     const unsigned nb = (unsigned)M.nb;
