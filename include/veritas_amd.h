@@ -266,10 +266,11 @@ int vx_neutralize(vx_ctx *ctx, const vx_field_state *fs);
  * (host arrays q, m, dp_finest); result written to *out on the host. */
 int vx_cfl_bound(vx_ctx *ctx, const vx_field_state *fs, int n_species, const double *q,
                  const double *m, const double *dp_finest, double *out);
-/* The same bound computed on the device and copied to pinned host memory
- * without waiting; vx_cfl_result waits for that copy and returns the bound
- * (bit-identical to vx_cfl_bound: the maximum is exact in any order).  Lets a
- * caller that steps several runs queue all of them before it waits for one. */
+/* The same without waiting: the launch writes the maxima of its workgroups straight
+ * to pinned host memory, and vx_cfl_result waits for it and returns the bound from
+ * them (bit-identical to vx_cfl_bound, which waits at once and takes more than 8
+ * species too: the maximum is exact in any order).  Lets a caller that steps several
+ * runs queue all of them before it waits for one. */
 int vx_cfl_bound_async(vx_ctx *ctx, const vx_field_state *fs, int n_species, const double *q,
                        const double *m, const double *dp_finest);
 int vx_cfl_result(vx_ctx *ctx, double *out);

@@ -457,6 +457,7 @@ void Rectangle::UnaliasSlots() {
                "unalias slots");
 }
 
+// (of the class interface; the solver's assembly takes all patches in one call)
 void Rectangle::CalculateRhoAndJ() {
     dev->check(vx_moments_patches(dev->ctx, &P, 1, &EMSolver->fields(), EMSolver->compensated_moments), "moments");
 }

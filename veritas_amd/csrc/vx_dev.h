@@ -282,34 +282,9 @@ __device__ __forceinline__ double shup1(double v) { return wave_shift1<DPP_WAVE_
 // Mixed-precision helpers: f scaled by an exact power of two (sinv = 2^-k
 // with 2^k near the patch's max |f|) and rounded to FP32 for the WENO weights
 // and the Zalesak ratios; face values, fluxes and updates stay FP64.
-// WENO face value with the weights in FP32 (g: f * sinv in FP32) and the
-// candidates and the blend in FP64; same candidate choice as vxd::weno.
-__device__ __forceinline__ double weno_mp(double f1, double f2, double f3, double f4, float g1, float g2,
-                                          float g3, float g4, float eps, bool right) {
-    const double fL = (1.0 / 6) * (-f1 + 5 * f2 + 2 * f3);
-    const double fR = (1.0 / 6) * (2 * f2 + 5 * f3 - f4);
-    const float AL = g1 - 2 * g2 + g3, BL = g3 - g1;
-    const float AR = g2 - 2 * g3 + g4, BR = g4 - g2;
-    const float bL = eps + (4.0f / 3 * (AL * AL) + 0.5f * AL * BL + 0.25f * (BL * BL));
-    const float bR = eps + (4.0f / 3 * (AR * AR) - 0.5f * AR * BR + 0.25f * (BR * BR));
-    // oL / (oL + oR) with o = 0.5 / b^2 is bR^2 / (bL^2 + bR^2); both are
-    // divided by the larger b first, so the squares stay in [0, 1]
-    const float m = fmaxf(bL, bR);
-    const bool ok = m > 1e-30f;
-    const float rm = __builtin_amdgcn_rcpf(ok ? m : 1.0f);
-    const float x = bL * rm, y = bR * rm, x2 = x * x, y2 = y * y;
-    const float rden = __builtin_amdgcn_rcpf(x2 + y2);
-    const float wL = ok ? y2 * rden : 0.5f, wR = ok ? x2 * rden : 0.5f;
-    const float wL0 = wL * (0.75f + wL * (wL - 0.5f));
-    const float wR0 = wR * (0.75f + wR * (wR - 0.5f));
-    const bool takeL = right ? (wL0 > wR0) : (wL0 < wR0);
-    const float w = (takeL ? wL0 : wR0) * __builtin_amdgcn_rcpf(wL0 + wR0);
-    return fR + (double)w * (fL - fR);
-}
-
-// The parts of weno_mp that belong to one cell, as vxd::WenoCell: candidates
-// in FP64 and smoothness measures in FP32 (the same operations, so the same
-// bits), each formed once per cell instead of once per face and side.
+// The parts of the mixed-precision WENO that belong to one cell, as vxd::WenoCell:
+// candidates in FP64 and smoothness measures in FP32 (g: f * sinv in FP32), each
+// formed once per cell instead of once per face and side.
 struct WenoCellMp {
     double fL, fR;
     float bL, bR;
@@ -326,7 +301,11 @@ __device__ __forceinline__ WenoCellMp weno_cell_mp(double fm, double f, double f
     c.bR = eps + (aa - ab + bb);
     return c;
 }
+// Face value from the left cell's (fL, bL) and the right cell's (fR, bR): weights in
+// FP32, the blend in FP64; same candidate choice as vxd::weno.
 __device__ __forceinline__ double weno_face_mp(double fL, float bL, double fR, float bR, bool right) {
+    // oL / (oL + oR) with o = 0.5 / b^2 is bR^2 / (bL^2 + bR^2); both are
+    // divided by the larger b first, so the squares stay in [0, 1]
     const float m = fmaxf(bL, bR);
     const bool ok = m > 1e-30f;
     const float rm = __builtin_amdgcn_rcpf(ok ? m : 1.0f);

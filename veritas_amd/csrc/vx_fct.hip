@@ -67,7 +67,7 @@ __device__ __forceinline__ double patch_E(const vx_patch &p, const vx_fields &fl
 // there, and FxH_s/FpH_s (FxL0/FpL0 at stage 0) where the reference's loops
 // compute them; later stages read the stored FxL0/FpL0 (the coarse-fine flux
 // program may have replaced them at interface faces).
-// MP: the WENO weights from FP32 copies of f scaled by A.sinv (vxd::weno_mp);
+// MP: the WENO weights from FP32 copies of f scaled by A.sinv (vxd::weno_face_mp);
 // candidates, fluxes and the RK combination stay FP64.
 // Stage 5 needs the earlier stages' fluxes only through its combination: stage
 // 4 also writes stage 5's partial sum b_0 F_0 + ... + b_4 F_4 (left to right,

@@ -501,9 +501,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
     stage_tile<STEP, MP>(A, xcd_tile());
 }
 // The same stage compiled for four resident waves per SIMD (at most 128
-// VGPRs; some stages then keep a few loop-invariant values in scratch): more
-// waves to hide latency against a few more loads.  The strip-height timing
-// picks between the two forms per patch shape and stage; both give the same bits.
+// VGPRs; the stages after 0 then keep values in scratch): more waves to hide
+// latency against a few more loads.  The strip-height timing picks between the two
+// forms at stage 0 only (tile_rows has the figures); VX_TILE_ROWS pins either at
+// every stage.  Both give the same bits.
 template <int STEP, bool MP>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_stage_w4(StageArgs A) {
     stage_tile<STEP, MP>(A, xcd_tile());
