@@ -10,7 +10,9 @@
  * Conventions: every call is stream-ordered on the context's HIP stream and
  * returns 0 on success or a negative VX_E* code; vx_last_error() gives the
  * message.  Pointers inside the descriptors are device pointers owned by the
- * caller (allocate them with vx_malloc).  Planes are FP64, laid out row-major
+ * caller (allocate them with vx_malloc).  The copies between host and device and
+ * vx_cfl_bound may run in several threads on one context; its other calls belong
+ * to one thread at a time.  Planes are FP64, laid out row-major
  * over x with p contiguous: element (i, j), i in [-2, n_x + 2), j in
  * [-2, n_p + 2), lives at (i + 2) * pitch + (j + 2); pitch is a multiple of 8.
  */
