@@ -1473,11 +1473,11 @@ int vx_cfl_result(vx_ctx *ctx, double *out) {
 
 // EMSolver.cpp:631-664 (the reference indexes the slot-0 fields without the
 // n_prepad offset): the maxima on the device, straight into the context's pinned
-// buffer, for the species the kernel holds and arrays that it may read, else on the
-// host from downloaded arrays, whose copies refuse what is not the device's (five
-// copies from pageable memory took 110 us at 64 cells, the launch and a wait 14).
-// The buffer serves the context's copies too: its mutex is held until the
-// maxima are read.
+// buffer if there is one, for the species the kernel holds and arrays that it may
+// read, else on the host from downloaded arrays, whose copies refuse what is not the
+// device's (five copies from pageable memory took 110 us at 64 cells, the launch and
+// a wait 14).  The buffer serves the context's copies too: its mutex is held until
+// the maxima are read.
 int vx_cfl_bound(vx_ctx *ctx, const vx_field_state *fs, int n_species, const double *q,
                  const double *m, const double *dp_finest, double *out) {
     int rc = validate_fs(ctx, fs);
@@ -1487,11 +1487,12 @@ int vx_cfl_bound(vx_ctx *ctx, const vx_field_state *fs, int n_species, const dou
     for (const double *a : {fs->Ay, fs->Az, fs->By, fs->Bz, fs->E}) here = here && vx_device_range(ctx, a, fs->n_f);
     if (here) {
         std::lock_guard<std::mutex> lock(ctx->stage_mu);
-        if ((rc = vx_stage_init(ctx))) return rc;
-        const int n = cfl_launch(ctx, fs, n_species, q, m, dp_finest, ctx->stage);
-        if ((rc = check_launch(ctx, "k_cfl")) || (rc = vx_sync(ctx))) return rc;
-        *out = cfl_bound(vx_cs / fs->dx_f, ctx->stage, n);
-        return VX_OK;
+        if (vx_stage_init(ctx) == VX_OK) {
+            const int n = cfl_launch(ctx, fs, n_species, q, m, dp_finest, ctx->stage);
+            if ((rc = check_launch(ctx, "k_cfl")) || (rc = vx_sync(ctx))) return rc;
+            *out = cfl_bound(vx_cs / fs->dx_f, ctx->stage, n);
+            return VX_OK;
+        }
     }
     int N = fs->n_f;
     std::vector<double> Ay(N), Az(N), By(N), Bz(N), E(N);

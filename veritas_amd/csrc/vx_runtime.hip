@@ -162,6 +162,12 @@ static bool pageable(const void *host) {
     return true;
 }
 
+// Whether there are pinned buffers to stage through; without them a copy is HIP's.
+static bool stage_there(vx_ctx *ctx) {
+    std::lock_guard<std::mutex> lock(ctx->stage_mu);
+    return vx_stage_init(ctx) == VX_OK;
+}
+
 // h rows of w doubles between a pitched device array and pageable host memory,
 // through the context's two pinned buffers: a kernel packs one (or unpacks it)
 // over the link while the host copies the other.  hipMemcpy2DAsync on pageable
@@ -173,8 +179,7 @@ static int staged_rows(vx_ctx *ctx, double *dev, size_t pitch, double *host, siz
                        const char *what) {
     constexpr size_t BUF = vx_ctx::STAGE_BYTES / sizeof(double);
     std::lock_guard<std::mutex> lock(ctx->stage_mu);
-    int rc = vx_stage_init(ctx);
-    if (rc) return rc;
+    int rc = VX_OK;
     const size_t rows = BUF / w;  // (the caller checked w <= BUF)
     double *prev_host = nullptr;  // downloads: the chunk whose kernel is under way
     size_t prev_n = 0;
@@ -214,7 +219,7 @@ static int host_copy(vx_ctx *ctx, void *dev, void *host, size_t bytes, bool up, 
     if (bytes == 0) return vx_sync(ctx);
     const size_t n = bytes / sizeof(double);
     const bool size = bytes % sizeof(double) == 0 && (bytes <= (16 << 10) || bytes >= (2 << 20));
-    if (!up && size && host && vx_device_range(ctx, (const double *)dev, n) && pageable(host))
+    if (!up && size && host && vx_device_range(ctx, (const double *)dev, n) && pageable(host) && stage_there(ctx))
         return staged_rows(ctx, (double *)dev, 1, (double *)host, 1, n, false, what);
     int rc = check_hip(ctx, up ? hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, ctx->stream)
                                : hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, ctx->stream), what);
@@ -391,7 +396,7 @@ static int patch_copy(vx_ctx *ctx, const vx_patch *p, int slot, int ghosts, doub
     const char *what = up ? "patch upload" : "patch download";
     // (an empty shape copies nothing, rows that lap over each other are HIP's to refuse too)
     const bool rows = p->n_x + 2 * ghosts > 0 && w > 0 && w <= (size_t)p->pitch && w * sizeof(double) <= vx_ctx::STAGE_BYTES;
-    if (rows && vx_device_range(ctx, dev, (h - 1) * p->pitch + w) && pageable(host))
+    if (rows && vx_device_range(ctx, dev, (h - 1) * p->pitch + w) && pageable(host) && stage_there(ctx))
         return staged_rows(ctx, dev, p->pitch, host, w, h, up, what);
     hipError_t e = up ? hipMemcpy2DAsync(dev, sizeof(double) * p->pitch, host, sizeof(double) * w,
                                          sizeof(double) * w, h, hipMemcpyHostToDevice, ctx->stream)
