@@ -220,7 +220,7 @@ def test_whole_patch_keeps_its_own_moments(shape, comp):
 @pytest.mark.parametrize("a", ["zero", "uniform", "pulse"])
 @pytest.mark.parametrize("comp", [False, True])
 def test_tall_patches_around_the_rules(a, comp):
-    """Heights on either side of those from which a small patch has a table, alone
+    """Heights on either side of those from which a small rtb 1 patch has a table, alone
     (with it) and in one launch with another (without); full launches of tall columns
     (8 a workgroup) with a ragged last workgroup, against a part of their columns."""
     tall = [(10, 1022, 1, False), (9, 1026, 1, False), (6, 1088, 2, True), (10, 1536, 1, False), (11, 1538, 1, False),

@@ -190,12 +190,12 @@ __device__ __forceinline__ double log_ratio(double a, double b) {
 }
 
 __device__ __forceinline__ void put_charge(const MomPatch &P, long e, double v) {
-    if (P.chargeR) P.chargeR[e] = v;
+    P.chargeR[e] = v;
     if (P.charge) P.charge[e] = P.species[e] = 0.0 + v;
 }
 __device__ __forceinline__ void put_current(const MomPatch &P, long e, double v) {
-    if (P.currentR) P.currentR[e] = v;
-    if (P.J) P.J[e] = 0.0 + v;
+    P.currentR[e] = v;
+    if (P.charge) P.J[e] = 0.0 + v;
 }
 
 // COMP (mixed-precision form): no consumer; each producer keeps its lanes'
@@ -272,7 +272,7 @@ __device__ __forceinline__ void moments_columns(const MomPatch &P, const vx_fiel
         // and its ring of chunks in flight is unrolled: slot d holds chunk
         // k0 + d in fixed registers and is reloaded with chunk k0 + d + WDEPTH
         // once its values are formed (a rotating copy would wait for the loads
-        // in flight).  COMP with a table, a loop of few instructions, has no exit
+        // in flight).  COMP with a table at RTB 1, a loop of few instructions, has no exit
         // inside it (the chunks past the last are skipped cells) and reloads a slot
         // behind the chunk's sums: 4096 x 4096 29.0 us against 32.6, 2048 x 4096 18.3
         // and 20.9.
@@ -282,7 +282,7 @@ __device__ __forceinline__ void moments_columns(const MomPatch &P, const vx_fiel
         auto run = [&](auto tab_c) __attribute__((always_inline)) {
             constexpr bool TAB = decltype(tab_c)::value;
             constexpr int NL = TAB ? 1 : RTB;  // logarithm sequences
-            constexpr bool WHOLE = COMP && TAB;  // whole rounds of the ring, loads behind the sums
+            constexpr bool WHOLE = COMP && TAB && RTB == 1;  // whole rounds of the ring, loads behind the sums
             double pv[WDEPTH][NR], pt[WDEPTH];
             int pn[WDEPTH];
             auto load = [&](int k, int d) __attribute__((always_inline)) {
@@ -386,8 +386,14 @@ __device__ __forceinline__ void moments_columns(const MomPatch &P, const vx_fiel
                 wave_two_sum(aR[s], cR[s], sr, er);
                 wave_two_sum(aJ[s], cJ[s], sj, ej);
                 if (lane == 0 && col_ok) {
-                    put_charge(P, (long)i * RTB + s, (sr + er) * P.dpq);
-                    put_current(P, (long)i * RTB + s, (sj + ej) * P.jscale);
+                    const long e = (long)i * RTB + s;
+                    const double q = (sr + er) * P.dpq, J = (sj + ej) * P.jscale;
+                    P.chargeR[e] = q;
+                    P.currentR[e] = J;
+                    if (P.charge) {
+                        P.charge[e] = P.species[e] = 0.0 + q;
+                        P.J[e] = 0.0 + J;
+                    }
                 }
             }
         }
@@ -574,6 +580,9 @@ static int moments_patch(vx_ctx *ctx, const vx_patch *p, const vx_fields *fl, bo
         A.p.charge = whole[0];
         A.p.J = whole[1];
         A.p.species = whole[2];
+        // (a patch without arrays of its own: written, then written again as assembled)
+        if (!A.p.chargeR) A.p.chargeR = whole[0];
+        if (!A.p.currentR) A.p.currentR = whole[1];
     }
     // The table saves each column its logarithms but costs a launch (3.1 us).
     // us with / without it: 1024 x 512 at rtb 1 8.3 / 7.0, 1024 x 1024 11.9 / 10.7,
@@ -582,11 +591,12 @@ static int moments_patch(vx_ctx *ctx, const vx_patch *p, const vx_fields *fl, bo
     // 4 21.1 / 19.1).  A wavefront that forms the terms for its workgroup's columns
     // instead: 9.2 at 1024 x 1024, but 52 at 4096 x 4096, 46 with the table.
     // In launches that do not fill the device a column's chain of chunks counts: any
-    // up to 512 columns, of 1280 p-cells 12.4 / 11.8, 1536 13.6 / 13.7, 2048 16.2 / 17.4,
+    // up to 512 columns at rtb 1, of 1280 p-cells 12.4 / 11.8, 1536 13.6 / 13.7, 2048 16.2 / 17.4,
     // 4096 27.3 / 31.7; compensated, of 1024 8.7 / 9.5, 2048 10.6 / 15.8, 4096 15 / 28.
     // (They go without where a graph is recorded before there is a table.)
     size_t need = (size_t)tab_entries(2, p->n_p);
-    const bool tall = p->n_p > (comp ? 1024 : 1536) && !(ctx->capturing && ctx->mom_table_n < need);
+    const bool tall = p->rtb == 1 && p->n_p > (comp ? 1024 : 1536) &&
+                      !(ctx->capturing && ctx->mom_table_n < need);
     if (tall || (long)p->n_x * p->n_p > TAB_CELLS) {
         if (ctx->mom_table_n < need) {
             if (ctx->capturing) return fail(ctx, VX_EINVAL, "moments: table growth while a step graph is recorded");
